@@ -249,6 +249,8 @@ int sphfem_destroy(sphfem_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     timing_collect(ctx);
     dfree(ctx->d_flags);
+    dfree(ctx->pre_vol);
+    dfree(ctx->pre_s);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return SPHFEM_OK;
@@ -636,6 +638,15 @@ int sphfem_interactions_monaghan(sphfem_ctx *ctx, sphfem_particles *p, const int
     if (!ctx || !p || !cell_start || !cell_end || num_cell != ctx->c.geom.nx * ctx->c.geom.ny) return SPHFEM_ERR_ARG;
     return guarded(ctx, [&] {
         if (int rc = need(ctx, SET_PHYS | SET_CORR)) return rc;
+        if (p->N > ctx->pre_cap) {      // the factors' workspace grows to the largest particle count
+            SPHFEM_HIP_CHECK(hipStreamSynchronize(ctx->stream));
+            ctx->pre_cap = 0;
+            dfree(ctx->pre_vol);
+            dfree(ctx->pre_s);
+            ctx->pre_vol = dalloc<double>(p->N);
+            ctx->pre_s = dalloc<sphfem_double4>(p->N);
+            ctx->pre_cap = p->N;
+        }
         launch_interactions_ref(ctx, *p, cell_start, cell_end);
         return SPHFEM_OK;
     });

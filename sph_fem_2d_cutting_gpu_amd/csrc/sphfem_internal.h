@@ -24,7 +24,10 @@
 #define SPHFEM_SEG_SINK_CAP 4096
 #define SPHFEM_FLAG_SINK_FRIC 6
 #define SPHFEM_FLAG_SINK_S2 7
-#define SPHFEM_NUM_FLAGS 8
+// interactions_monaghan's own two switches of the same kind, used in turn by its calls: a call's first
+// kernel sets one and clears the other for the next call (each is read by the call's second kernel)
+#define SPHFEM_FLAG_MONAGHAN 8
+#define SPHFEM_NUM_FLAGS 10
 // position records a wavefront of the staged FP32C pair kernel copies into LDS (8 KiB)
 #define SPHFEM_STAGE_CAP 512
 // blocks of the report_force reduction (its partials: 2 doubles per block) and the largest particle
@@ -117,6 +120,12 @@ struct sphfem_ctx {
                                   // [3]: re-sort mode (1 full, 2 incremental), [4]: changed count,
                                   // [5]: non-finite pair inputs present (SPHFEM_FLAG_NONFINITE)
     double *force_scratch = nullptr;  // this device's `scratch` array (sphfem_api.cpp)
+    // interactions_monaghan: the neighbour factors of k_pre_state for the largest particle count seen
+    // (pre_vol [pre_cap], pre_s [pre_cap]) and which of its two switches the next call uses
+    double *pre_vol = nullptr;
+    sphfem_double4 *pre_s = nullptr;
+    unsigned pre_cap = 0;
+    int monaghan_turn = 0;
     sphfem::Timing timing;
 };
 

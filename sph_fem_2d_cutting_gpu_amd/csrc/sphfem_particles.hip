@@ -31,23 +31,20 @@ __device__ __forceinline__ void column_range(const int *__restrict__ cs, const i
     }
 }
 
-// PRE: the neighbour factors m/rho_j, (S_j - p_j)/rho_j^2, S_xy,j/rho_j^2 and sqrtf(K/rho_j) come
-// from pre_vol/pre_s (computed per particle by the reorder with the same operations, so the sums
-// are bit-identical); otherwise they are computed per pair as in the reference.
-// LIST_BS > 0: the in-support neighbours go through a per-lane list of CHUNK entries in LDS
-// (list = this lane's first entry, stride LIST_BS) before their terms are evaluated.
+// The neighbour factors m/rho_j, (S_j - p_j)/rho_j^2, S_xy,j/rho_j^2 and sqrtf(K/rho_j) come from
+// pre_vol / pre_s, computed once per particle with the operations the reference repeats per pair, so
+// the sums are bit-identical.  The in-support neighbours go through a per-lane list of CHUNK entries in
+// LDS (list = this lane's first entry, stride LIST_BS) before their terms are evaluated.
 // WIN: every non-blanked particle of the 5x5 cells is evaluated, as the reference does, instead of
 // the in-support ones only.  The kernel's zeros outside the support make the two the same sums for
 // finite inputs; a neighbour with a non-finite input turns the sums NaN (0 * NaN) in the reference
 // wherever it lies in the window, and only the WIN form reproduces that.
-template <bool PRE, int LIST_BS = 0, int CHUNK = 0, bool WIN = false>
+template <int LIST_BS, int CHUNK, bool WIN>
 __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sphfem_particles &P, int pidx,
                                                    double thermal_alpha, const int *__restrict__ cs,
-                                                   const int *__restrict__ ce,
-                                                   const double *__restrict__ pre_vol = nullptr,
-                                                   const sphfem_double4 *__restrict__ pre_s = nullptr,
-                                                   int *__restrict__ list = nullptr) {
-    const double mass = c.phys.mass, K = c.phys.K;
+                                                   const int *__restrict__ ce, const double *__restrict__ pre_vol,
+                                                   const sphfem_double4 *__restrict__ pre_s, int *__restrict__ list) {
+    const double mass = c.phys.mass;
     const double wdeltap = c.corr.wdeltap, alpha = c.corr.alpha, beta = c.corr.beta;
     const double eta = c.corr.eta, eps = c.corr.xspheps;
     const int nx = c.geom.nx, ny = c.geom.ny;
@@ -61,8 +58,7 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
     const double rhoi21 = 1. / (rhoi * rhoi);
     const double fourh2 = 4 * hi * hi;
     const bool unit_wdp = wdeltap == 1.;      // w / 1 == w exactly
-    double ci_pre = 0.;
-    if constexpr (PRE) ci_pre = pre_s[pidx].w;
+    const double ci = pre_s[pidx].w;
     const int hashi = P.hash[pidx];
     const int gi = hashi / ny;
     const int gj = hashi - gi * ny;
@@ -87,22 +83,9 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
             const sphfem_double2 vj = P.vel[iter];
             const sphfem_double4 Rj = P.R[iter];
             const double hj = P.h[iter];
-            double volj, sjx, sjy, sjz;
-            if constexpr (PRE) {
-                volj = pre_vol[iter];
-                const sphfem_double4 f = pre_s[iter];
-                sjx = f.x;
-                sjy = f.y;
-                sjz = f.z;
-            } else {
-                const sphfem_double4 Sj = P.S[iter];
-                const double prsj = P.p[iter];
-                volj = mass / rhoj;
-                const double rhoj21 = 1. / (rhoj * rhoj);
-                sjx = (Sj.x - prsj) * rhoj21;
-                sjy = Sj.y * rhoj21;
-                sjz = (Sj.z - prsj) * rhoj21;
-            }
+            const double volj = pre_vol[iter];
+            const sphfem_double4 fj = pre_s[iter];
+            const double sjx = fj.x, sjy = fj.y, sjz = fj.z, cj = fj.w;
             r.v_der.x += (vj.x - vi.x) * w_x * volj;
             r.v_der.y += (vj.x - vi.x) * w_y * volj;
             r.v_der.z += (vj.y - vi.y) * w_x * volj;
@@ -122,14 +105,6 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
             double vijposij = vijx * xij + vijy * yij;
             double rhoij = 0.5 * (rhoi + rhoj);
             if (vijposij < 0.) {
-                double ci, cj;
-                if constexpr (PRE) {
-                    ci = ci_pre;
-                    cj = pre_s[iter].w;
-                } else {
-                    ci = sqrtf_d(K / rhoi);
-                    cj = sqrtf_d(K / rhoj);
-                }
                 double cij = 0.5 * (ci + cj);
                 double hij = 0.5 * (hi + hj);
                 double r2ij = xij * xij + yij * yij;
@@ -148,59 +123,41 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
                 double eijx = xij / rij;
                 double eijy = yij / rij;
                 double rij1 = 1. / rij;
-                const double volT = PRE ? pre_vol[iter] : mass / rhoj;
-                r.T_lapl += 2.0 * volT * (Ti - Tj) * rij1 * (eijx * w_x + eijy * w_y);
+                r.T_lapl += 2.0 * pre_vol[iter] * (Ti - Tj) * rij1 * (eijx * w_x + eijy * w_y);
             }
         }
     };
-    if constexpr (LIST_BS == 0) {
-        for (int ii = low_i; ii < high_i; ii++) {
-            int first, last;
-            column_range(cs, ce, ii * ny, low_j, high_j, first, last);
-            if (first < 0 || last > (int)P.N) continue;   // empty column (or an inconsistent cell table)
-            for (int iter = first; iter < last; iter++) {
-                if (P.blanked[iter] == 1.) continue;
-                const sphfem_double2 pj = P.pos[iter];
-                double xij = pi.x - pj.x;
-                double yij = pi.y - pj.y;
-                double rr2 = xij * xij + yij * yij;
-                if (!WIN && (rr2 >= fourh2 || rr2 < rr2_min)) continue;
-                pair(iter, pj, xij, yij);
-            }
+    // the in-support neighbours are listed first (in the same order) and the pair terms are
+    // evaluated from the list, so the lanes of a wavefront evaluate pairs together instead of
+    // idling on candidates outside the support
+    int n = 0;
+    auto run = [&]() {
+        for (int k = 0; k < n; k++) {
+            const int iter = list[k * LIST_BS];
+            const sphfem_double2 pj = P.pos[iter];
+            pair(iter, pj, pi.x - pj.x, pi.y - pj.y);
         }
-    } else {
-        // the in-support neighbours are listed first (in the same order) and the pair terms are
-        // evaluated from the list, so the lanes of a wavefront evaluate pairs together instead of
-        // idling on candidates outside the support
-        int n = 0;
-        auto run = [&]() {
-            for (int k = 0; k < n; k++) {
-                const int iter = list[k * LIST_BS];
-                const sphfem_double2 pj = P.pos[iter];
-                pair(iter, pj, pi.x - pj.x, pi.y - pj.y);
-            }
-            n = 0;
-        };
-        for (int ii = low_i; ii < high_i; ii++) {
-            int first, last;
-            column_range(cs, ce, ii * ny, low_j, high_j, first, last);
-            if (first < 0 || last > (int)P.N) continue;
-            for (int iter = first; iter < last; iter++) {
-                if (P.blanked[iter] == 1.) continue;
-                const sphfem_double2 pj = P.pos[iter];
-                double xij = pi.x - pj.x;
-                double yij = pi.y - pj.y;
-                double rr2 = xij * xij + yij * yij;
-                if (!WIN && (rr2 >= fourh2 || rr2 < rr2_min)) continue;
-                list[n * LIST_BS] = iter;
-                ++n;
-                // a full list empties every active lane's list at once: lanes that flushed at
-                // their own points would each run their list with the rest of the wavefront idle
-                if (__any(n == CHUNK)) run();
-            }
+        n = 0;
+    };
+    for (int ii = low_i; ii < high_i; ii++) {
+        int first, last;
+        column_range(cs, ce, ii * ny, low_j, high_j, first, last);
+        if (first < 0 || last > (int)P.N) continue;
+        for (int iter = first; iter < last; iter++) {
+            if (P.blanked[iter] == 1.) continue;
+            const sphfem_double2 pj = P.pos[iter];
+            double xij = pi.x - pj.x;
+            double yij = pi.y - pj.y;
+            double rr2 = xij * xij + yij * yij;
+            if (!WIN && (rr2 >= fourh2 || rr2 < rr2_min)) continue;
+            list[n * LIST_BS] = iter;
+            ++n;
+            // a full list empties every active lane's list at once: lanes that flushed at
+            // their own points would each run their list with the rest of the wavefront idle
+            if (__any(n == CHUNK)) run();
         }
-        run();
     }
+    run();
     return r;
 }
 
@@ -940,17 +897,53 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const do
 }
 
 
-// interactions_gpu.cu:143-379 as one kernel (drop-in entry point): every particle of the 5x5 cells,
-// as the reference visits them
+// interactions_gpu.cu:143-379 for the drop-in entry point, first kernel: the neighbour factors of
+// k_pairs_fp64's pair loop from the arrays as they stand (the same operations the reference repeats
+// per pair), and the switch to the reference's full window: a live particle with a non-finite input
+// or factor, or without a positive density (a zero kernel value times such a factor is not zero).
+__global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_particles P, double *__restrict__ pre_vol,
+                                                   sphfem_double4 *__restrict__ pre_s, int *__restrict__ window,
+                                                   int *__restrict__ next_window) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *next_window = 0;
+    if (i >= (int)P.N) return;
+    const double rho = P.rho[i], pr = P.p[i];
+    const sphfem_double4 S = P.S[i], R = P.R[i];
+    const sphfem_double2 pos = P.pos[i], vel = P.vel[i];
+    const double blanked = P.blanked[i], T = P.T[i], h = P.h[i];
+    const double vol = c.phys.mass / rho;
+    const double rho21 = 1. / (rho * rho);
+    const sphfem_double4 f = {(S.x - pr) * rho21, S.y * rho21, (S.z - pr) * rho21, sqrtf_d(c.phys.K / rho)};
+    pre_vol[i] = vol;
+    pre_s[i] = f;
+    const double s = ((pos.x + pos.y) + (vel.x + vel.y)) + ((T + h) + (R.x + R.y)) + (R.z + vol) +
+                     ((f.x + f.y) + (f.z + f.w));
+    if (blanked != 1. && !(isfinite(s) && rho > 0.)) *window = 1;
+}
+
+// second kernel: the pair sums in the reference's arithmetic and neighbour order.  With finite inputs
+// the candidates outside the support add exact zeros and are skipped; otherwise (`window`) every
+// particle of the 5x5 cells is evaluated, as the reference visits them.  Bound by the FP64 divisions
+// and the neighbour gathers of the in-support pairs: evaluating the whole window instead (about twice
+// the pairs, with each neighbour's factors divided out again per pair) took 3106 us per launch at
+// 2.07M particles of the chip domain, this and k_pre_state 2140 us.
 __global__ void __launch_bounds__(256) k_interactions_ref(DevConsts c, sphfem_particles P, const int *__restrict__ cs,
-                                                          const int *__restrict__ ce) {
+                                                          const int *__restrict__ ce,
+                                                          const double *__restrict__ pre_vol,
+                                                          const sphfem_double4 *__restrict__ pre_s,
+                                                          const int *__restrict__ window) {
     __shared__ int nb_list[48 * 256];
-    int pidx = blockIdx.x * blockDim.x + threadIdx.x;
+    const int pidx = xcd_logical_block() * 256 + (int)threadIdx.x;
     if (pidx >= (int)P.N) return;
     if (P.blanked[pidx] == 1.) return;
-    double thermal_alpha = interaction_alpha(c, P.tool_particle[pidx]);
-    PairSums r = pair_sums_fp64<false, 256, 48, true>(c, P, pidx, thermal_alpha, cs, ce, nullptr, nullptr,
+    const double thermal_alpha = interaction_alpha(c, P.tool_particle[pidx]);
+    PairSums r;
+    if (*window != 0)
+        r = pair_sums_fp64<256, 48, true>(c, P, pidx, thermal_alpha, cs, ce, pre_vol, pre_s,
                                                 nb_list + threadIdx.x);
+    else
+        r = pair_sums_fp64<256, 48, false>(c, P, pidx, thermal_alpha, cs, ce, pre_vol, pre_s,
+                                                 nb_list + threadIdx.x);
     P.S_der[pidx] = r.S_der;
     P.v_der[pidx] = r.v_der;
     P.pos_t[pidx] = r.pos_t;
@@ -1005,8 +998,15 @@ void launch_interactions_pse(sphfem_ctx *ctx, const sphfem_particles &p, const i
 }
 
 void launch_interactions_ref(sphfem_ctx *ctx, const sphfem_particles &p, const int *cs, const int *ce) {
+    int *window = ctx->d_flags + SPHFEM_FLAG_MONAGHAN + ctx->monaghan_turn;
+    ctx->monaghan_turn ^= 1;
+    int *next_window = ctx->d_flags + SPHFEM_FLAG_MONAGHAN + ctx->monaghan_turn;
+    {
+        KTimer t(ctx, "interactions_pre");
+        k_pre_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, ctx->pre_vol, ctx->pre_s, window, next_window);
+    }
     KTimer t(ctx, "interactions_ref");
-    k_interactions_ref<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, cs, ce);
+    k_interactions_ref<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, cs, ce, ctx->pre_vol, ctx->pre_s, window);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1159,10 +1159,10 @@ __global__ void __launch_bounds__(BS) k_pairs_fp64(DevConsts c, sphfem_particles
     const double thermal_alpha = interaction_alpha(c, B.tool_particle[i]);
     // the window form when a live particle carries a non-finite input (see pair_sums_fp64)
     if (*nonfinite != 0)
-        psum64[i] = pair_sums_fp64<true, BS, CHUNK, true>(c, B, i, thermal_alpha, cs, ce, pre_vol, pre_s,
+        psum64[i] = pair_sums_fp64<BS, CHUNK, true>(c, B, i, thermal_alpha, cs, ce, pre_vol, pre_s,
                                                           nb_list + threadIdx.x);
     else
-        psum64[i] = pair_sums_fp64<true, BS, CHUNK, false>(c, B, i, thermal_alpha, cs, ce, pre_vol, pre_s,
+        psum64[i] = pair_sums_fp64<BS, CHUNK, false>(c, B, i, thermal_alpha, cs, ce, pre_vol, pre_s,
                                                            nb_list + threadIdx.x);
 }
 
