@@ -1,0 +1,63 @@
+// Correctly rounded FP64 quotients and square roots that share their reciprocals, from the
+// fused-multiply-add iterations of P. Markstein ("Computation of elementary functions on the IBM RISC
+// System/6000 processor", IBM J. Res. Dev. 34 (1990) 111): with y the correctly rounded reciprocal of b
+// and q within an ulp or two of a / b, q + (a - b q) y rounded once is the correctly rounded quotient.
+// A pair of the FP64 sums divides three times by its distance and twice by its mean density; one
+// reciprocal serves each, where a division of its own per quotient repeats the reciprocal and adds the
+// scaling of extreme operands.  Valid for divisors and radicands whose reciprocal, square and remainder
+// are normal numbers; the callers keep others on the plain operators.
+//
+// y0 is a seed of at least 20 good bits: the hardware's approximation, or any other in a host test.
+#pragma once
+
+#include <cmath>
+
+namespace sphfem {
+
+#if defined(__HIPCC__)
+#define SPHFEM_HD __host__ __device__ __forceinline__
+#else
+#define SPHFEM_HD inline
+#endif
+
+// a divisor and its reciprocal, correctly rounded but (by an ulp) for some of the divisors in the last
+// 2^-46 below a power of two; the quotients by such a divisor are correctly rounded all the same
+struct Recip {
+    double b, y;
+};
+
+// two Newton steps: 20 -> 40 -> 80 good bits, the second rounded once
+SPHFEM_HD Recip recip_from(double b, double y0) {
+    const double y = std::fma(std::fma(-b, y0, 1.), y0, y0);
+    return {b, std::fma(std::fma(-b, y, 1.), y, y)};
+}
+
+SPHFEM_HD double quot(double a, const Recip &r) {
+    const double q = a * r.y;
+    return std::fma(std::fma(-r.b, q, a), r.y, q);
+}
+
+// square root of x and the half reciprocal root the iteration carries (h = 1 / (2 sqrt(x)) to 40 bits)
+SPHFEM_HD double sqrt_from(double x, double y0, double &h) {
+    double g = x * y0;
+    h = 0.5 * y0;
+    const double r = std::fma(-h, g, 0.5);
+    g = std::fma(g, r, g);
+    h = std::fma(h, r, h);
+    g = std::fma(std::fma(-g, g, x), h, g);
+    return std::fma(std::fma(-g, g, x), h, g);
+}
+
+// single-precision root of a radicand that is a single-precision number: the double root rounded to
+// single precision is the correctly rounded single root (53 >= 2 * 24 + 2 bits), so it needs no final
+// correction; h as above
+SPHFEM_HD double sqrtf_from(double x, double y0, double &h) {
+    double g = x * y0;
+    h = 0.5 * y0;
+    const double r = std::fma(-h, g, 0.5);
+    g = std::fma(g, r, g);
+    h = std::fma(h, r, h);
+    return (double)(float)std::fma(std::fma(-g, g, x), h, g);
+}
+
+}  // namespace sphfem

@@ -19,6 +19,10 @@
 // d_flags slot set by the reorder when a live particle carries a non-finite pair input (the pair
 // kernels then use the reference's full 5x5-cell window) and cleared by the update kernel
 #define SPHFEM_FLAG_NONFINITE 5
+// densities whose sums, reciprocals and quotients are normal numbers; a live particle outside them
+// switches the FP64 pair sums to the window form and its plain divisions
+#define SPHFEM_RHO_MIN 1e-290
+#define SPHFEM_RHO_MAX 1e290
 // records per step of each ordered segment sum (friction heat, contact heat exchange); the
 // reduction sorts them in LDS
 #define SPHFEM_SEG_SINK_CAP 4096

@@ -57,6 +57,7 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
     if (thermal_alpha != 0.) Ti = P.T[pidx];
     const double rhoi21 = 1. / (rhoi * rhoi);
     const double fourh2 = 4 * hi * hi;
+    const double h1 = 1 / hi;
     const bool unit_wdp = wdeltap == 1.;      // w / 1 == w exactly
     const double ci = pre_s[pidx].w;
     const int hashi = P.hash[pidx];
@@ -75,8 +76,14 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
     // one in-support pair (xij, yij from the sorted positions); the order of the calls is the
     // reference's neighbour order, so the sums are the same whichever loop drives them
     auto pair = [&](int iter, const sphfem_double2 pj, double xij, double yij) {
-        double w, w_x, w_y;
-        cubic_spline(pi.x, pi.y, pj.x, pj.y, hi, rr2_min, w, w_x, w_y);
+        const bool heat = thermal_alpha != 0.;
+        const double r2 = xij * xij + yij * yij;
+        // the shared-reciprocal form (the 1M-particle step's k_pairs_fp64 529 -> 497 us) while the single-precision radius and the quotients by it are normal
+        // numbers (in any length unit a case is set up in), else, and in the window form, the plain one
+        RadialTerms t;
+        if (!WIN && r2 > 1e-36 && r2 < 1e36) t = radial_terms(xij, yij, r2, hi, h1, heat);
+        else t = radial_terms_plain(pi.x, pi.y, pj.x, pj.y, xij, yij, r2, hi, rr2_min, heat);
+        const double w = t.w, w_x = t.w_x, w_y = t.w_y;
         const double rhoj = P.rho[iter];
         const double is_tool_j = P.tool_particle[iter];
         if (!(is_tool_i == 1.) && !(is_tool_j == 1.)) {
@@ -104,27 +111,28 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
             double vijy = vi.y - vj.y;
             double vijposij = vijx * xij + vijy * yij;
             double rhoij = 0.5 * (rhoi + rhoj);
+            // both densities lie in the range that keeps the window form off (flag_nonfinite)
+            Recip by_rhoij{};
+            if constexpr (!WIN) by_rhoij = recip_from(rhoij, __builtin_amdgcn_rcp(rhoij));
+            auto over_rhoij = [&](double a) {
+                if constexpr (WIN) return a / rhoij;
+                else return quot(a, by_rhoij);
+            };
             if (vijposij < 0.) {
                 double cij = 0.5 * (ci + cj);
                 double hij = 0.5 * (hi + hj);
-                double r2ij = xij * xij + yij * yij;
-                double muij = (hij * vijposij) / (r2ij + eta * eta * hij * hij);
-                double piij = (-alpha * cij * muij + beta * muij * muij) / rhoij;
+                double muij = (hij * vijposij) / (r2 + eta * eta * hij * hij);
+                double piij = over_rhoij(-alpha * cij * muij + beta * muij * muij);
                 r.vel_t.x += -mass * piij * w_x;
                 r.vel_t.y += -mass * piij * w_y;
             }
-            r.pos_t.x += -eps * w * mass / rhoij * vijx;
-            r.pos_t.y += -eps * w * mass / rhoij * vijy;
+            const double xsph = over_rhoij(-eps * w * mass);
+            r.pos_t.x += xsph * vijx;
+            r.pos_t.y += xsph * vijy;
         }
-        if (thermal_alpha != 0.) {
-            double rij = sqrt(xij * xij + yij * yij);
-            if (rij > 1e-8) {
-                const double Tj = P.T[iter];
-                double eijx = xij / rij;
-                double eijy = yij / rij;
-                double rij1 = 1. / rij;
-                r.T_lapl += 2.0 * pre_vol[iter] * (Ti - Tj) * rij1 * (eijx * w_x + eijy * w_y);
-            }
+        if (heat && t.rij > 1e-8) {
+            const double Tj = P.T[iter];
+            r.T_lapl += 2.0 * pre_vol[iter] * (Ti - Tj) * t.rij1 * (t.ex * w_x + t.ey * w_y);
         }
     };
     // the in-support neighbours are listed first (in the same order) and the pair terms are
@@ -900,7 +908,8 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const do
 // interactions_gpu.cu:143-379 for the drop-in entry point, first kernel: the neighbour factors of
 // k_pairs_fp64's pair loop from the arrays as they stand (the same operations the reference repeats
 // per pair), and the switch to the reference's full window: a live particle with a non-finite input
-// or factor, or without a positive density (a zero kernel value times such a factor is not zero).
+// or factor, or with a density out of the range of flag_nonfinite (a zero kernel value times such a
+// factor is not zero).
 __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_particles P, double *__restrict__ pre_vol,
                                                    sphfem_double4 *__restrict__ pre_s, int *__restrict__ window,
                                                    int *__restrict__ next_window) {
@@ -918,15 +927,15 @@ __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_par
     pre_s[i] = f;
     const double s = ((pos.x + pos.y) + (vel.x + vel.y)) + ((T + h) + (R.x + R.y)) + (R.z + vol) +
                      ((f.x + f.y) + (f.z + f.w));
-    if (blanked != 1. && !(isfinite(s) && rho > 0.)) *window = 1;
+    if (blanked != 1. && !(isfinite(s) && rho > SPHFEM_RHO_MIN && rho < SPHFEM_RHO_MAX)) *window = 1;
 }
 
 // second kernel: the pair sums in the reference's arithmetic and neighbour order.  With finite inputs
 // the candidates outside the support add exact zeros and are skipped; otherwise (`window`) every
-// particle of the 5x5 cells is evaluated, as the reference visits them.  Bound by the FP64 divisions
-// and the neighbour gathers of the in-support pairs: evaluating the whole window instead (about twice
+// particle of the 5x5 cells is evaluated, as the reference visits them.  Bound by the neighbour gathers
+// and the FP64 arithmetic of the in-support pairs: evaluating the whole window instead (about twice
 // the pairs, with each neighbour's factors divided out again per pair) took 3106 us per launch at
-// 2.07M particles of the chip domain, this and k_pre_state 2140 us.
+// 2.07M particles of the chip domain, this and k_pre_state 2140 us, 2010 us with the shared reciprocals.
 __global__ void __launch_bounds__(256) k_interactions_ref(DevConsts c, sphfem_particles P, const int *__restrict__ cs,
                                                           const int *__restrict__ ce,
                                                           const double *__restrict__ pre_vol,

@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "sphfem_fpmath.h"
 #include "sphfem_internal.h"
 
 #pragma clang fp contract(off)
@@ -53,6 +54,59 @@ __device__ __forceinline__ bool cubic_spline(double pix, double piy, double pjx,
     w_x = der * xij * fac;
     w_y = der * yij * fac;
     return true;
+}
+
+// The distance terms of one in-support pair: the kernel's value and gradient (cubic_spline above, the
+// same operations and roundings) and, for the heat term, the distance and 1 / distance and the unit
+// vector (interactions_gpu.cu:340-352), the quotients by shared reciprocals (sphfem_fpmath.h)
+struct RadialTerms {
+    double w, w_x, w_y, rij, rij1, ex, ey;
+};
+
+__device__ __forceinline__ RadialTerms radial_terms(double xij, double yij, double rr2, double hi, double h1,
+                                                    bool heat) {
+    RadialTerms t{};
+    const double y0 = __builtin_amdgcn_rsq(rr2);
+    double h;
+    const double rad = sqrtf_from((double)(float)rr2, y0, h);
+    const double q = rad * h1;
+    const double fac = SPHFEM_PI_FAC * h1 * h1;
+    double val, num;
+    if (q > 1) {
+        const double tmq = 2 - q, tmq2 = tmq * tmq;
+        val = 0.25 * tmq2 * tmq2 * tmq2;
+        num = -0.75 * tmq2 * h1;
+    } else {
+        val = 1 - 1.5 * q * q * (1 - 0.5 * q);
+        num = -3.0 * q * (1 - 0.75 * q) * h1;
+    }
+    const double der = quot(num, recip_from(rad, 2. * h));
+    t.w = val * fac;
+    t.w_x = der * xij * fac;
+    t.w_y = der * yij * fac;
+    if (heat) {
+        t.rij = sqrt_from(rr2, y0, h);
+        const Recip r = recip_from(t.rij, 2. * h);
+        t.rij1 = r.y;
+        t.ex = quot(xij, r);
+        t.ey = quot(yij, r);
+    }
+    return t;
+}
+
+// the same with the plain operators, for distances whose intermediate values leave the normal range
+__device__ __forceinline__ RadialTerms radial_terms_plain(double pix, double piy, double pjx, double pjy, double xij,
+                                                          double yij, double rr2, double hi, double rr2_min,
+                                                          bool heat) {
+    RadialTerms t{};
+    cubic_spline(pix, piy, pjx, pjy, hi, rr2_min, t.w, t.w_x, t.w_y);
+    if (heat) {
+        t.rij = sqrt(rr2);
+        t.ex = xij / t.rij;
+        t.ey = yij / t.rij;
+        t.rij1 = 1. / t.rij;
+    }
+    return t;
 }
 
 // actions_gpu.cu:222-232

@@ -1,0 +1,54 @@
+"""The shared-reciprocal quotients and roots of the FP64 pair sums (csrc/sphfem_fpmath.h) on the CPU:
+equal to the correctly rounded operators for random operands over 120 binades and for divisors just
+below a power of two, from seeds with 20 good bits (the hardware's approximations have more)."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+SOURCE = r"""
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <random>
+#include "%s/sph_fem_2d_cutting_gpu_amd/csrc/sphfem_fpmath.h"
+using namespace sphfem;
+int main() {
+    std::mt19937_64 g(3);
+    std::uniform_real_distribution<double> u(-1, 1);
+    long bad = 0;
+    for (long k = 0; k < 4000000; k++) {
+        double b = std::ldexp(1.5 + 0.5 * u(g), (int)(60 * u(g)));
+        const double a = std::ldexp(u(g), (int)(60 * u(g)));
+        if (k %% 5 == 0) {
+            const unsigned long long m = 0x3ff0000000000000ull | ((1ull << 52) - 1 - (g() %% 64));
+            std::memcpy(&b, &m, 8);
+        }
+        const double s = 1 + u(g) * std::ldexp(1, -20);
+        double h;
+        bad += quot(a, recip_from(b, 1 / b * s)) != a / b;
+        const double q = sqrt_from(b, 1 / std::sqrt(b) * s, h);
+        bad += q != std::sqrt(b);
+        bad += quot(a, recip_from(q, 2 * h)) != a / q;
+        const double x = (double)(float)b;     // the seed belongs to b, as in the pair term
+        const double f = sqrtf_from(x, 1 / std::sqrt(b) * s, h);
+        bad += f != (double)(float)std::sqrt(x);
+        const Recip r = recip_from(f, 2 * h);
+        bad += r.y != 1 / f || quot(a, r) != a / f;
+    }
+    std::printf("%%ld\n", bad);
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_quotients_and_roots_are_correctly_rounded(tmp_path):
+    src = tmp_path / "q.cpp"
+    src.write_text(SOURCE % ROOT)
+    exe = tmp_path / "q"
+    subprocess.run(["g++", "-O2", "-mfma", "-ffp-contract=off", "-std=c++17", str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.strip() == "0"
