@@ -333,10 +333,8 @@ int sphfem_leap_frog_correct(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_parti
  * result bit for bit, with the FEM tool and with a rigid tool.  The FP64 form always runs its
  * pair and update kernels separately (pair_kernel does not apply to it). */
 enum { SPHFEM_PAIRS_LIST = 0, SPHFEM_PAIRS_STAGED = 1, SPHFEM_PAIRS_LIST_FUSED = 2, SPHFEM_PAIRS_STAGED_FUSED = 3 };
-/* resort_one_block: the step's full-sort fallback (first step, or more particles changed cells than
- * the incremental re-sort takes) by one workgroup in one launch instead of the multi-block radix
- * sort's per-pass launches, which are queued every step and return at once on the incremental
- * path; the same permutation.  Only for N <= 2^19 (rejected above). */
+/* resort_one_block: 0 or 1, 1 only for N <= 2^19 (rejected above).  Both run the same kernels: the
+ * step's full-sort fallback is one launch in either setting. */
 typedef struct { int pair_block, pair_chunk, update_block, pair_kernel, resort_one_block; } sphfem_tuning;
 int sphfem_leap_frog_set_tuning(sphfem_ctx *ctx, sphfem_leap_frog *lf, const sphfem_tuning *tuning);
 int sphfem_leap_frog_get_tuning(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_tuning *tuning);

@@ -10,9 +10,8 @@ Tunables (all result-neutral except the FP32 summation blocks of the FP32C form)
                     one wavefront per workgroup, so pair_block does not apply); same sums.  Each
                     also fused with the update (the particle's update right after its sums: no
                     pair-sum round trip, update_block does not apply); same step result
-  * resort_one_block -- the step's full-sort fallback by one workgroup in one launch instead of the
-                    multi-block radix sort's eight per-step launches (N <= 2^19; tried with the best
-                    of the others: it pays when launches dominate and full sorts are rare)
+  * resort_one_block -- 0 or 1 (N <= 2^19); both run the same kernels (the step's full-sort fallback
+                    is one launch), tried with the best of the others
   * graph_steps  -- steps per captured graph in a batch (2 ... 32): fewer graph launches per step
 The tuner times each candidate on the live workload (it advances the simulation: run it in the
 warm-up), keeps the fastest and can store the choice in a JSON cache keyed by workload size,

@@ -401,13 +401,13 @@ static void grid_alloc(sphfem_ctx *ctx, sphfem_grid *g, int kind, int num_part) 
     g->nblocks = nblk(num_part, 4096);
     g->hist = dalloc<int>(256ul * g->nblocks);
     g->digit_tot = dalloc<int>(256);
-    const int nw = nblk(num_part, 64);
-    g->cmask = dalloc<unsigned long long>(nw);
-    g->wprefix = dalloc<int>(nw + 1);
-    g->bprefix = dalloc<int>(g->nblocks + 1);
+    g->keys_tmp = dalloc<int>(num_part);
+    g->sync = dalloc<int>(SPHFEM_RESORT_SYNC);
+    launch_fill_int(ctx, g->sync, SPHFEM_RESORT_SYNC, 0);
     g->clist = dalloc<int2>(SPHFEM_RESORT_CAP);
-    g->csorted = dalloc<unsigned long long>(SPHFEM_RESORT_CAP);
-    g->cdest = dalloc<int4>(SPHFEM_RESORT_CAP);
+    g->changed = dalloc<int2>(SPHFEM_RESORT_CAP);
+    g->dests = dalloc<int>(SPHFEM_RESORT_CAP);
+    g->removed = dalloc<int>(SPHFEM_RESORT_CAP);
     alloc_particles(ctx->stream, (unsigned)num_part, g->buf);
     g->first_sort = true;
     g->kind = kind;
@@ -544,7 +544,7 @@ int sphfem_grid_destroy(sphfem_ctx *ctx, sphfem_grid *g) {
         SPHFEM_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         dfree(g->cell_start); dfree(g->cell_end); dfree(g->keys_alt); dfree(g->vals_alt);
         dfree(g->hist); dfree(g->digit_tot);
-        dfree(g->cmask); dfree(g->wprefix); dfree(g->bprefix); dfree(g->clist); dfree(g->csorted); dfree(g->cdest);
+        dfree(g->keys_tmp); dfree(g->sync); dfree(g->clist); dfree(g->changed); dfree(g->dests); dfree(g->removed);
         dfree(g->perm); dfree(g->iota); dfree(g->bbox_part); dfree(g->bbox_out);
         free_particles(g->buf);
         delete g;
@@ -564,7 +564,7 @@ int sphfem_grid_assign_hashes(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles 
     return guarded(ctx, [&] {
         if (!(g->geom.dx > 0.)) return fail(ctx, SPHFEM_ERR_STATE, "unlocked grid: update_geometry first");
         ctx->c.geom = g->geom;
-        launch_hash(ctx, g, *p, false, nullptr);
+        launch_hash(ctx, g, *p);
         // p.hash no longer holds the keys of the (Green) cell table
         if (g->kind == SPHFEM_GRID_GREEN) g->first_sort = true;
         return SPHFEM_OK;
@@ -578,7 +578,7 @@ int sphfem_grid_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles *p) {
             launch_rothlin_sort(ctx, g, *p);
             return SPHFEM_OK;
         }
-        launch_radix_sort(ctx, g, *p, false);
+        launch_radix_sort(ctx, g, *p);
         launch_fill_int(ctx, g->cell_start, g->num_cell, -1);
         launch_reorder_full(ctx, g, *p);
         swap_gathered(*p, g->buf);
@@ -1748,19 +1748,21 @@ static int step_body(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_particles *p,
     // leap_frog.cu:175 (a no-op for a locked grid)
     if (int rc = update_geometry(ctx, g, *p, 2.)) return rc;
     ctx->c.geom = g->geom;
-    // the FEM tool's step start runs inside the hash pass of the Green re-sort (below), else here
-    const bool tool_in_hash = t && g->kind != SPHFEM_GRID_ROTHLIN;
-    if (t && !tool_in_hash) launch_tool_begin(ctx, t);
-    else if (!t) launch_fill_int(ctx, ctx->d_flags + 1, SPHFEM_FLAG_NONFINITE, 0);   // [1] .. [5]
-    if (rt) launch_rigid_advance(ctx, rt);
+    // the tool's step start runs inside the hash pass of the Green re-sort (below), else here
+    const bool green = g->kind != SPHFEM_GRID_ROTHLIN;
+    if (!green) {
+        if (t) launch_tool_begin(ctx, t);
+        else launch_fill_int(ctx, ctx->d_flags + 1, SPHFEM_FLAG_NONFINITE, 0);   // [1] .. [5]
+        if (rt) launch_rigid_advance(ctx, rt);
+    }
     // the source of each sorted position: the permutation of the sort (Green), or the identity
     // after the Rothlin sort has gathered in place
     sphfem_particles A = *p;
     const bool f32c = lf->precision == SPHFEM_FP32C;
     const size_t nr = lf->num_part;
     sync_rate_form(ctx, lf, *p);
-    if (g->kind == SPHFEM_GRID_ROTHLIN) {
-        launch_hash(ctx, g, *p, false, nullptr);
+    if (!green) {
+        launch_hash(ctx, g, *p);
         launch_rothlin_sort(ctx, g, *p);    // sorted keys, in-place gathers, dense cell table
         if (f32c) {                         // the carry follows the in-place gathers
             launch_rates_gather(ctx, rate_view(lf->rate32[lf->rate_cur], nr), rate_view(lf->rate32[lf->rate_cur ^ 1], nr),
@@ -1769,15 +1771,16 @@ static int step_body(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_particles *p,
         }
         A.idx = g->iota;
     } else {
-        // the cell table is cleared by the hash pass (cells of the previous keys) except when the
+        // the cell table is cleared by the re-sort (cells of the previous keys) except when the
         // previous keys are unknown
         if (g->first_sort) launch_fill_int(ctx, g->cell_start, g->num_cell, -1);
-        launch_resort(ctx, g, *p, lf->tuning.resort_one_block != 0, tool_in_hash ? t : nullptr);
+        launch_resort(ctx, g, *p, t, rt);
         g->first_sort = false;
     }
     const RateView r_old = rate_view(lf->rate32[lf->rate_cur], nr);
     const RateView r_new = rate_view(lf->rate32[lf->rate_cur ^ 1], nr);
-    launch_reorder_predict(ctx, g, A, lf, f32c ? &r_old : nullptr);
+    launch_reorder_predict(ctx, g, A, lf, f32c ? &r_old : nullptr, green);
+    if (green) std::swap(p->hash, g->keys_alt);     // the sorted keys
     sphfem_particles B = g->buf;
     B.hash = p->hash;
     B.idx = A.idx;

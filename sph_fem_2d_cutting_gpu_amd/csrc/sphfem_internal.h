@@ -12,8 +12,12 @@
 
 // largest number of particles that may change cells in one step for the incremental re-sort
 #define SPHFEM_RESORT_CAP 4096
-// largest N whose full-sort fallback may run in one workgroup (tuning resort_one_block)
+// largest N for which the tuning resort_one_block is accepted
 #define SPHFEM_SORT_ONE_BLOCK_MAX (1 << 19)
+// largest N for which a step known to sort in full does so inside the re-sort's one launch
+#define SPHFEM_SORT_ONE_LAUNCH_MAX (1 << 18)
+// counters of the re-sort (sphfem_grid::sync)
+#define SPHFEM_RESORT_SYNC 16
 // blocks of the bounding-box reduction of an unlocked grid
 #define SPHFEM_BBOX_BLOCKS 1024
 // d_flags slot set by the reorder when a live particle carries a non-finite pair input (the pair
@@ -148,13 +152,13 @@ struct sphfem_grid {
     // double buffer of the 20 gathered arrays (grid_gpu_green.h:21-50)
     sphfem_particles buf{};
     bool first_sort = true;
-    // incremental re-sort of the step (particles stored in the previous sorted order)
-    unsigned long long *cmask = nullptr;   // [nw] bit per position: cell changed this step
-    int *wprefix = nullptr;                // [nw] changed positions before each 64-block, within its tile
-    int *bprefix = nullptr;                // [nblocks + 1] changed positions before each 4096-tile
-    int2 *clist = nullptr;                 // [SPHFEM_RESORT_CAP] changed (key, position), position order
-    unsigned long long *csorted = nullptr; // [SPHFEM_RESORT_CAP] changed (key << 32 | position), sorted
-    int4 *cdest = nullptr;                 // [SPHFEM_RESORT_CAP] (destination, key, position)
+    // re-sort of the step (particles stored in the previous sorted order)
+    int *keys_tmp = nullptr;               // [N] radix scratch: the previous keys stay in p.hash
+    int *sync = nullptr;                   // [SPHFEM_RESORT_SYNC] changed count, work queue; zero between steps
+    int2 *clist = nullptr;                 // [SPHFEM_RESORT_CAP] changed (key, position), any order
+    int2 *changed = nullptr;               // [SPHFEM_RESORT_CAP] changed (key, position), sorted
+    int *dests = nullptr;                  // [SPHFEM_RESORT_CAP] their destinations, ascending
+    int *removed = nullptr;                // [SPHFEM_RESORT_CAP] their positions, ascending
     int resort_limit = SPHFEM_RESORT_CAP;  // max changed particles for the incremental path (0: off)
     // grid_gpu_rothlin: in-place gathers and dense cell offsets
     int kind = SPHFEM_GRID_GREEN;
@@ -340,21 +344,21 @@ template <bool NT, class T> __device__ __forceinline__ void st_maybe_stream(T *p
 }
 
 // sort / cells (sphfem_sort.hip)
-void launch_hash(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, bool clear_old, int *hist0);
-void launch_radix_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, bool hash_done_with_hist0,
-                       int *vals_out = nullptr);
+void launch_hash(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p);
+void launch_radix_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, int *vals_out = nullptr);
 void launch_rothlin_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p);
 void launch_cells_dense(sphfem_ctx *ctx, const int *sorted_keys, int N, int num_cell, int *cell_start, int *cell_end);
 void launch_iota(sphfem_ctx *ctx, int *ptr, int n);
 void launch_bbox(sphfem_ctx *ctx, const sphfem_particles &p, double *part, double *out);
-// t: the FEM tool whose step start (tool_begin_item) runs in extra workgroups of the hash pass, or NULL
-void launch_resort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, bool one_block_fallback,
-                   sphfem_tool *t = nullptr);
+// t, rt: the FEM tool whose step start (tool_begin_item), or the rigid tool whose motion, runs in extra
+// workgroups of the hash pass, or NULL
+void launch_resort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, sphfem_tool *t, sphfem_rigid_tool *rt);
 void launch_fill_int(sphfem_ctx *ctx, int *ptr, long n, int value);
 void launch_reorder_full(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p);
-// FP32C: the pre-step rates are read from the carry buffer rates (in the order of p)
+// FP32C: the pre-step rates are read from the carry buffer rates (in the order of p); resorted: the
+// sorted order comes from launch_resort, not from p.hash and p.idx
 void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, sphfem_leap_frog *lf,
-                            const RateView *rates = nullptr);
+                            const RateView *rates, bool resorted);
 void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, float4 *rec);
 
 // particles (sphfem_particles.hip)
@@ -384,14 +388,19 @@ void launch_fric_heat(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_tool *t
 void launch_contact(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_tool *t);
 void launch_tool_begin(sphfem_ctx *ctx, sphfem_tool *t);
 
+// the step's counters: the near list's length and the window-form switch of the pair kernels
+__device__ __forceinline__ void step_counters_clear(int *counters) {
+    counters[1] = 0;
+    counters[SPHFEM_FLAG_NONFINITE] = 0;
+}
+
 // the start of a step for the FEM tool, item i of max(nodes, segments): reset_FEM_server's
 // T_old = T and calculate_temp(0.5 dt) for the nodes; zero the wear accumulators
 // (segments_wear_rate_reset) and, item 0, the near-list and segment-sink counters and the
 // window-form switch of the pair kernels
 __device__ __forceinline__ void tool_begin_item(const sphfem_tool &t, double half_dt, int *counters, int i) {
     if (i == 0) {
-        counters[1] = 0;
-        counters[SPHFEM_FLAG_NONFINITE] = 0;
+        step_counters_clear(counters);
         counters[SPHFEM_FLAG_SINK_FRIC] = 0;
         counters[SPHFEM_FLAG_SINK_S2] = 0;
     }

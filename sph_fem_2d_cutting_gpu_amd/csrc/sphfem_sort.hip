@@ -6,6 +6,7 @@
 //    particle arrays (all 20 for the reference-form sort, or fused with init/predict/EOS/
 //    artificial stress for the step).
 #include "sphfem_physics.h"
+#include "sphfem_rigid.h"
 
 #pragma clang fp contract(off)
 
@@ -23,42 +24,26 @@ __device__ __forceinline__ int hash_of(const DevConsts &c, sphfem_double2 pos) {
     return ix * c.geom.ny + iy;
 }
 
-// grid.cu:25-42; also clears the cells the previous step occupied (their starts were the only
-// non -1 entries) and, optionally, counts digit 0 of the new keys per 4096-key tile.
+// grid.cu:25-42 (blanked particles keep their previous hash)
 __global__ void __launch_bounds__(SORT_BS) k_hash(DevConsts c, const double *__restrict__ blanked,
-                                                  const sphfem_double2 *__restrict__ pos,
-                                                  const int *__restrict__ old_hash, int *__restrict__ hash_out,
-                                                  int *__restrict__ cell_start, int clear_old, int N,
-                                                  int num_cell, int *__restrict__ hist0, int nblocks,
-                                                  int *__restrict__ flags) {
-    __shared__ int lh[RADIX];
-    for (int d = threadIdx.x; d < RADIX; d += SORT_BS) lh[d] = 0;
-    __syncthreads();
+                                                  const sphfem_double2 *__restrict__ pos, int *__restrict__ hash, int N,
+                                                  int num_cell, int *__restrict__ flags) {
     const int base = blockIdx.x * SORT_TILE;
     for (int it = 0; it < SORT_ITEMS; it++) {
         int i = base + it * SORT_BS + threadIdx.x;
         if (i >= N) break;
-        int oh = old_hash[i];
-        if (clear_old && oh >= 0 && oh < num_cell) cell_start[oh] = -1;
-        int h = oh;
+        int h = hash[i];
         if (blanked[i] != 1.) h = hash_of(c, pos[i]);
         if (h < 0 || h >= num_cell) {
             atomicOr(&flags[0], 1);
             h = h < 0 ? 0 : num_cell - 1;
         }
-        hash_out[i] = h;
-        if (hist0) atomicAdd(&lh[h & (RADIX - 1)], 1);
-    }
-    if (hist0) {
-        __syncthreads();
-        for (int d = threadIdx.x; d < RADIX; d += SORT_BS) hist0[d * nblocks + blockIdx.x] = lh[d];
+        hash[i] = h;
     }
 }
 
-// `mode`, when given, points at the device re-sort mode: the full-sort kernels run only in mode 1
 __global__ void __launch_bounds__(SORT_BS) k_upsweep(const int *__restrict__ keys, int N, int shift,
-                                                     int *__restrict__ hist, int nblocks, const int *mode) {
-    if (mode && *mode != 1) return;
+                                                     int *__restrict__ hist, int nblocks) {
     __shared__ int lh[RADIX];
     for (int d = threadIdx.x; d < RADIX; d += SORT_BS) lh[d] = 0;
     __syncthreads();
@@ -74,8 +59,7 @@ __global__ void __launch_bounds__(SORT_BS) k_upsweep(const int *__restrict__ key
 
 // one block per digit: exclusive scan of that digit's per-tile counts, total into digit_tot
 __global__ void __launch_bounds__(SORT_BS) k_scan_digits(int *__restrict__ hist, int nblocks,
-                                                         int *__restrict__ digit_tot, const int *mode) {
-    if (mode && *mode != 1) return;
+                                                         int *__restrict__ digit_tot) {
     __shared__ int part[SORT_BS];
     int *row = hist + (long)blockIdx.x * nblocks;
     int per = (nblocks + SORT_BS - 1) / SORT_BS;
@@ -106,14 +90,16 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
     return lane ? ((~0ull) >> (64 - lane)) : 0ull;
 }
 
-// stable scatter of one pass; vals_in == nullptr means the values are the input positions
+// stable scatter of one pass; vals_in == nullptr means the values are the input positions.  old_keys
+// (pass 0 of the step's sort): the previous sorted keys, whose cells are cleared by the particles that
+// left them (a cell that keeps one of its particles gets its start again from the reorder)
 __global__ void __launch_bounds__(SORT_BS) k_downsweep(const int *__restrict__ keys_in,
                                                        const int *__restrict__ vals_in,
                                                        int *__restrict__ keys_out, int *__restrict__ vals_out,
                                                        int N, int shift, const int *__restrict__ hist,
                                                        int nblocks, const int *__restrict__ digit_tot,
-                                                       int *__restrict__ flags, const int *mode) {
-    if (mode && *mode != 1) return;
+                                                       int *__restrict__ flags, const int *__restrict__ old_keys,
+                                                       int *__restrict__ cell_start, int num_cell) {
     __shared__ int block_off[RADIX];
     __shared__ int wcount[SORT_BS / WAVE][RADIX];
     __shared__ int scan[RADIX];
@@ -143,6 +129,10 @@ __global__ void __launch_bounds__(SORT_BS) k_downsweep(const int *__restrict__ k
         int k = valid ? keys_in[i] : 0;
         key[r] = k;
         val[r] = valid ? (vals_in ? vals_in[i] : i) : 0;
+        if (valid && old_keys) {
+            const int oh = old_keys[i];
+            if (oh != k && oh >= 0 && oh < num_cell) cell_start[oh] = -1;
+        }
         int d = (k >> shift) & (RADIX - 1);
         uint64_t peers = __ballot(valid);
 #pragma unroll
@@ -185,194 +175,6 @@ __global__ void __launch_bounds__(SORT_BS) k_downsweep(const int *__restrict__ k
     }
 }
 
-// The full stable LSD radix sort of the step's fallback (mode 1) by one workgroup, for up to
-// SPHFEM_SORT_ONE_BLOCK_MAX particles: one launch, which returns at once on the incremental path,
-// in place of the per-pass upsweep / digit-scan / downsweep launches.  The passes, the digit
-// offsets and the stable order within a pass (tiles in increasing index; within a tile waves, item
-// rows and lanes in index order, as k_downsweep ranks them) are those of the multi-block sort, so
-// the permutation is the same.  Unsorted keys in keys_in (values: their positions); passes ping-pong
-// between (ka, va) and (kb, vb) and the result ends in (ka, va).  kb may be keys_in: pass 0 reads
-// keys_in and writes ka, later passes no longer need it.  Every lane runs every loop (bounds are
-// uniform), so the ballots see whole wavefronts.
-// It also does k_resort_scan's work first (the changed counts of the hash pass -> re-sort mode) and,
-// on the incremental path, k_resort_compact's and k_resort_rank's (the changed particles gathered
-// into LDS from the changed bits, then ranked): the step's sort is then three launches (hash pass,
-// this, scatter) instead of five.
-__device__ __forceinline__ int changed_before(const unsigned long long *__restrict__ cmask,
-                                              const int *__restrict__ wlocal, const int *__restrict__ bprefix,
-                                              int p, int N, int m);
-
-__global__ void __launch_bounds__(SORT_BS) k_sort_one_block(const int *keys_in, int *ka, int *va, int *kb, int *vb,
-                                                            int N, int passes, int *flags, int *bprefix, int nb,
-                                                            int force_full, int cap,
-                                                            const unsigned long long *cmask, const int *wlocal,
-                                                            unsigned long long *csorted, int4 *cdest) {
-    __shared__ int off[RADIX];
-    __shared__ int cnt[RADIX];
-    __shared__ int wcount[SORT_BS / WAVE][RADIX];
-    __shared__ unsigned long long comp[SPHFEM_RESORT_CAP];
-    __shared__ int s_mode, s_m;
-    const int tid = threadIdx.x;
-    {   // exclusive scan of the tiles' changed counts, as k_resort_scan
-        int carry = 0;
-        for (int c0 = 0; c0 < nb; c0 += SORT_BS) {
-            const int j = c0 + tid;
-            const int v = j < nb ? bprefix[j] : 0;
-            cnt[tid] = v;
-            __syncthreads();
-            for (int o = 1; o < SORT_BS; o <<= 1) {
-                const int u = tid >= o ? cnt[tid - o] : 0;
-                __syncthreads();
-                cnt[tid] += u;
-                __syncthreads();
-            }
-            if (j < nb) bprefix[j] = carry + cnt[tid] - v;
-            carry += cnt[SORT_BS - 1];
-            __syncthreads();
-        }
-        if (tid == 0) {
-            bprefix[nb] = carry;
-            flags[4] = carry;
-            s_mode = (force_full || carry > cap) ? 1 : 2;
-            s_m = carry;
-            flags[3] = s_mode;
-        }
-        __threadfence();
-        __syncthreads();
-    }
-    if (s_mode == 2) {
-        // the changed particles in position order (k_resort_compact), as (new key, position)
-        const int m = s_m;
-        const int words = (N + 63) >> 6;
-        for (int w = tid; w < words; w += SORT_BS) {
-            const unsigned long long bits = cmask[w];
-            unsigned long long rest = bits;
-            while (rest) {
-                const int b = __ffsll((long long)rest) - 1;
-                rest &= rest - 1;
-                const int i = (w << 6) + b;
-                const int k = changed_before(cmask, wlocal, bprefix, i, N, m);
-                if ((unsigned)k < (unsigned)m)
-                    comp[k] = ((unsigned long long)(unsigned)keys_in[i] << 32) | (unsigned)i;
-                else
-                    atomicOr(&flags[0], 2);
-            }
-        }
-        __syncthreads();
-        // their ranks and destinations (k_resort_rank), the old keys being ka (the sorted keys)
-        for (int k = tid; k < m; k += SORT_BS) {
-            const unsigned long long ck = comp[k];
-            int r = 0;
-            for (int q = 0; q < m; q++) r += comp[q] < ck;
-            int lo = 0, hi = N;
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                const unsigned long long cm = ((unsigned long long)(unsigned)ka[mid] << 32) | (unsigned)mid;
-                if (cm < ck) lo = mid + 1;
-                else hi = mid;
-            }
-            const int dest = r + lo - changed_before(cmask, wlocal, bprefix, lo, N, m);
-            if ((unsigned)dest >= (unsigned)N || r >= m) {
-                atomicOr(&flags[0], 2);
-                continue;
-            }
-            csorted[r] = ck;
-            cdest[r] = make_int4(dest, (int)(ck >> 32), (int)(ck & 0xffffffffu), 0);
-        }
-        return;
-    }
-    if (s_mode != 1) return;
-    const int w = tid / WAVE;
-    const int lane = tid % WAVE;
-    const uint64_t lt = lanemask_lt();
-    const int *kin = keys_in, *vin = nullptr;
-    int *kout = ka, *vout = va;
-    for (int ps = 0; ps < passes; ps++) {
-        const int shift = 8 * ps;
-        // digit totals of the pass, then their exclusive scan
-        cnt[tid] = 0;
-        __syncthreads();
-        for (int i = tid; i < N; i += SORT_BS) atomicAdd(&cnt[(kin[i] >> shift) & (RADIX - 1)], 1);
-        __syncthreads();
-        for (int o = 1; o < RADIX; o <<= 1) {
-            const int v = tid >= o ? cnt[tid - o] : 0;
-            __syncthreads();
-            cnt[tid] += v;
-            __syncthreads();
-        }
-        off[tid] = tid ? cnt[tid - 1] : 0;
-        __syncthreads();
-        for (int t0 = 0; t0 < N; t0 += SORT_TILE) {
-            for (int k = 0; k < SORT_BS / WAVE; k++) wcount[k][tid] = 0;
-            __syncthreads();
-            int key[SORT_ITEMS], val[SORT_ITEMS], rank[SORT_ITEMS];
-            const int base = t0 + w * (SORT_ITEMS * WAVE);
-#pragma unroll
-            for (int r = 0; r < SORT_ITEMS; r++) {
-                const int i = base + r * WAVE + lane;
-                const bool valid = i < N;
-                const int k = valid ? kin[i] : 0;
-                key[r] = k;
-                val[r] = valid ? (vin ? vin[i] : i) : 0;
-                const int d = (k >> shift) & (RADIX - 1);
-                uint64_t peers = __ballot(valid);
-#pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const uint64_t m = __ballot((d >> b) & 1);
-                    peers &= ((d >> b) & 1) ? m : ~m;
-                }
-                const int before = __popcll(peers & lt);
-                const int c = __popcll(peers);
-                int old = 0;
-                if (valid) old = wcount[w][d];
-                __builtin_amdgcn_wave_barrier();
-                if (valid && before == 0) wcount[w][d] = old + c;
-                __builtin_amdgcn_wave_barrier();
-                rank[r] = valid ? old + before : -1;
-            }
-            __syncthreads();
-            {   // per digit: prefix over the waves of the tile, and the tile's count
-                int run = 0;
-                for (int k = 0; k < SORT_BS / WAVE; k++) {
-                    const int v = wcount[k][tid];
-                    wcount[k][tid] = run;
-                    run += v;
-                }
-                cnt[tid] = run;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int r = 0; r < SORT_ITEMS; r++) {
-                if (rank[r] < 0) continue;
-                const int d = (key[r] >> shift) & (RADIX - 1);
-                const int dst = off[d] + wcount[w][d] + rank[r];
-                if ((unsigned)dst >= (unsigned)N) {   // cannot happen for consistent counts
-                    atomicOr(&flags[0], 2);
-                    continue;
-                }
-                kout[dst] = key[r];
-                vout[dst] = val[r];
-            }
-            __syncthreads();
-            off[tid] += cnt[tid];
-            __syncthreads();
-        }
-        // this pass's output, written by all waves, is the next pass's input
-        __threadfence();
-        __syncthreads();
-        kin = kout;
-        vin = vout;
-        kout = kout == ka ? kb : ka;
-        vout = vout == va ? vb : va;
-    }
-    if (kin != ka) {
-        for (int i = tid; i < N; i += SORT_BS) {
-            ka[i] = kin[i];
-            va[i] = vin[i];
-        }
-    }
-}
-
 __global__ void k_fill_int(int *p, long n, int v) {
     long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
     long stride = (long)gridDim.x * blockDim.x;
@@ -386,369 +188,603 @@ void launch_fill_int(sphfem_ctx *ctx, int *ptr, long n, int value) {
     k_fill_int<<<blocks, 256, 0, ctx->stream>>>(ptr, n, value);
 }
 
-void launch_hash(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, bool clear_old, int *hist0) {
-    // writes into p.hash (the reference's in-place layout); the fused step passes hist0
-    (void)hist0;
+void launch_hash(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p) {
+    // writes into p.hash (the reference's in-place layout)
     int N = (int)p.N;
     int nb = nblk(N, SORT_TILE);
     KTimer t(ctx, "hash");
-    k_hash<<<nb, SORT_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, p.hash, g->cell_start,
-                                            clear_old ? 1 : 0, N, g->num_cell, nullptr, nb, ctx->d_flags);
+    k_hash<<<nb, SORT_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, N, g->num_cell, ctx->d_flags);
+}
+
+// The passes of the multi-block radix sort from the unsorted keys in `src` to the sorted keys and the
+// permutation in (k1, v1), by way of (k2, v2); `src` is k2 for an odd number of passes and k1 for an
+// even one.  hist0: pass 0's per-tile histogram is already in g->hist; old_keys: see k_downsweep.
+static void launch_radix_passes(sphfem_ctx *ctx, sphfem_grid *g, int N, int *k1, int *v1, int *k2, int *v2, bool hist0,
+                                const int *old_keys) {
+    const int nb = nblk(N, SORT_TILE);
+    const int passes = (g->key_bits + 7) / 8;
+    int *kin = passes % 2 ? k2 : k1, *vin = nullptr;
+    for (int ps = 0; ps < passes; ps++) {
+        const int shift = 8 * ps;
+        int *kout = kin == k1 ? k2 : k1, *vout = kin == k1 ? v2 : v1;
+        if (ps > 0 || !hist0) {
+            KTimer t(ctx, "radix_upsweep");
+            k_upsweep<<<nb, SORT_BS, 0, ctx->stream>>>(kin, N, shift, g->hist, nb);
+        }
+        {
+            KTimer t(ctx, "radix_scan");
+            k_scan_digits<<<RADIX, SORT_BS, 0, ctx->stream>>>(g->hist, nb, g->digit_tot);
+        }
+        {
+            KTimer t(ctx, "radix_downsweep");
+            k_downsweep<<<nb, SORT_BS, 0, ctx->stream>>>(kin, vin, kout, vout, N, shift, g->hist, nb, g->digit_tot,
+                                                         ctx->d_flags, ps == 0 ? old_keys : nullptr, g->cell_start,
+                                                         g->num_cell);
+        }
+        kin = kout;
+        vin = vout;
+    }
 }
 
 // Radix sort of (p.hash, index) leaving sorted keys in p.hash and the permutation in p.idx
 // (in vals_out when given).
-// If hash_with_hist0, the hash pass (which computes the keys) is run here with the digit-0
-// histogram fused and writes the keys into the buffer the pass parity requires.
-void launch_radix_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, bool hash_with_hist0, int *vals_out) {
+void launch_radix_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, int *vals_out) {
     const int N = (int)p.N;
-    const int nb = nblk(N, SORT_TILE);
-    const int passes = (g->key_bits + 7) / 8;
-    int *kin, *vin = nullptr;
-    // choose buffers so that the last pass writes p.hash / p.idx
-    int *kbuf[2] = {p.hash, g->keys_alt};
-    int *vbuf[2] = {vals_out ? vals_out : p.idx, g->vals_alt};
-    int src = (passes % 2 == 1) ? 1 : 0;   // buffer holding the unsorted keys
-    if (hash_with_hist0) {
-        KTimer t(ctx, "hash");
-        k_hash<<<nb, SORT_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, kbuf[src], g->cell_start,
-                                                g->first_sort ? 0 : 1, N, g->num_cell, g->hist, nb,
-                                                ctx->d_flags);
-    } else if (src == 1) {
+    if ((g->key_bits + 7) / 8 % 2)
         (void)hipMemcpyAsync(g->keys_alt, p.hash, sizeof(int) * (size_t)N, hipMemcpyDeviceToDevice, ctx->stream);
-    }
-    kin = kbuf[src];
-    for (int ps = 0; ps < passes; ps++) {
-        int shift = 8 * ps;
-        int dst = 1 - src;
-        if (!(ps == 0 && hash_with_hist0)) {
-            KTimer t(ctx, "radix_upsweep");
-            k_upsweep<<<nb, SORT_BS, 0, ctx->stream>>>(kin, N, shift, g->hist, nb, nullptr);
-        }
-        {
-            KTimer t(ctx, "radix_scan");
-            k_scan_digits<<<RADIX, SORT_BS, 0, ctx->stream>>>(g->hist, nb, g->digit_tot, nullptr);
-        }
-        {
-            KTimer t(ctx, "radix_downsweep");
-            k_downsweep<<<nb, SORT_BS, 0, ctx->stream>>>(kin, ps == 0 ? nullptr : vin, kbuf[dst], vbuf[dst], N,
-                                                         shift, g->hist, nb, g->digit_tot, ctx->d_flags, nullptr);
-        }
-        kin = kbuf[dst];
-        vin = vbuf[dst];
-        src = dst;
-    }
+    launch_radix_passes(ctx, g, N, p.hash, vals_out ? vals_out : p.idx, g->keys_alt, g->vals_alt, false, nullptr);
 }
 
 // ---------------------------------------------------------------------------------------------
-// Incremental re-sort for the step.  After a step the particles are stored in the previous sorted
-// order, so `old` (the previous sorted keys) is ascending.  A particle keeps its cell unless it
-// crossed a cell boundary (rare at dt ~ 1e-4 of the cell crossing time).  The stable sort of the
-// new keys with the previous position as tie-break is then the merge of
+// Re-sort of the step.  After a step the particles are stored in the previous sorted order, so the
+// previous keys (p.hash) are ascending.  A particle keeps its cell unless it crossed a cell boundary
+// (rare at dt ~ 1e-4 of the cell crossing time).  The stable sort of the new keys with the previous
+// position as tie-break is then the merge of
 //   U: unchanged positions, already in (key, position) order, and
 //   C: changed positions sorted by (new key, position):
-//   dest(u) = u - changed_before(u) + |{c in C : (key_c, c) < (key_u, u)}|
-//   dest(C[r]) = r + P - changed_before(P),  P = first p with (old[p], p) >= (key_c, c)
+//   dest(C[r]) = r + P - |{c in C : c < P}|,  P = first p with (old[p], p) >= (key_c, c),
+//   and the unchanged positions fill the other destinations in order,
 // which is exactly the result of the full stable radix sort (same keys, same order).
-// The path is chosen on the device: the full radix sort runs on the first step and whenever more
-// than `cap` particles changed cells.
+// Three launches: the hash pass lists the changed particles (k_hash_mark), one workgroup ranks them
+// (k_resort), and the reorder reads each destination's source off the sorted lists (ResortView), so no
+// key or index array is written and read back in between.  The full sort runs on the first step and
+// whenever more than `cap` particles changed cells: k_resort's workgroups run it in that one launch.
+// Where the host knows of it before (force) and N is above SPHFEM_SORT_ONE_LAUNCH_MAX it is the
+// multi-block radix sort, whose launches beat the queue's waits there.  (Per step with the incremental
+// path before: the hash pass, scan, three idle launches per radix pass, compaction, ranking and
+// scatter, each a dependent launch of about 4.5 us.)
+// Sorted keys and permutation end in (g->keys_alt, p.idx); the caller swaps keys_alt and p.hash.
 // ---------------------------------------------------------------------------------------------
-__device__ __forceinline__ int changed_before(const unsigned long long *__restrict__ cmask,
-                                              const int *__restrict__ wlocal, const int *__restrict__ bprefix,
-                                              int p, int N, int m) {
-    if (p >= N) return m;
-    const unsigned long long bits = cmask[p >> 6];
-    const int b = p & 63;
-    return bprefix[p / SORT_TILE] + wlocal[p >> 6] + __popcll(b ? (bits & ((~0ull) >> (64 - b))) : 0ull);
-}
 
-// grid.cu:25-42 hash (as k_hash, with the digit-0 histogram for the full-sort fallback), plus the
-// changed bit of every position, the changed count before each 64 positions within the tile
-// (wlocal) and the tile's total (bcount)
-// Workgroups past nblocks (tool_blocks of them, when a FEM tool is given) do the tool's step start
-// instead (tool_begin_item), which shares no data with the hash pass: one launch fewer per step.
+// grid.cu:25-42 hash; the changed particles (new hash, position) appended to clist in any order, their
+// number counted in sync[RS_COUNT].  KEYS: also the new keys, and their digit-0 histogram per tile, for
+// the multi-block sort.  Workgroups past nblocks (tool_blocks of them, when a FEM tool is given) do the
+// tool's step start instead (tool_begin_item), which shares no data with the hash pass; a step without
+// one clears its counters here, and a rigid tool advances in the first lane past nblocks.
+// Bound by HBM: 28 B read per particle.
 constexpr int HASH_BS = 1024;                       // 16 wavefronts per tile, 4 items per lane
 constexpr int HASH_ITEMS = SORT_TILE / HASH_BS;
+// slots of sphfem_grid::sync: changed particles of this step, then the work queue of k_resort
+enum { RS_COUNT = 0, RS_TICKET = 1, RS_DONE = 2 };   // RS_DONE + phase: finished items of a phase
+constexpr int RS_USED = RS_DONE + 3 * 4;             // at most four passes of three phases
+static_assert(RS_USED <= SPHFEM_RESORT_SYNC, "counters");
+constexpr int RS_SCAN_TILES = 64;                    // above, a phase of its own scans the tiles' counts
+
+struct StepStart {            // what else begins with the step (see k_hash_mark)
+    sphfem_tool tool;
+    int tool_blocks;
+    double dt;
+    RigidTool *rigid;
+};
+
+template <bool KEYS>
 __global__ void __launch_bounds__(HASH_BS) k_hash_mark(DevConsts c, const double *__restrict__ blanked,
                                                        const sphfem_double2 *__restrict__ pos,
                                                        const int *__restrict__ old_hash, int *__restrict__ hash_out,
-                                                       int *__restrict__ cell_start, int clear_old, int N,
-                                                       int num_cell, int *__restrict__ hist0, int nblocks,
-                                                       int *flags, unsigned long long *__restrict__ cmask,
-                                                       int *__restrict__ wlocal, int *__restrict__ bcount,
-                                                       sphfem_tool tool, int tool_blocks, double half_dt) {
+                                                       int N, int num_cell, int *__restrict__ hist0, int nblocks,
+                                                       int *flags, int *__restrict__ sync, int2 *__restrict__ clist,
+                                                       int cap, StepStart st) {
     if ((int)blockIdx.x >= nblocks) {
-        if (tool_blocks > 0)
-            tool_begin_item(tool, half_dt, flags, ((int)blockIdx.x - nblocks) * HASH_BS + (int)threadIdx.x);
+        const int item = ((int)blockIdx.x - nblocks) * HASH_BS + (int)threadIdx.x;
+        if (st.tool_blocks > 0) tool_begin_item(st.tool, 0.5 * st.dt, flags, item);
+        else if (item == 0) rigid_move(st.rigid->g, st.dt);
         return;
     }
-    __shared__ int lh[RADIX];
+    __shared__ int lh[KEYS ? RADIX : 1];
     __shared__ int wc[SORT_TILE / 64];
-    for (int d = threadIdx.x; d < RADIX; d += HASH_BS) lh[d] = 0;
-    __syncthreads();
+    __shared__ int s_base;
+    if constexpr (KEYS) {
+        for (int d = threadIdx.x; d < RADIX; d += HASH_BS) lh[d] = 0;
+        __syncthreads();
+    }
+    if (blockIdx.x == 0 && st.tool_blocks == 0 && threadIdx.x == 0) step_counters_clear(flags);
     const int base = blockIdx.x * SORT_TILE;
     // every load of the lane's items first, then the hashes: the pass waits for memory once
-    int ohs[HASH_ITEMS];
+    int h[HASH_ITEMS];
     double bls[HASH_ITEMS];
     sphfem_double2 pss[HASH_ITEMS];
 #pragma unroll
     for (int it = 0; it < HASH_ITEMS; it++) {
         const int i = base + it * HASH_BS + threadIdx.x;
-        ohs[it] = i < N ? old_hash[i] : 0;
+        h[it] = i < N ? old_hash[i] : 0;
         bls[it] = i < N ? blanked[i] : 1.;
         pss[it] = i < N ? pos[i] : sphfem_double2{0., 0.};
     }
+    unsigned long long moved[HASH_ITEMS];
 #pragma unroll
     for (int it = 0; it < HASH_ITEMS; it++) {
         const int i = base + it * HASH_BS + threadIdx.x;
+        const int oh = h[it];
         bool changed = false;
         if (i < N) {
-            const int oh = ohs[it];
-            int h = oh;
-            if (bls[it] != 1.) h = hash_of(c, pss[it]);
-            if (h < 0 || h >= num_cell) {
+            if (bls[it] != 1.) h[it] = hash_of(c, pss[it]);
+            if (h[it] < 0 || h[it] >= num_cell) {
                 atomicOr(&flags[0], 1);
-                h = h < 0 ? 0 : num_cell - 1;
+                h[it] = h[it] < 0 ? 0 : num_cell - 1;
             }
-            hash_out[i] = h;
-            atomicAdd(&lh[h & (RADIX - 1)], 1);
-            changed = h != oh;
-            // a cell that keeps one of its particles stays occupied (the reorder rewrites its start);
-            // one that all of them left is cleared by each of them
-            if (clear_old && changed && oh >= 0 && oh < num_cell) cell_start[oh] = -1;
+            if constexpr (KEYS) {
+                hash_out[i] = h[it];
+                atomicAdd(&lh[h[it] & (RADIX - 1)], 1);
+            }
+            changed = h[it] != oh;
         }
-        const unsigned long long bits = __ballot(changed);
-        if (__lane_id() == 0) {
-            wc[(i - base) >> 6] = __popcll(bits);
-            if (i < N) cmask[i >> 6] = bits;
-        }
+        moved[it] = __ballot(changed);
+        if (__lane_id() == 0) wc[it * (HASH_BS / 64) + (threadIdx.x >> 6)] = __popcll(moved[it]);
     }
     __syncthreads();
-    for (int d = threadIdx.x; d < RADIX; d += HASH_BS) hist0[d * nblocks + blockIdx.x] = lh[d];
-    if (threadIdx.x == 0) {
-        int run = 0;
-        for (int k = 0; k < SORT_TILE / 64; k++) {
-            const int g = (base >> 6) + k;
-            if ((long)g * 64 < N) wlocal[g] = run;
-            run += wc[k];
+    if constexpr (KEYS)
+        for (int d = threadIdx.x; d < RADIX; d += HASH_BS) hist0[d * nblocks + blockIdx.x] = lh[d];
+    // one reservation per tile: the prefix over its 64 wavefront rows by the first wavefront
+    if (threadIdx.x < 64) {
+        const int v = wc[threadIdx.x];
+        int incl = v;
+        for (int off = 1; off < 64; off <<= 1) {
+            const int u = __shfl_up(incl, off);
+            if ((int)threadIdx.x >= off) incl += u;
         }
-        bcount[blockIdx.x] = run;
+        wc[threadIdx.x] = incl - v;
+        if (threadIdx.x == 63) s_base = incl ? atomicAdd(&sync[RS_COUNT], incl) : 0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < HASH_ITEMS; it++) {
+        if (!((moved[it] >> __lane_id()) & 1ull)) continue;
+        const int k = s_base + wc[it * (HASH_BS / 64) + (threadIdx.x >> 6)] + __popcll(moved[it] & lanemask_lt());
+        if (k < cap) clist[k] = make_int2(h[it], base + it * HASH_BS + (int)threadIdx.x);
     }
 }
 
-// one block: exclusive prefix of the tile totals (in place, coalesced chunks), the total and the
-// path decision
-constexpr int RESORT_SCAN_BS = 1024;
-__global__ void __launch_bounds__(RESORT_SCAN_BS) k_resort_scan(int *__restrict__ bprefix, int nb,
-                                                                int *__restrict__ flags, int force_full, int cap) {
-    __shared__ int part[RESORT_SCAN_BS];
-    int carry = 0;
-    for (int c0 = 0; c0 < nb; c0 += RESORT_SCAN_BS) {
-        const int j = c0 + threadIdx.x;
-        const int v = j < nb ? bprefix[j] : 0;
-        part[threadIdx.x] = v;
-        __syncthreads();
-        for (int off = 1; off < RESORT_SCAN_BS; off <<= 1) {
-            const int u = threadIdx.x >= off ? part[threadIdx.x - off] : 0;
-            __syncthreads();
-            part[threadIdx.x] += u;
-            __syncthreads();
+// First position p with (old[p], p) >= (key, c), the old keys ascending.  The previous cell table gives
+// the cell's run when it is occupied (checked against the keys: the table may be older than they are);
+// else a binary search.
+__device__ __forceinline__ int insert_position(const int *__restrict__ old_keys, const int *__restrict__ cell_start,
+                                               int N, int key, int c) {
+    const int s = cell_start[key];
+    int lo = 0, hi = N;
+    if (s >= 0 && s < N && old_keys[s] == key && (s == 0 || old_keys[s - 1] != key)) {
+        if (c <= s) return s;
+        lo = s;                          // the run starts here: gallop along it
+        for (int w = 1; lo + w < N; w <<= 1) {
+            const int q = lo + w;
+            if (old_keys[q] != key || q >= c) { hi = q; break; }
         }
-        if (j < nb) bprefix[j] = carry + part[threadIdx.x] - v;
-        carry += part[RESORT_SCAN_BS - 1];
-        __syncthreads();
     }
-    if (threadIdx.x == 0) {
-        bprefix[nb] = carry;
-        flags[4] = carry;
-        flags[3] = (force_full || carry > cap) ? 1 : 2;
+    while (lo < hi) {
+        const int mid = (lo + hi) >> 1;
+        const int k = old_keys[mid];
+        if (k < key || (k == key && mid < c)) lo = mid + 1;
+        else hi = mid;
     }
+    return lo;
 }
 
-// changed positions, in position order
-__global__ void __launch_bounds__(256) k_resort_compact(const int *__restrict__ keys, int N,
-                                                        const unsigned long long *__restrict__ cmask,
-                                                        const int *__restrict__ wlocal,
-                                                        const int *__restrict__ bprefix, int2 *__restrict__ clist,
-                                                        const int *flags) {
-    if (flags[3] != 2) return;
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i >= N) return;
-    const unsigned long long bits = cmask[i >> 6];
-    if (!((bits >> (i & 63)) & 1ull)) return;
-    const int k = changed_before(cmask, wlocal, bprefix, i, N, 0);
-    clist[k] = make_int2(keys[i], i);
+// waits until `want` items of a phase are done; false (with the error bit set) if that never comes,
+// which a queue in order cannot do: an item only waits for items taken before it, by running workgroups
+__device__ __forceinline__ bool wait_done(int *counter, int want, int *flags) {
+    for (int spin = 0; spin < (1 << 22); spin++) {
+        if (__hip_atomic_load(counter, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= want) return true;
+        __builtin_amdgcn_s_sleep(2);
+    }
+    atomicOr(&flags[0], 2);
+    return false;
 }
 
-// one block: rank of each changed position among the changed ones (counting in LDS; the composite
-// keys are distinct) and its destination
-__global__ void __launch_bounds__(RESORT_SCAN_BS) k_resort_rank(const int2 *__restrict__ clist,
-                                                                const int *__restrict__ old_keys, int N,
-                                                                const unsigned long long *__restrict__ cmask,
-                                                                const int *__restrict__ wlocal,
-                                                                const int *__restrict__ bprefix,
-                                                                unsigned long long *__restrict__ csorted,
-                                                                int4 *__restrict__ cdest, int *__restrict__ flags) {
+// The ranking of the changed particles by the first workgroup, or (more than cap of them, or force) the
+// full stable LSD radix sort by all of them.  The sort is a queue of items handed out in order by one
+// counter: per pass the tiles' digit counts, above RS_SCAN_TILES tiles the digits' scans over the tiles,
+// then the tiles' scatter (tile order, and within a tile wavefront, row and lane order, as k_downsweep
+// ranks them, so the permutation is the same).  Items of a phase wait for every item of the phase
+// before, all of which were taken by workgroups that are running: the queue needs no co-resident grid.
+// Latency bound: one workgroup on the incremental path (4.5 us at 160k and 5.6 us at 4M particles, where
+// its launches took 46 us and 55 us); the full sort of 131k particles 69 us, the multi-block launches
+// 68 us without their gaps.
+constexpr int RESORT_BS = 1024;
+constexpr int RESORT_ITEMS = SORT_TILE / RESORT_BS;
+__global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double *__restrict__ blanked,
+                                                      const sphfem_double2 *__restrict__ pos,
+                                                      const int *__restrict__ old_keys, int *__restrict__ cell_start,
+                                                      int N, int num_cell, int nb, int passes, int force, int cap,
+                                                      int clear_old, int sort_here, int *k1, int *v1, int *k2, int *v2,
+                                                      int *__restrict__ hist, int *__restrict__ digit_tot, int *flags,
+                                                      int *sync, const int2 *__restrict__ clist, int2 *__restrict__ changed,
+                                                      int *__restrict__ dests, int *__restrict__ removed) {
     __shared__ unsigned long long comp[SPHFEM_RESORT_CAP];
-    if (flags[3] != 2) return;
-    const int m = flags[4];
-    for (int k = threadIdx.x; k < m; k += RESORT_SCAN_BS) {
-        const int2 e = clist[k];
-        comp[k] = ((unsigned long long)(unsigned)e.x << 32) | (unsigned)e.y;
+    __shared__ int gone[SPHFEM_RESORT_CAP];
+    // the sort's per-wavefront digit counts, in the bytes of the ranking's composites
+    static_assert(sizeof(int) * (RESORT_BS / WAVE) * RADIX <= sizeof(unsigned long long) * SPHFEM_RESORT_CAP, "LDS");
+    int (*wcount)[RADIX] = reinterpret_cast<int (*)[RADIX]>(comp);
+    __shared__ int off[RADIX], cnt[RADIX];
+    __shared__ int s_item, s_go;
+    const int tid = threadIdx.x;
+    const int m = sync[RS_COUNT];
+    const bool full = force || m > cap;
+    if (blockIdx.x == 0 && tid == 0) {
+        flags[3] = full ? 1 : 2;
+        flags[4] = m;
     }
+    if (!full) {
+        if (blockIdx.x != 0) return;
+        for (int k = tid; k < m; k += RESORT_BS) {
+            const int2 e = clist[k];
+            comp[k] = ((unsigned long long)(unsigned)e.x << 32) | (unsigned)e.y;
+        }
+        __syncthreads();
+        // ranks by counting: r by (new key, position), rp by position
+        int r[SPHFEM_RESORT_CAP / RESORT_BS], P[SPHFEM_RESORT_CAP / RESORT_BS];
+#pragma unroll
+        for (int u = 0; u < SPHFEM_RESORT_CAP / RESORT_BS; u++) {
+            const int k = tid + u * RESORT_BS;
+            if (k >= m) continue;
+            const unsigned long long ck = comp[k];
+            const int at = (int)(unsigned)ck;
+            P[u] = insert_position(old_keys, cell_start, N, (int)(ck >> 32), at);
+            int rank = 0, rp = 0;
+            for (int q = 0; q < m; q++) {
+                const unsigned long long cq = comp[q];
+                rank += cq < ck;
+                rp += (int)(unsigned)cq < at;
+            }
+            r[u] = rank;
+            gone[rp] = at;
+            removed[rp] = at;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < SPHFEM_RESORT_CAP / RESORT_BS; u++) {
+            const int k = tid + u * RESORT_BS;
+            if (k >= m) continue;
+            const unsigned long long ck = comp[k];
+            const int at = (int)(unsigned)ck;
+            int lo = 0, hi = m;                       // removed positions below P
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (gone[mid] < P[u]) lo = mid + 1;
+                else hi = mid;
+            }
+            dests[r[u]] = r[u] + P[u] - lo;
+            changed[r[u]] = make_int2((int)(ck >> 32), at);
+            // a cell that keeps one of its particles gets its start again from the reorder; one that all
+            // of them left is cleared by each of them
+            const int oh = old_keys[at];
+            if (clear_old && oh >= 0 && oh < num_cell) cell_start[oh] = -1;
+        }
+        return;
+    }
+    if (!sort_here) return;
+    const int w = tid / WAVE, lane = tid % WAVE;
+    const uint64_t lt = lanemask_lt();
+    const bool scans = nb > RS_SCAN_TILES;
+    const int per_pass = scans ? 2 * nb + RADIX : 2 * nb;
+    const int items = passes * per_pass;
+    // the item of a turn is taken and published between two barriers and read into a scalar, so that the
+    // loop's control flow is uniform for the compiler too: a lane-dependent branch next to the back edge
+    // lets it send the other lanes round the loop alone
+    if (tid == 0) s_item = atomicAdd(&sync[RS_TICKET], 1);
     __syncthreads();
-    for (int k = threadIdx.x; k < m; k += RESORT_SCAN_BS) {
-        const unsigned long long ck = comp[k];
-        int r = 0;
-        for (int q = 0; q < m; q++) r += comp[q] < ck;
-        // P: first position p with (old[p], p) >= (key, position); (old[p], p) increases with p
-        int lo = 0, hi = N;
-        while (lo < hi) {
-            const int mid = (lo + hi) >> 1;
-            const unsigned long long cm = ((unsigned long long)(unsigned)old_keys[mid] << 32) | (unsigned)mid;
-            if (cm < ck) lo = mid + 1;
-            else hi = mid;
+    int item = __builtin_amdgcn_readfirstlane(s_item);
+    while (item < items) {
+        // pass, step of the pass (0 counts, 1 scan, 2 scatter) and the item's number in it
+        const int ps = item / per_pass, at = item - ps * per_pass, shift = 8 * ps;
+        const int step = at < nb ? 0 : (scans && at < nb + RADIX ? 1 : 2);
+        const int tile = step == 0 ? at : (step == 1 ? at - nb : at - (per_pass - nb));
+        const int phase = 3 * ps + step;
+        if (phase > 0) {
+            const int before = step == 2 && !scans ? phase - 2 : phase - 1;
+            if (tid == 0) {
+                s_go = wait_done(&sync[RS_DONE + before], step == 2 && scans ? RADIX : nb, flags) ? 1 : 0;
+                __threadfence();                      // the finished items' writes, from any XCD
+            }
+            __syncthreads();
+            if (__builtin_amdgcn_readfirstlane(s_go) == 0) return;
         }
-        const int dest = r + lo - changed_before(cmask, wlocal, bprefix, lo, N, m);
-        if ((unsigned)dest >= (unsigned)N || r >= m) {
-            atomicOr(&flags[0], 2);
-            continue;
+        // pass ps reads (ki, vi) and writes (ko, vo); the last pass ends in (k1, v1)
+        const bool to1 = (passes - ps) % 2 != 0;
+        const int *ki = to1 ? k2 : k1, *vi = to1 ? v2 : v1;
+        int *ko = to1 ? k1 : k2, *vo = to1 ? v1 : v2;
+        const int base = tile * SORT_TILE;
+        if (step == 0) {                              // digit counts of the tile
+            if (tid < RADIX) cnt[tid] = 0;
+            __syncthreads();
+            for (int it = 0; it < RESORT_ITEMS; it++) {
+                const int i = base + it * RESORT_BS + tid;
+                if (i >= N) break;
+                int h;
+                if (ps == 0) {                        // the keys themselves, as k_hash_mark computed them
+                    const int oh = old_keys[i];
+                    h = oh;
+                    if (blanked[i] != 1.) h = hash_of(c, pos[i]);
+                    h = h < 0 ? 0 : (h >= num_cell ? num_cell - 1 : h);
+                    if (clear_old && h != oh && oh >= 0 && oh < num_cell) cell_start[oh] = -1;
+                    const_cast<int *>(ki)[i] = h;
+                } else {
+                    h = ki[i];
+                }
+                atomicAdd(&cnt[(h >> shift) & (RADIX - 1)], 1);
+            }
+            __syncthreads();
+            if (tid < RADIX) hist[(long)tile * RADIX + tid] = cnt[tid];
+        } else if (step == 1) {                       // one digit's counts scanned over the tiles
+            int carry = 0;
+            for (int q0 = 0; q0 < nb; q0 += RESORT_BS) {
+                const int q = q0 + tid;
+                const int v = q < nb ? hist[(long)q * RADIX + tile] : 0;
+                int incl = v;
+                for (int o = 1; o < WAVE; o <<= 1) {
+                    const int u = __shfl_up(incl, o);
+                    if (lane >= o) incl += u;
+                }
+                if (lane == WAVE - 1) cnt[w] = incl;
+                __syncthreads();
+                int below = carry, all = carry;
+                for (int k = 0; k < RESORT_BS / WAVE; k++) {
+                    below += k < w ? cnt[k] : 0;
+                    all += cnt[k];
+                }
+                if (q < nb) hist[(long)q * RADIX + tile] = below + incl - v;
+                carry = all;
+                __syncthreads();
+            }
+            if (tid == 0) digit_tot[tile] = carry;
+        } else {
+            // offsets of the tile's digits: lower digits of all tiles, then lower tiles
+            if (tid < RADIX) {
+                int below = 0, all = 0;
+                if (scans) {
+                    below = hist[(long)tile * RADIX + tid];
+                    all = digit_tot[tid];
+                } else {
+                    for (int q = 0; q < nb; q++) {
+                        const int v = hist[(long)q * RADIX + tid];
+                        all += v;
+                        below += q < tile ? v : 0;
+                    }
+                }
+                off[tid] = below;
+                cnt[tid] = all;
+            }
+            for (int k = tid; k < (RESORT_BS / WAVE) * RADIX; k += RESORT_BS) (&wcount[0][0])[k] = 0;
+            __syncthreads();
+            for (int o = 1; o < RADIX; o <<= 1) {
+                const int v = tid < RADIX && tid >= o ? cnt[tid - o] : 0;
+                __syncthreads();
+                if (tid < RADIX) cnt[tid] += v;
+                __syncthreads();
+            }
+            if (tid < RADIX && tid > 0) off[tid] += cnt[tid - 1];
+            int key[RESORT_ITEMS], val[RESORT_ITEMS], rank[RESORT_ITEMS];
+#pragma unroll
+            for (int q = 0; q < RESORT_ITEMS; q++) {
+                const int i = base + w * (RESORT_ITEMS * WAVE) + q * WAVE + lane;
+                const bool valid = i < N;
+                const int k = valid ? ki[i] : 0;
+                key[q] = k;
+                val[q] = valid ? (ps == 0 ? i : vi[i]) : 0;
+                const int d = (k >> shift) & (RADIX - 1);
+                uint64_t peers = __ballot(valid);
+#pragma unroll
+                for (int b = 0; b < 8; b++) {
+                    const uint64_t mm = __ballot((d >> b) & 1);
+                    peers &= ((d >> b) & 1) ? mm : ~mm;
+                }
+                const int before = __popcll(peers & lt);
+                int old = 0;
+                if (valid) old = wcount[w][d];
+                __builtin_amdgcn_wave_barrier();
+                if (valid && before == 0) wcount[w][d] = old + __popcll(peers);
+                __builtin_amdgcn_wave_barrier();
+                rank[q] = valid ? old + before : -1;
+            }
+            __syncthreads();
+            if (tid < RADIX) {                        // prefix of each digit over the tile's wavefronts
+                int run = off[tid];
+                for (int k = 0; k < RESORT_BS / WAVE; k++) {
+                    const int v = wcount[k][tid];
+                    wcount[k][tid] = run;
+                    run += v;
+                }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int q = 0; q < RESORT_ITEMS; q++) {
+                if (rank[q] < 0) continue;
+                const int dst = wcount[w][(key[q] >> shift) & (RADIX - 1)] + rank[q];
+                if ((unsigned)dst >= (unsigned)N) {   // cannot happen for consistent counts
+                    atomicOr(&flags[0], 2);
+                    continue;
+                }
+                ko[dst] = key[q];
+                vo[dst] = val[q];
+            }
         }
-        csorted[r] = ck;
-        cdest[r] = make_int4(dest, (int)(ck >> 32), (int)(ck & 0xffffffffu), 0);
+        // this item's writes before it counts as done: the barrier orders the workgroup's before lane 0's
+        // fence (a fence by every wavefront writes the L2 back sixteen times)
+        __syncthreads();
+        if (tid == 0) {
+            __threadfence();
+            atomicAdd(&sync[RS_DONE + phase], 1);
+            s_item = atomicAdd(&sync[RS_TICKET], 1);
+        }
+        __syncthreads();
+        item = __builtin_amdgcn_readfirstlane(s_item);
     }
 }
 
-// scatter: unchanged positions by the merge formula, changed ones from cdest
-__global__ void __launch_bounds__(256) k_resort_scatter(const int *__restrict__ keys, int N,
-                                                        const unsigned long long *__restrict__ cmask,
-                                                        const int *__restrict__ wlocal,
-                                                        const int *__restrict__ bprefix,
-                                                        const unsigned long long *__restrict__ csorted,
-                                                        const int4 *__restrict__ cdest, int *__restrict__ keys_out,
-                                                        int *__restrict__ idx_out, int *__restrict__ flags) {
-    if (flags[3] != 2) return;
-    const int m = flags[4];
-    const int i = blockIdx.x * 256 + threadIdx.x;
-    if (i < m) {
-        const int4 e = cdest[i];
-        if ((unsigned)e.x < (unsigned)N) {
-            keys_out[e.x] = e.y;
-            idx_out[e.x] = e.z;
-        }
+// Re-sort of the step: the lists of the incremental path, or the sorted keys and permutation in
+// (g->keys_alt, p.idx); what each destination's source is, resort_source tells the reorder.
+void launch_resort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, sphfem_tool *tool, sphfem_rigid_tool *rt) {
+    const int N = (int)p.N;
+    const int nb = nblk(N, SORT_TILE);
+    int *flags = ctx->d_flags;
+    const int cap = std::min(g->resort_limit, SPHFEM_RESORT_CAP);
+    const int force = (g->first_sort || cap <= 0) ? 1 : 0;
+    const int passes = (g->key_bits + 7) / 8;
+    const int clear_old = g->first_sort ? 0 : 1;
+    // a full sort known beforehand, and above the size where the multi-block launches win
+    const bool launches = force && N > SPHFEM_SORT_ONE_LAUNCH_MAX;
+    int *unsorted = passes % 2 ? g->keys_tmp : g->keys_alt;
+    StepStart st{};
+    if (tool) {
+        st.tool = *tool;
+        st.tool_blocks = nblk(std::max(std::max(tool->n_nodes, tool->n_seg), 1), HASH_BS);
     }
-    if (i >= N) return;
-    if ((cmask[i >> 6] >> (i & 63)) & 1ull) return;
-    const int key = keys[i];
-    const unsigned long long ck = ((unsigned long long)(unsigned)key << 32) | (unsigned)i;
+    st.dt = ctx->c.dt;
+    st.rigid = rt ? rt->dev : nullptr;
+    const int extra = tool ? st.tool_blocks : (rt ? 1 : 0);
+    {
+        KTimer t(ctx, tool ? "hash_tool_begin" : "hash");
+        if (!launches)
+            k_hash_mark<false><<<nb + extra, HASH_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, nullptr, N,
+                                                                        g->num_cell, nullptr, nb, flags, g->sync,
+                                                                        g->clist, cap, st);
+        else
+            k_hash_mark<true><<<nb + extra, HASH_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, unsorted, N,
+                                                                       g->num_cell, g->hist, nb, flags, g->sync,
+                                                                       g->clist, cap, st);
+    }
+    {
+        KTimer t(ctx, "resort");
+        const int blocks = launches ? 1 : std::min(nb, 256);
+        k_resort<<<blocks, RESORT_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, g->cell_start, N,
+                                                        g->num_cell, nb, passes, force, cap, clear_old,
+                                                        launches ? 0 : 1, g->keys_alt, p.idx, g->keys_tmp,
+                                                        g->vals_alt, g->hist, g->digit_tot, flags, g->sync, g->clist,
+                                                        g->changed, g->dests, g->removed);
+    }
+    if (launches)
+        launch_radix_passes(ctx, g, N, g->keys_alt, p.idx, g->keys_tmp, g->vals_alt, true,
+                            clear_old ? p.hash : nullptr);
+}
+
+// What the reorder reads of the re-sort: on the incremental path (flags[3] == 2) the sorted destinations
+// of the changed particles, the changed particles (key, position) in that order and the removed
+// positions, else the sorted keys and sources.  It writes the sorted keys and sources of the incremental
+// path, and clears the re-sort's counters for the next step.
+struct ResortView {
+    const int *old_keys;
+    int *keys, *src;                 // sorted keys and sources: read (full sort) or written (incremental)
+    const int *dests, *removed;
+    const int2 *changed;
+    int *sync;
+};
+
+// number of entries of the ascending list a[0..m) below x, by the lanes of a wavefront (all 64 of them,
+// x uniform): one load per 64-fold step
+__device__ __forceinline__ int wave_lower_bound(const int *__restrict__ a, int m, int x) {
+    const int lane = (int)__lane_id();
+    const int stride = (m + 63) >> 6;
+    int first = 0;
+    if (stride > 1) {
+        const bool below = lane * stride < m && a[lane * stride] < x;
+        const int c = __popcll(__ballot(below));
+        if (c == 0) return 0;
+        first = (c - 1) * stride;
+    }
+    const int left = m - first < stride ? m - first : stride;
+    const int span = stride > 1 ? left : m;
+    return first + __popcll(__ballot(lane < span && a[first + (lane < span ? lane : 0)] < x));
+}
+
+// the same for entries a[j] - j, by one lane
+__device__ __forceinline__ int lower_bound_lane(const int *__restrict__ a, int m, int x, bool minus_j) {
     int lo = 0, hi = m;
     while (lo < hi) {
         const int mid = (lo + hi) >> 1;
-        if (csorted[mid] < ck) lo = mid + 1;
+        if (a[mid] - (minus_j ? mid : 0) < x) lo = mid + 1;
         else hi = mid;
     }
-    const int dest = i - changed_before(cmask, wlocal, bprefix, i, N, m) + lo;
-    if ((unsigned)dest >= (unsigned)N) {
-        atomicOr(&flags[0], 2);
+    return lo;
+}
+
+// source s and key h of sorted position i on the incremental path, by one lane
+__device__ __forceinline__ void resort_source_lane(const ResortView &v, int m, int N, int i, int &h, int &s) {
+    const int a = lower_bound_lane(v.dests, m, i, false);
+    if (a < m && v.dests[a] == i) {
+        const int2 e = v.changed[a];
+        h = e.x;
+        s = e.y;
         return;
     }
-    keys_out[dest] = key;
-    idx_out[dest] = i;
+    const int k = i - a;                                             // rank among the unchanged
+    s = k + lower_bound_lane(v.removed, m, k + 1, true);
+    h = (unsigned)s < (unsigned)N ? v.old_keys[s] : -1;
 }
 
-__global__ void k_copy_keys_if_full(const int *__restrict__ src, int *__restrict__ dst, int N, const int *mode) {
-    if (*mode != 1) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < N; i += gridDim.x * blockDim.x) dst[i] = src[i];
-}
-
-static void launch_resort_radix(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, int passes);
-
-// Re-sort of the step: new keys and the permutation end in p.hash / p.idx (as launch_radix_sort);
-// the full-sort fallback by one workgroup (one launch) when asked and N allows, else the multi-block
-// radix sort
-void launch_resort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, bool one_block_fallback,
-                   sphfem_tool *tool) {
-    const int N = (int)p.N;
-    const int nb = nblk(N, SORT_TILE);
-    int *flags = ctx->d_flags;
-    {
-        KTimer t(ctx, tool ? "hash_tool_begin" : "hash");
-        const int tb = tool ? nblk(std::max(std::max(tool->n_nodes, tool->n_seg), 1), HASH_BS) : 0;
-        k_hash_mark<<<nb + tb, HASH_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, g->keys_alt,
-                                                          g->cell_start, g->first_sort ? 0 : 1, N, g->num_cell,
-                                                          g->hist, nb, flags, g->cmask, g->wprefix, g->bprefix,
-                                                          tool ? *tool : sphfem_tool{}, tb, 0.5 * ctx->c.dt);
+// source s and key h of sorted position i = i0 + lane, and the key hp of position i - 1, for a whole
+// wavefront (every lane executes this; lanes past N get sources that are not used).  Most wavefronts lie
+// between two changes: one shift for all lanes, found by two wavefront-wide searches.
+__device__ __forceinline__ void resort_source(const ResortView &v, const int *__restrict__ flags, int N, int i, int &h,
+                                              int &s, int &hp) {
+    const int lane = (int)__lane_id();
+    const int i0 = __builtin_amdgcn_readfirstlane(i);
+    const bool in = i < N;
+    if (flags[3] != 2) {
+        h = in ? v.keys[i] : 0;
+        s = in ? v.src[i] : 0;
+        hp = __shfl_up(h, 1);
+        if (lane == 0 && i > 0) hp = v.keys[i - 1];
+        return;
     }
-    // re-sort mode (full or incremental), then the full stable radix sort in mode 1: unsorted keys
-    // are in keys_alt
-    const int cap = std::min(g->resort_limit, SPHFEM_RESORT_CAP);
-    const int force_full = (g->first_sort || cap <= 0) ? 1 : 0;
-    const int passes = (g->key_bits + 7) / 8;
-    if (one_block_fallback && N <= SPHFEM_SORT_ONE_BLOCK_MAX) {
-        KTimer t(ctx, "resort_one_block");
-        k_sort_one_block<<<1, SORT_BS, 0, ctx->stream>>>(g->keys_alt, p.hash, p.idx, g->keys_alt, g->vals_alt, N,
-                                                         passes, flags, g->bprefix, nb, force_full, cap, g->cmask,
-                                                         g->wprefix, g->csorted, g->cdest);
+    const int m = flags[4];
+    const int lo = i0 > 0 ? i0 - 1 : 0;
+    const int last = i0 + 63 < N ? i0 + 63 : N - 1;
+    const int a = wave_lower_bound(v.dests, m, lo);
+    const int next = a < m ? v.dests[a] : N;
+    // removed positions up to the unchanged of rank lo - a: of the ascending removed[j] - j, those <= it
+    const int k0 = lo - a;
+    int b = 0;
+    {
+        const int stride = (m + 63) >> 6;
+        int first = 0;
+        bool none = m == 0;
+        if (stride > 1) {
+            const int j = lane * stride;
+            const int c = __popcll(__ballot(j < m && v.removed[j] - j <= k0));
+            none = c == 0;
+            first = none ? 0 : (c - 1) * stride;
+        }
+        const int span = stride > 1 ? (m - first < stride ? m - first : stride) : m;
+        const int j = first + (lane < span ? lane : 0);
+        const int c = __popcll(__ballot(!none && lane < span && v.removed[j] - j <= k0));
+        b = none ? 0 : first + c;
+    }
+    const int next_gone = b < m ? v.removed[b] - b : N;
+    if (next > last && next_gone > last - a) {
+        s = i - a + b;
+        h = in && (unsigned)s < (unsigned)N ? v.old_keys[s] : -1;
+        hp = __shfl_up(h, 1);
+        const int sp = i - 1 - a + b;
+        if (lane == 0 && i > 0) hp = (unsigned)sp < (unsigned)N ? v.old_keys[sp] : -1;
     } else {
-        {
-            KTimer t(ctx, "resort_scan");
-            k_resort_scan<<<1, RESORT_SCAN_BS, 0, ctx->stream>>>(g->bprefix, nb, flags, force_full, cap);
-        }
-        launch_resort_radix(ctx, g, p, passes);
-        // incremental path (mode 2)
-        {
-            KTimer t(ctx, "resort_compact");
-            k_resort_compact<<<nblk(N, 256), 256, 0, ctx->stream>>>(g->keys_alt, N, g->cmask, g->wprefix,
-                                                                    g->bprefix, g->clist, flags);
-        }
-        {
-            KTimer t(ctx, "resort_rank");
-            k_resort_rank<<<1, RESORT_SCAN_BS, 0, ctx->stream>>>(g->clist, p.hash, N, g->cmask, g->wprefix,
-                                                                  g->bprefix, g->csorted, g->cdest, flags);
-        }
+        h = -1;
+        s = 0;
+        if (in) resort_source_lane(v, m, N, i, h, s);
+        hp = __shfl_up(h, 1);
+        int sp = 0;
+        if (lane == 0 && i > 0) resort_source_lane(v, m, N, i - 1, hp, sp);
     }
-    {
-        KTimer t(ctx, "resort_scatter");
-        k_resort_scatter<<<nblk(N, 256), 256, 0, ctx->stream>>>(g->keys_alt, N, g->cmask, g->wprefix, g->bprefix,
-                                                                g->csorted, g->cdest, p.hash, p.idx, flags);
-    }
-}
-
-// the multi-block fallback of launch_resort: per pass an upsweep (pass 0's histogram came with the
-// hash), the digit scan and the downsweep, each returning at once on the incremental path
-static void launch_resort_radix(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, int passes) {
-    const int N = (int)p.N;
-    const int nb = nblk(N, SORT_TILE);
-    int *flags = ctx->d_flags;
-    const int *mode = flags + 3;
-    int *kbuf[2] = {p.hash, g->keys_alt};
-    int *vbuf[2] = {p.idx, g->vals_alt};
-    int src = 1;
-    if (passes % 2 == 0) {
-        KTimer t(ctx, "radix_copy");
-        k_copy_keys_if_full<<<std::min(nblk(N, 256), 2048), 256, 0, ctx->stream>>>(g->keys_alt, p.hash, N, mode);
-        src = 0;
-    }
-    int *kin = kbuf[src], *vin = nullptr;
-    for (int ps = 0; ps < passes; ps++) {
-        const int shift = 8 * ps;
-        const int dst = 1 - src;
-        if (ps > 0) {
-            KTimer t(ctx, "radix_upsweep");
-            k_upsweep<<<nb, SORT_BS, 0, ctx->stream>>>(kin, N, shift, g->hist, nb, mode);
-        }
-        {
-            KTimer t(ctx, "radix_scan");
-            k_scan_digits<<<RADIX, SORT_BS, 0, ctx->stream>>>(g->hist, nb, g->digit_tot, mode);
-        }
-        {
-            KTimer t(ctx, "radix_downsweep");
-            k_downsweep<<<nb, SORT_BS, 0, ctx->stream>>>(kin, ps == 0 ? nullptr : vin, kbuf[dst], vbuf[dst], N,
-                                                         shift, g->hist, nb, g->digit_tot, flags, mode);
-        }
-        kin = kbuf[dst];
-        vin = vbuf[dst];
-        src = dst;
+    if (in) {
+        v.keys[i] = h;
+        v.src[i] = s;
     }
 }
 
@@ -964,7 +1000,7 @@ void launch_bbox(sphfem_ctx *ctx, const sphfem_particles &p, double *part, doubl
 // p.hash must hold the keys; leaves the sorted keys in p.hash, the gathered arrays in place and
 // the dense cell table in the grid
 void launch_rothlin_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p) {
-    launch_radix_sort(ctx, g, p, false, g->perm);
+    launch_radix_sort(ctx, g, p, g->perm);
     {
         KTimer t(ctx, "rothlin_gather");
         k_rothlin_gather<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(p, g->buf, g->perm, ctx->d_flags);
@@ -1057,22 +1093,30 @@ void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_ce
     k_records_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, num_cell, ctx->d_flags, rec);
 }
 
-// cell boundaries of the sorted keys (grid_gpu_green.cu:13-51); false if the key or the source
-// index is out of range (flagged)
-__device__ __forceinline__ bool cell_bounds(const sphfem_particles &p, int i, int N, int num_cell,
+// source and key of sorted position i (from the re-sort's lists, or the sorted arrays when there are
+// none) and the cell boundaries (grid_gpu_green.cu:13-51); false if the position, the key or the source
+// is out of range (flagged).  Every lane of the workgroup calls it.
+__device__ __forceinline__ bool cell_bounds(const sphfem_particles &p, const ResortView &rs, int i, int N, int num_cell,
                                             int *__restrict__ cell_start, int *__restrict__ cell_end,
                                             int *__restrict__ flags, int &h, int &s) {
-    h = p.hash[i];
-    s = p.idx[i];
+    int hp = -1;
+    if (rs.keys) {
+        resort_source(rs, flags, N, i, h, s, hp);
+        if (i < RS_USED) rs.sync[i] = 0;           // k_resort has read them
+    } else {
+        h = i < N ? p.hash[i] : 0;
+        s = i < N ? p.idx[i] : 0;
+        hp = __shfl_up(h, 1);
+        if (__lane_id() == 0 && i > 0 && i < N) hp = p.hash[i - 1];
+    }
+    if (i >= N) return false;
     if ((unsigned)h >= (unsigned)num_cell || (unsigned)s >= (unsigned)N) {
         atomicOr(&flags[0], 4);
         return false;
     }
-    int hp = __shfl_up(h, 1);
-    if (__lane_id() == 0 && i > 0) hp = p.hash[i - 1];
     if (i == 0 || h != hp) {
         cell_start[h] = i;
-        if (i > 0) cell_end[hp] = i;
+        if (i > 0 && (unsigned)hp < (unsigned)num_cell) cell_end[hp] = i;
     }
     if (i == N - 1) cell_end[h] = i + 1;
     return true;
@@ -1089,12 +1133,11 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
                                                          double *__restrict__ rho_init, double *__restrict__ T_init,
                                                          int num_cell, int *__restrict__ flags,
                                                          double *__restrict__ pre_vol,
-                                                         sphfem_double4 *__restrict__ pre_s) {
+                                                         sphfem_double4 *__restrict__ pre_s, ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
-    if (i >= N) return;
     int h, s;
-    if (!cell_bounds(p, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
+    if (!cell_bounds(p, rs, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
     sphfem_double2 pos = p.pos[s], vel = p.vel[s];
     sphfem_double4 S = p.S[s];
     double rho = p.rho[s], T = p.T[s];
@@ -1161,12 +1204,12 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
 __global__ void __launch_bounds__(256) k_reorder_records(DevConsts c, const sphfem_particles p,
                                                          int *__restrict__ cell_start, int *__restrict__ cell_end,
                                                          int num_cell, int *__restrict__ flags,
-                                                         float4 *__restrict__ rec, const RateView rates) {
+                                                         float4 *__restrict__ rec, const RateView rates,
+                                                         ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
-    if (i >= N) return;
     int h, s;
-    if (!cell_bounds(p, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
+    if (!cell_bounds(p, rs, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
     sphfem_double2 pos = ld_stream(&p.pos[s]), vel = ld_stream(&p.vel[s]);
     sphfem_double4 S = ld_stream(&p.S[s]);
     double rho = ld_stream(&p.rho[s]), T = ld_stream(&p.T[s]);
@@ -1200,18 +1243,20 @@ __global__ void __launch_bounds__(256) k_reorder_records(DevConsts c, const sphf
 }
 
 void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, sphfem_leap_frog *lf,
-                            const RateView *rates) {
+                            const RateView *rates, bool resorted) {
+    ResortView rs{};
+    if (resorted) rs = ResortView{p.hash, g->keys_alt, p.idx, g->dests, g->removed, g->changed, g->sync};
     if (lf->precision == SPHFEM_FP32C) {
         KTimer t(ctx, "reorder_records");
         k_reorder_records<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, g->cell_start, g->cell_end,
-                                                                   g->num_cell, ctx->d_flags, lf->rec, *rates);
+                                                                   g->num_cell, ctx->d_flags, lf->rec, *rates, rs);
         return;
     }
     KTimer t(ctx, "reorder_predict");
     k_reorder_predict<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, g->buf, g->cell_start, g->cell_end,
                                                                lf->pos_init, lf->vel_init, lf->S_init,
                                                                lf->rho_init, lf->T_init, g->num_cell,
-                                                               ctx->d_flags, lf->pre_vol, lf->pre_s);
+                                                               ctx->d_flags, lf->pre_vol, lf->pre_s, rs);
 }
 
 }  // namespace sphfem
