@@ -1229,6 +1229,9 @@ int sphfem_tool_create(sphfem_ctx *ctx, const sphfem_tool_desc *d, sphfem_tool *
         }
         t->sink_keys = dalloc<unsigned long long>(2ul * SPHFEM_SEG_SINK_CAP);
         t->sink_vals = dalloc<double>(8ul * SPHFEM_SEG_SINK_CAP);
+        t->T_half = dalloc<double>(nn);
+        t->robin = dalloc<sphfem_double2>(ns);
+        t->pos_shift = dalloc<sphfem_double2>(nn);
         SPHFEM_HIP_CHECK(hipStreamSynchronize(s));
         *out = t;
         return SPHFEM_OK;
@@ -1248,7 +1251,7 @@ int sphfem_tool_destroy(sphfem_ctx *ctx, sphfem_tool *t) {
         dfree(t->layer_new); dfree(t->nnz_layer_ptr); dfree(t->nnz_layer); dfree(t->node_layer_ptr);
         dfree(t->node_layer); dfree(t->kin); dfree(t->node_flags); dfree(t->dir_node); dfree(t->dir_ptr);
         dfree(t->dir_entry); dfree(t->pos_map); dfree(t->T_map); dfree(t->bk_ptr); dfree(t->bk_list);
-        dfree(t->sink_keys); dfree(t->sink_vals);
+        dfree(t->sink_keys); dfree(t->sink_vals); dfree(t->T_half); dfree(t->robin); dfree(t->pos_shift);
         delete[] t->h_elem;
         delete t;
         return SPHFEM_OK;
@@ -1800,12 +1803,7 @@ static int step_body(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_particles *p,
         swap_fused(*p, g->buf);
     }
     if (t) {
-        if (ctx->c.wear_pro) {
-            launch_tool_fem_end_wear(ctx, t);      // the wear reads the new temperatures, before the motion
-            launch_tool_move(ctx, t, ctx->c.dt, true, true);
-        } else {
-            launch_tool_fem_end_move(ctx, t);
-        }
+        launch_tool_end(ctx, t);
         launch_near_contact(ctx, *p, t, lf);
     }
     return SPHFEM_OK;

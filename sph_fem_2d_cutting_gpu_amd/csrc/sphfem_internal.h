@@ -35,7 +35,9 @@
 // interactions_monaghan's own two switches of the same kind, used in turn by its calls: a call's first
 // kernel sets one and clears the other for the next call (each is read by the call's second kernel)
 #define SPHFEM_FLAG_MONAGHAN 8
-#define SPHFEM_NUM_FLAGS 10
+// workgroups of the near-tool pass that are done; zero between launches
+#define SPHFEM_FLAG_NEAR_DONE 10
+#define SPHFEM_NUM_FLAGS 11
 // position records a wavefront of the staged FP32C pair kernel copies into LDS (8 KiB)
 #define SPHFEM_STAGE_CAP 512
 // blocks of the report_force reduction (its partials: 2 doubles per block) and the largest particle
@@ -194,6 +196,11 @@ struct sphfem_tool {
     int n_layer = 0;
     int *layer_elems = nullptr;        // [n_layer] element ids in (colour, element) order
     double *layer_old = nullptr, *layer_new = nullptr;   // [n_layer * 10] mass + 3x3 stiffness
+    // workspaces of a step: half-step temperatures [n_nodes]; per segment the Robin inputs of the step's
+    // start, {contact particle temperature, length} or length -1 without contact [n_seg]; the worn node
+    // positions before the tool moves [n_nodes]
+    double *T_half = nullptr;
+    sphfem_double2 *robin = nullptr, *pos_shift = nullptr;
     int *nnz_layer_ptr = nullptr;      // [nnz + 1] CSR over layer contributions (layer slot * 16 + a*3+b)
     int *nnz_layer = nullptr;
     int *node_layer_ptr = nullptr;     // [n_nodes + 1]
@@ -394,10 +401,11 @@ __device__ __forceinline__ void step_counters_clear(int *counters) {
     counters[SPHFEM_FLAG_NONFINITE] = 0;
 }
 
-// the start of a step for the FEM tool, item i of max(nodes, segments): reset_FEM_server's
-// T_old = T and calculate_temp(0.5 dt) for the nodes; zero the wear accumulators
-// (segments_wear_rate_reset) and, item 0, the near-list and segment-sink counters and the
-// window-form switch of the pair kernels
+// the start of a step for the FEM tool, item i of max(nodes, segments): reset_FEM_server's T_old = T and
+// calculate_temp(0.5 dt) for the nodes, into T_half; the Robin inputs of the segments (which the previous
+// step's contact left), then their accumulators cleared (segments_wear_rate_reset, and the heat exchange
+// for this step's contact); item 0, the near-list and segment-sink counters and the window-form switch
+// of the pair kernels
 __device__ __forceinline__ void tool_begin_item(const sphfem_tool &t, double half_dt, int *counters, int i) {
     if (i == 0) {
         step_counters_clear(counters);
@@ -407,21 +415,23 @@ __device__ __forceinline__ void tool_begin_item(const sphfem_tool &t, double hal
     if (i < t.n_nodes) {
         double T = t.T[i];
         t.T_old[i] = T;
-        t.T[i] = half_dt * t.k[i] + T;
+        t.T_half[i] = half_dt * t.k[i] + T;
     }
     if (i < t.n_seg) {
+        const sphfem_double2 he = t.heat_exchange[i], l = t.left[i], r = t.right[i];
+        const double ddx = l.x - r.x, ddy = l.y - r.y;
+        const double dist = (double)(float)sqrt((double)(float)(ddx * ddx + ddy * ddy));
+        t.robin[i] = he.y == 0 ? sphfem_double2{0., -1.} : sphfem_double2{he.x / he.y, dist};
+        t.heat_exchange[i] = {0., 0.};
         t.wear_rate[i] = {0., 0.};
         t.wear_nodes[i] = 0.;
         t.physical_para[i] = {0., 0., 0., 0.};
         t.sliding_force[i] = 0.;
     }
 }
-void launch_tool_fem_end(sphfem_ctx *ctx, sphfem_tool *t);
+// the FEM tool's end of a step: friction-heat sums, temperatures, wear, motion
+void launch_tool_end(sphfem_ctx *ctx, sphfem_tool *t);
 void launch_tool_move(sphfem_ctx *ctx, sphfem_tool *t, double dt, bool segments, bool nodes);
-// launch_tool_fem_end then launch_tool_move(dt, segments, nodes), the temperature update and the motion
-// in one launch (the step without wear)
-void launch_tool_fem_end_move(sphfem_ctx *ctx, sphfem_tool *t);
-void launch_tool_fem_end_wear(sphfem_ctx *ctx, sphfem_tool *t);
 void launch_wear(sphfem_ctx *ctx, sphfem_tool *t);
 void launch_remesh_low_level(sphfem_ctx *ctx, sphfem_tool *t, int freq, const ElemBuckets &b);
 void launch_interp_new(sphfem_ctx *ctx, const sphfem_tool *old_t, const sphfem_double2 *new_pos, int n_new,
@@ -432,8 +442,6 @@ void launch_fem_robin(sphfem_ctx *ctx, sphfem_tool *t);
 void launch_fem_rate(sphfem_ctx *ctx, sphfem_tool *t);
 void launch_wear_reset(sphfem_ctx *ctx, sphfem_tool *t);
 void launch_near_contact(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_tool *t, sphfem_leap_frog *lf);
-// the ordered segment sums of the friction-heat records (after the pass that produced them)
-void launch_fric_heat_sums(sphfem_ctx *ctx, sphfem_tool *t);
 
 // rigid tool (sphfem_rigid.hip)
 void launch_rigid_advance(sphfem_ctx *ctx, sphfem_rigid_tool *rt);

@@ -1283,7 +1283,7 @@ void launch_fused_update(sphfem_ctx *ctx, const sphfem_particles &B, const sphfe
     const int skip = skip_contact ? 1 : 0;
     ToolView tv{};
     if (t) {
-        tv.T_nodes = t->T;
+        tv.T_nodes = t->T_half;
         tv.marks = t->marks;
         tv.fric_heat = t->fric_heat;
         tv.physical_para = t->physical_para;
@@ -1315,7 +1315,6 @@ void launch_fused_update(sphfem_ctx *ctx, const sphfem_particles &B, const sphfe
         const int pk = lf->tuning.pair_kernel;
         if (pk == SPHFEM_PAIRS_LIST_FUSED || pk == SPHFEM_PAIRS_STAGED_FUSED) {
             launch_pairs_fp32c_tuned(ctx, B, lf, cs, ce, &u);
-            if (t) launch_fric_heat_sums(ctx, t);
             return;
         }
         launch_pairs_fp32c_tuned(ctx, B, lf, cs, ce);
@@ -1353,7 +1352,6 @@ void launch_fused_update(sphfem_ctx *ctx, const sphfem_particles &B, const sphfe
         }
 #undef SPHFEM_UPDATE
     }
-    if (t) launch_fric_heat_sums(ctx, t);     // the friction-heat segment sums, in particle order
 }
 
 // FP32C derivative carry <-> the particle arrays' FP64 rates, and its gather by a permutation

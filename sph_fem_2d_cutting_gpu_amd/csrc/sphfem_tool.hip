@@ -14,7 +14,15 @@ namespace sphfem {
 // FEM heat conduction
 // ---------------------------------------------------------------------------------------------
 
-// Robin contribution of segment s to the rhs and to the stiffness diagonal (FEM_thermal_gpu.cu:342-384)
+// Robin contribution of segment s to the rhs and to the stiffness diagonal (FEM_thermal_gpu.cu:342-384);
+// in the step the contact temperature and the length come from the step's start (t.robin) and the
+// friction heat from its caller
+__device__ __forceinline__ void robin_add(const DevConsts &c, double T_cont_particle, double dist, double fric_eng,
+                                          double &f, double &kd) {
+    f += 0.5 * c.tc.h * dist * T_cont_particle + 0.5 * fric_eng;
+    kd += c.tc.h * (0.5 * dist);
+}
+
 __device__ __forceinline__ bool robin_term(const DevConsts &c, const sphfem_tool &t, int s, double &df, double &dk) {
     sphfem_double2 he = t.heat_exchange[s];
     if (he.y == 0) return false;
@@ -38,40 +46,11 @@ void launch_tool_begin(sphfem_ctx *ctx, sphfem_tool *t) {
     k_tool_begin<<<nblk(n, 256), 256, 0, ctx->stream>>>(*t, 0.5 * ctx->c.dt, ctx->d_flags);
 }
 
-// k = M^-1 (f + robin - (K + robin_diag) T), one row per thread (FEM_thermal_gpu.cu:443-458 with
-// the Robin terms of :342-384 applied to the copies f_temp / K_temp of reset_FEM_server)
-__global__ void __launch_bounds__(256) k_fem_rate_fused(DevConsts c, sphfem_tool t) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= t.n_nodes) return;
-    double f = t.f[i];
-    double kd = t.K[t.diag[i]];
-    int2 rs = t.node_robin[i];
-    double df, dk;
-    if (rs.x >= 0 && robin_term(c, t, rs.x, df, dk)) { f += df; kd += dk; }
-    if (rs.y >= 0 && robin_term(c, t, rs.y, df, dk)) { f += df; kd += dk; }
-    double buffer = 0.;
-    const int dg = t.diag[i];
-    for (int k = t.row_ptr[i]; k < t.row_ptr[i + 1]; k++) {
-        double kv = (k == dg) ? kd : t.K[k];
-        buffer += kv * t.T[t.col_ind[k]];
-    }
-    t.k[i] = t.Minv[i] * (f - buffer);
-}
-
 // calculate_temp (FEM_thermal_gpu.cu:460-468)
 __global__ void __launch_bounds__(256) k_fem_temp(sphfem_tool t, double dt) {
     int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= t.n_nodes) return;
     t.T[i] = dt * t.k[i] + t.T_old[i];
-}
-
-void launch_tool_fem_end(sphfem_ctx *ctx, sphfem_tool *t) {
-    {
-        KTimer tm(ctx, "fem_rate");
-        k_fem_rate_fused<<<nblk(t->n_nodes, 256), 256, 0, ctx->stream>>>(ctx->c, *t);
-    }
-    KTimer tm(ctx, "fem_temp");
-    k_fem_temp<<<nblk(t->n_nodes, 256), 256, 0, ctx->stream>>>(*t, ctx->c.dt);
 }
 
 // drop-in pieces: reset_FEM_server, apply_robin_bdc, calculate_temp_rate, calculate_temp
@@ -136,21 +115,26 @@ void launch_wear_reset(sphfem_ctx *ctx, sphfem_tool *t) {
 // ---------------------------------------------------------------------------------------------
 // tool_FEM.cu:1552-1570 for segment and node i with the step's kinematics k (read by every item
 // before item 0 rewrites them; the motion uses vel and flank_retreat, which the rewrite keeps)
+__device__ __forceinline__ void segment_move(const sphfem_tool &t, const ToolKin &k, double dt, int i, sphfem_double2 l,
+                                             sphfem_double2 r) {
+    t.left[i] = {l.x + k.vel_x * dt, l.y + k.vel_y * dt + k.flank_retreat};
+    t.right[i] = {r.x + k.vel_x * dt, r.y + k.vel_y * dt + k.flank_retreat};
+}
+
+__device__ __forceinline__ void node_move(const sphfem_tool &t, const ToolKin &k, double dt, int i, sphfem_double2 p) {
+    p.x += k.vel_x * dt;
+    p.y += k.vel_y * dt + k.flank_retreat;
+    t.pos[i] = p;
+}
+
 __device__ __forceinline__ void tool_move_item(const sphfem_tool &t, const ToolKin &k, double dt, int do_segments,
                                                int do_nodes, int i) {
     if (do_segments && i < t.n_seg) {
-        sphfem_double2 l = t.left[i], r = t.right[i];
-        t.left[i] = {l.x + k.vel_x * dt, l.y + k.vel_y * dt + k.flank_retreat};
-        t.right[i] = {r.x + k.vel_x * dt, r.y + k.vel_y * dt + k.flank_retreat};
+        segment_move(t, k, dt, i, t.left[i], t.right[i]);
         t.heat_exchange[i] = {0., 0.};
         t.fric_heat[i] = 0.;
     }
-    if (do_nodes && i < t.n_nodes) {
-        sphfem_double2 p = t.pos[i];
-        p.x += k.vel_x * dt;
-        p.y += k.vel_y * dt + k.flank_retreat;
-        t.pos[i] = p;
-    }
+    if (do_nodes && i < t.n_nodes) node_move(t, k, dt, i, t.pos[i]);
 }
 
 __device__ __forceinline__ void tool_move_kinematics(const sphfem_tool &t, const ToolKin &k, double dt) {
@@ -174,26 +158,6 @@ __global__ void __launch_bounds__(256) k_tool_move(sphfem_tool t, double dt, int
     if (do_nodes && i == 0) tool_move_kinematics(t, k, dt);
 }
 
-// k_fem_temp and k_tool_move in one launch (the step without wear: nothing between them reads the
-// temperatures or moves the tool otherwise); the same per-item arithmetic
-__global__ void __launch_bounds__(256) k_fem_temp_tool_move(sphfem_tool t, double dt) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const ToolKin k = *t.kin;
-    if (i < t.n_nodes) t.T[i] = dt * t.k[i] + t.T_old[i];
-    tool_move_item(t, k, dt, 1, 1, i);
-    if (i == 0) tool_move_kinematics(t, k, dt);
-}
-
-void launch_tool_fem_end_move(sphfem_ctx *ctx, sphfem_tool *t) {
-    {
-        KTimer tm(ctx, "fem_rate");
-        k_fem_rate_fused<<<nblk(t->n_nodes, 256), 256, 0, ctx->stream>>>(ctx->c, *t);
-    }
-    KTimer tm(ctx, "fem_temp_tool_move");
-    const int n = std::max(std::max(t->n_nodes, t->n_seg), 1);
-    k_fem_temp_tool_move<<<nblk(n, 256), 256, 0, ctx->stream>>>(*t, ctx->c.dt);
-}
-
 void launch_tool_move(sphfem_ctx *ctx, sphfem_tool *t, double dt, bool segments, bool nodes) {
     int n = std::max(std::max(t->n_nodes, t->n_seg), 1);
     KTimer tm(ctx, "tool_move");
@@ -205,9 +169,8 @@ void launch_tool_move(sphfem_ctx *ctx, sphfem_tool *t, double dt, bool segments,
 // ---------------------------------------------------------------------------------------------
 
 // element matrices of FEM_thermal_gpu.cu:71-109, 126-152 (Ke[a][b] = row a, column b)
-__device__ __forceinline__ void element_matrices(const DevConsts &c, const sphfem_tool &t, int e, double *out) {
-    sphfem_int4 el = t.elem[e];
-    sphfem_double2 p0 = t.pos[el.x], p1 = t.pos[el.y], p2 = t.pos[el.z];
+__device__ __forceinline__ void element_matrices_at(const DevConsts &c, sphfem_double2 p0, sphfem_double2 p1,
+                                                    sphfem_double2 p2, double *out) {
     double j00 = p1.x - p0.x, j01 = p1.y - p0.y;
     double j10 = p2.x - p0.x, j11 = p2.y - p0.y;
     double det = fabs(j00 * j11 - j10 * j01);
@@ -225,6 +188,11 @@ __device__ __forceinline__ void element_matrices(const DevConsts &c, const sphfe
     double s = (w * 3.) * (c.tc.k * det);
     for (int a = 0; a < 3; a++)
         for (int b = 0; b < 3; b++) out[1 + 3 * a + b] = (s * G0[a]) * G0[b] + (s * G1[a]) * G1[b];
+}
+
+__device__ __forceinline__ void element_matrices(const DevConsts &c, const sphfem_tool &t, int e, double *out) {
+    const sphfem_int4 el = t.elem[e];
+    element_matrices_at(c, t.pos[el.x], t.pos[el.y], t.pos[el.z], out);
 }
 
 __global__ void k_layer_mats(DevConsts c, sphfem_tool t, double *dst) {
@@ -261,17 +229,9 @@ __device__ __forceinline__ bool segment_wear(const DevConsts &c, const sphfem_to
 }
 
 // nodal shift: each node gathers the shifts of its segments in segment order
-__global__ void k_nodal_shift(DevConsts c, sphfem_tool t) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < t.n_seg) {
-        double wl, wr;
-        if (segment_wear(c, t, i, wl, wr)) t.wear_nodes[i] = (wl + wr) / c.dt;
-    }
-    if (i >= t.n_nodes) return;
-    int a = t.node_shift_ptr[i], b = t.node_shift_ptr[i + 1];
-    if (a == b) return;
+__device__ __forceinline__ sphfem_double2 shifted_node(const DevConsts &c, const sphfem_tool &t, int i) {
     sphfem_double2 p = t.pos[i];
-    for (int q = a; q < b; q++) {
+    for (int q = t.node_shift_ptr[i]; q < t.node_shift_ptr[i + 1]; q++) {
         int2 e = t.node_shift[q];
         double wl, wr;
         if (!segment_wear(c, t, e.x, wl, wr)) continue;
@@ -280,13 +240,24 @@ __global__ void k_nodal_shift(DevConsts c, sphfem_tool t) {
         p.x += nn.x * w;
         p.y += nn.y * w;
     }
-    t.pos[i] = p;
+    return p;
+}
+
+__device__ __forceinline__ void segment_wear_nodes(const DevConsts &c, const sphfem_tool &t, int i) {
+    double wl, wr;
+    if (segment_wear(c, t, i, wl, wr)) t.wear_nodes[i] = (wl + wr) / c.dt;
+}
+
+__global__ void k_nodal_shift(DevConsts c, sphfem_tool t) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < t.n_seg) segment_wear_nodes(c, t, i);
+    if (i >= t.n_nodes) return;
+    if (t.node_shift_ptr[i] != t.node_shift_ptr[i + 1]) t.pos[i] = shifted_node(c, t, i);
 }
 
 // K, M: subtract the old and add the new boundary-layer element matrices in (colour, element)
 // order (mesh_retreat_wear / mesh_resume_wear), then M^-1 (do_inverse_mass_matrix_lumped)
-__global__ void k_wear_assemble(sphfem_tool t) {
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+__device__ __forceinline__ void wear_assemble_item(const sphfem_tool &t, int i) {
     if (i < t.nnz) {
         int a = t.nnz_layer_ptr[i], b = t.nnz_layer_ptr[i + 1];
         if (a != b) {
@@ -314,6 +285,15 @@ __global__ void k_wear_assemble(sphfem_tool t) {
     }
 }
 
+__global__ void k_wear_assemble(sphfem_tool t) { wear_assemble_item(t, blockIdx.x * blockDim.x + threadIdx.x); }
+
+// inward normal of the segment lp -> rp (glm::normalize)
+__device__ __forceinline__ sphfem_double2 segment_normal(sphfem_double2 lp, sphfem_double2 rp) {
+    double vx = rp.y - lp.y, vy = -(rp.x - lp.x);
+    double inv = 1. / sqrt(vx * vx + vy * vy);
+    return {vx * inv, vy * inv};
+}
+
 // segment_wear_update (tool_FEM.cu:520-548) and correct_flank_contact (:559-587) for any number of
 // segments: one block, min over left.y
 __global__ void __launch_bounds__(1024) k_segment_wear_update(sphfem_tool t) {
@@ -324,9 +304,7 @@ __global__ void __launch_bounds__(1024) k_segment_wear_update(sphfem_tool t) {
         sphfem_double2 lp = t.pos[mk.z], rp = t.pos[mk.w];
         t.left[s] = lp;
         t.right[s] = rp;
-        double vx = rp.y - lp.y, vy = -(rp.x - lp.x);
-        double inv = 1. / sqrt(vx * vx + vy * vy);
-        t.n[s] = {vx * inv, vy * inv};
+        t.n[s] = segment_normal(lp, rp);
         mn = fmin(mn, lp.y);
     }
     red[threadIdx.x] = mn;
@@ -338,48 +316,62 @@ __global__ void __launch_bounds__(1024) k_segment_wear_update(sphfem_tool t) {
     if (threadIdx.x == 0) t.kin->flank_retreat = t.kin->flank_contact - red[0];
 }
 
-// the wear step after the old boundary-layer matrices: node shift, new matrices, K/M update,
-// segment geometry
-static void launch_wear_rest(sphfem_ctx *ctx, sphfem_tool *t) {
+// wear_adjustment as an entry point of its own, function by function
+void launch_wear(sphfem_ctx *ctx, sphfem_tool *t) {
+    KTimer tm(ctx, "wear");
     const int nl = std::max(t->n_layer, 1);
+    k_layer_mats<<<nblk(nl, 128), 128, 0, ctx->stream>>>(ctx->c, *t, t->layer_old);
     k_nodal_shift<<<nblk(std::max(t->n_nodes, t->n_seg), 256), 256, 0, ctx->stream>>>(ctx->c, *t);
     k_layer_mats<<<nblk(nl, 128), 128, 0, ctx->stream>>>(ctx->c, *t, t->layer_new);
     k_wear_assemble<<<nblk(std::max(t->nnz, t->n_nodes), 256), 256, 0, ctx->stream>>>(*t);
     k_segment_wear_update<<<1, 1024, 0, ctx->stream>>>(*t);
 }
 
-void launch_wear(sphfem_ctx *ctx, sphfem_tool *t) {
-    KTimer tm(ctx, "wear");
-    const int nl = std::max(t->n_layer, 1);
-    k_layer_mats<<<nblk(nl, 128), 128, 0, ctx->stream>>>(ctx->c, *t, t->layer_old);
-    launch_wear_rest(ctx, t);
-}
-
-// k_fem_temp and the wear step's old boundary-layer matrices in one launch: the matrices read the
-// node positions and constants only, the temperature update writes the temperatures only (the
-// same per-item arithmetic as the two kernels)
-__global__ void __launch_bounds__(256) k_fem_temp_layer_mats(DevConsts c, sphfem_tool t, double dt) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < t.n_nodes) t.T[i] = dt * t.k[i] + t.T_old[i];
+// The step's wear in two launches (five, and the tool's motion, as entry points; every launch of the
+// tool's chain waits for the one before, about 4.7 us each at any mesh size here).  First: the shifted
+// node positions into pos_shift, the new boundary-layer matrices from positions each element shifts for
+// itself, the segments' wear, and (last workgroup) the flank retreat from the shifted segment ends.
+__global__ void __launch_bounds__(256) k_wear_shift(DevConsts c, sphfem_tool t) {
+    if (blockIdx.x == gridDim.x - 1) {
+        __shared__ double red[256];
+        double mn = SPHFEM_FLT_MAX;
+        for (int s = threadIdx.x; s < t.n_seg; s += 256) mn = fmin(mn, shifted_node(c, t, t.marks[s].z).y);
+        red[threadIdx.x] = mn;
+        __syncthreads();
+        for (int w = 128; w > 0; w >>= 1) {
+            if ((int)threadIdx.x < w) red[threadIdx.x] = fmin(red[threadIdx.x], red[threadIdx.x + w]);
+            __syncthreads();
+        }
+        if (threadIdx.x == 0) t.kin->flank_retreat = t.kin->flank_contact - red[0];
+        return;
+    }
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < t.n_seg) segment_wear_nodes(c, t, i);
+    if (i < t.n_nodes) t.pos_shift[i] = shifted_node(c, t, i);
     if (i < t.n_layer) {
+        const sphfem_int4 el = t.elem[t.layer_elems[i]];
         double m[10];
-        element_matrices(c, t, t.layer_elems[i], m);
-        for (int q = 0; q < 10; q++) t.layer_old[(long)i * 10 + q] = m[q];
+        element_matrices_at(c, shifted_node(c, t, el.x), shifted_node(c, t, el.y), shifted_node(c, t, el.z), m);
+        for (int q = 0; q < 10; q++) t.layer_new[(long)i * 10 + q] = m[q];
     }
 }
 
-// the FEM tool's end of a step with wear: temperature rate, then the temperature update with the
-// old layer matrices, then the rest of the wear step (launch_tool_fem_end + launch_wear, one launch
-// fewer)
-void launch_tool_fem_end_wear(sphfem_ctx *ctx, sphfem_tool *t) {
-    {
-        KTimer tm(ctx, "fem_rate");
-        k_fem_rate_fused<<<nblk(t->n_nodes, 256), 256, 0, ctx->stream>>>(ctx->c, *t);
+// Second: K, M and M^-1, the segments' geometry from the shifted nodes, and the tool's motion (which
+// reads the velocity and the flank retreat that its last item keeps).
+__global__ void __launch_bounds__(256) k_wear_finish_move(sphfem_tool t, double dt) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const ToolKin k = *t.kin;
+    wear_assemble_item(t, i);
+    if (i < t.n_seg) {
+        const sphfem_int4 mk = t.marks[i];
+        const sphfem_double2 lp = t.pos_shift[mk.z], rp = t.pos_shift[mk.w];
+        t.n[i] = segment_normal(lp, rp);
+        segment_move(t, k, dt, i, lp, rp);
+        t.heat_exchange[i] = {0., 0.};
+        t.fric_heat[i] = 0.;
     }
-    KTimer tm(ctx, "fem_temp_wear");
-    const int n = std::max(std::max(t->n_nodes, t->n_layer), 1);
-    k_fem_temp_layer_mats<<<nblk(n, 256), 256, 0, ctx->stream>>>(ctx->c, *t, ctx->c.dt);
-    launch_wear_rest(ctx, t);
+    if (i < t.n_nodes) node_move(t, k, dt, i, t.pos_shift[i]);
+    if (i == 0) tool_move_kinematics(t, k, dt);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -617,6 +609,8 @@ __global__ void __launch_bounds__(256) k_fric_heat(DevConsts c, sphfem_particles
     P.T[i] = T;
 }
 
+static void launch_fric_heat_sums(sphfem_ctx *ctx, sphfem_tool *t);
+
 void launch_fric_heat(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_tool *t) {
     launch_fill_int(ctx, ctx->d_flags + SPHFEM_FLAG_SINK_FRIC, 1, 0);
     {
@@ -685,85 +679,198 @@ struct SegDst {
     int stride[6];
 };
 
-constexpr int SEG_REDUCE_BS = 1024;
-constexpr int SEG_REDUCE_PER = SPHFEM_SEG_SINK_CAP / SEG_REDUCE_BS;   // records per thread, at most
-static_assert(SPHFEM_SEG_SINK_CAP % SEG_REDUCE_BS == 0, "sink capacity: whole records per thread");
+struct SegLds {
+    unsigned long long sk[SPHFEM_SEG_SINK_CAP];   // keys; after the sort, one value per record
+    unsigned short sl[SPHFEM_SEG_SINK_CAP];       // record slots in sorted order
+    int sseg[SPHFEM_SEG_SINK_CAP];                // segments in sorted order
+};
 
-template <int NV>
-__global__ void __launch_bounds__(SEG_REDUCE_BS) k_segment_reduce(SegSink s, SegDst d) {
-    __shared__ unsigned long long sk[SPHFEM_SEG_SINK_CAP];   // keys; after the sort, one value per record
-    __shared__ int sl[SPHFEM_SEG_SINK_CAP];                  // record slots
-    __shared__ int sseg[SPHFEM_SEG_SINK_CAP];                // segments in sorted order
-    const int n = min(*s.count, s.cap);
-    if (n <= 0) return;
+// segments and slots of the n records in sorted order, by a workgroup of BS: ranks by counting while one
+// record per lane suffices (the usual few hundred: 1 us against 3 us at 256), else a bitonic sort
+template <int BS> __device__ __forceinline__ void seg_order(const SegSink &s, int n, SegLds &l) {
+    const int tid = threadIdx.x;
+    if (n <= BS) {
+        const unsigned long long key = tid < n ? s.keys[tid] : ~0ull;
+        if (tid < n) l.sk[tid] = key;
+        __syncthreads();
+        int rank = 0;
+        for (int q = 0; q < n; q++) rank += l.sk[q] < key;
+        if (tid < n) {
+            l.sl[rank] = (unsigned short)tid;
+            l.sseg[rank] = (int)(unsigned)(key >> 32);
+        }
+        __syncthreads();
+        return;
+    }
     int np = 1;
     while (np < n) np <<= 1;
-    for (int k = threadIdx.x; k < np; k += SEG_REDUCE_BS) {
-        sk[k] = k < n ? s.keys[k] : ~0ull;
-        sl[k] = k;
+    for (int k = tid; k < np; k += BS) {
+        l.sk[k] = k < n ? s.keys[k] : ~0ull;
+        l.sl[k] = (unsigned short)k;
     }
     __syncthreads();
     for (int size = 2; size <= np; size <<= 1) {          // bitonic sort of (key, slot), ascending
         for (int stride = size >> 1; stride > 0; stride >>= 1) {
-            for (int k = threadIdx.x; k < np; k += SEG_REDUCE_BS) {
+            for (int k = tid; k < np; k += BS) {
                 const int j = k ^ stride;
                 if (j > k) {
                     const bool up = (k & size) == 0;
-                    const unsigned long long a = sk[k], b = sk[j];
+                    const unsigned long long a = l.sk[k], b = l.sk[j];
                     if ((a > b) == up) {
-                        sk[k] = b;
-                        sk[j] = a;
-                        const int x = sl[k];
-                        sl[k] = sl[j];
-                        sl[j] = x;
+                        l.sk[k] = b;
+                        l.sk[j] = a;
+                        const unsigned short x = l.sl[k];
+                        l.sl[k] = l.sl[j];
+                        l.sl[j] = x;
                     }
                 }
             }
             __syncthreads();
         }
     }
-    for (int k = threadIdx.x; k < n; k += SEG_REDUCE_BS) sseg[k] = (int)(unsigned)(sk[k] >> 32);
+    for (int k = tid; k < n; k += BS) l.sseg[k] = (int)(unsigned)(l.sk[k] >> 32);
     __syncthreads();
-    // every global load of the additions is issued here, before the first is used: the values of
-    // this thread's records (sorted positions threadIdx.x + u * block) and, for a record that
-    // starts its segment's run, the segment's current sums (one memory wait instead of one per value)
-    double v[NV][SEG_REDUCE_PER], acc0[NV][SEG_REDUCE_PER];
-    int seg_of[SEG_REDUCE_PER];
-    bool head[SEG_REDUCE_PER];
+}
+
+// adds values Q0 .. Q0 + NV - 1 of the ordered records, PER records per lane.  Every global load of the
+// additions is issued before the first is used: the values of this lane's records and, for a record
+// that starts its segment's run, the segment's current sums (one memory wait instead of one per value)
+template <int Q0, int NV, int BS, int PER>
+__device__ __forceinline__ void seg_add(const SegSink &s, int n, SegLds &l, const SegDst &d) {
+    double v[NV][PER], acc0[NV][PER];
+    int seg_of[PER];
+    bool head[PER];
 #pragma unroll
-    for (int u = 0; u < SEG_REDUCE_PER; u++) {
-        const int k = threadIdx.x + u * SEG_REDUCE_BS;
+    for (int u = 0; u < PER; u++) {
+        const int k = threadIdx.x + u * BS;
         const bool in = k < n;
-        const int slot = in ? sl[k] : 0;
-        const int seg = in ? sseg[k] : 0;
+        const int slot = in ? l.sl[k] : 0;
+        const int seg = in ? l.sseg[k] : 0;
         seg_of[u] = seg;
-        head[u] = in && (k == 0 || sseg[k - 1] != seg);
+        head[u] = in && (k == 0 || l.sseg[k - 1] != seg);
 #pragma unroll
         for (int q = 0; q < NV; q++) {
-            v[q][u] = in ? s.vals[(size_t)q * s.cap + slot] : 0.;
-            acc0[q][u] = head[u] ? d.p[q][(size_t)seg * d.stride[q]] : 0.;
+            v[q][u] = in ? s.vals[(size_t)(Q0 + q) * s.cap + slot] : 0.;
+            acc0[q][u] = head[u] ? d.p[Q0 + q][(size_t)seg * d.stride[Q0 + q]] : 0.;
         }
     }
-    double *vbuf = reinterpret_cast<double *>(sk);
+    double *vbuf = reinterpret_cast<double *>(l.sk);
 #pragma unroll
     for (int q = 0; q < NV; q++) {
         // this value of every record in sorted order, then each segment's run added in order by
-        // the run's first thread (from LDS: long runs stay cheap)
+        // the run's first lane (from LDS: long runs stay cheap)
 #pragma unroll
-        for (int u = 0; u < SEG_REDUCE_PER; u++) {
-            const int k = threadIdx.x + u * SEG_REDUCE_BS;
+        for (int u = 0; u < PER; u++) {
+            const int k = threadIdx.x + u * BS;
             if (k < n) vbuf[k] = v[q][u];
         }
         __syncthreads();
 #pragma unroll
-        for (int u = 0; u < SEG_REDUCE_PER; u++) {
+        for (int u = 0; u < PER; u++) {
             if (!head[u]) continue;
-            const int k = threadIdx.x + u * SEG_REDUCE_BS;
+            const int k = threadIdx.x + u * BS;
             double acc = acc0[q][u];
-            for (int r = k; r < n && sseg[r] == seg_of[u]; r++) acc += vbuf[r];
-            d.p[q][(size_t)seg_of[u] * d.stride[q]] = acc;
+            for (int r = k; r < n && l.sseg[r] == seg_of[u]; r++) acc += vbuf[r];
+            d.p[Q0 + q][(size_t)seg_of[u] * d.stride[Q0 + q]] = acc;
         }
         __syncthreads();
+    }
+}
+
+template <int Q0, int NV, int BS> __device__ __forceinline__ void seg_sums(const SegSink &s, int n, SegLds &l, const SegDst &d) {
+    static_assert(SPHFEM_SEG_SINK_CAP % BS == 0, "sink capacity: whole records per lane");
+    seg_order<BS>(s, n, l);
+    if (n <= BS) seg_add<Q0, NV, BS, 1>(s, n, l, d);
+    else seg_add<Q0, NV, BS, SPHFEM_SEG_SINK_CAP / BS>(s, n, l, d);
+}
+
+constexpr int SEG_REDUCE_BS = 1024;
+template <int NV>
+__global__ void __launch_bounds__(SEG_REDUCE_BS) k_segment_reduce(SegSink s, SegDst d) {
+    __shared__ SegLds l;
+    const int n = min(*s.count, s.cap);
+    if (n <= 0) return;
+    seg_sums<0, NV, SEG_REDUCE_BS>(s, n, l, d);
+}
+
+// The FEM tool's end of a step in one launch: the friction heat's ordered segment sums, the temperature
+// rate k = M^-1 (f + robin - (K + robin_diag) T) (one row per lane, FEM_thermal_gpu.cu:443-458 with the
+// Robin terms of :342-384), the temperature update (:460-468) and, without wear, the tool's motion or,
+// with wear, the old boundary-layer matrices.  The rate reads the half-step temperatures from T_half, so
+// the update writes T while other rows still read; the Robin terms read the contact temperatures and
+// lengths of the step's start, so the segments may move.  Only the workgroups that hold contact nodes
+// order the friction records, each for itself; the last workgroup adds the wear inputs (physical_para,
+// sliding_force).  The friction heat's own sums are spent here and not written: the step clears them.
+// Latency bound: three launches of 8.6 + 5.8 + 4.7 us at 160k particles before.
+constexpr int TOOL_END_BS = 512;
+template <bool WEAR>
+__global__ void __launch_bounds__(TOOL_END_BS) k_tool_end(DevConsts c, sphfem_tool t, SegSink fr, SegDst d, double dt) {
+    __shared__ SegLds l;
+    const int n = min(*fr.count, fr.cap);
+    if (blockIdx.x == gridDim.x - 1) {
+        if (n > 0) seg_sums<1, 5, TOOL_END_BS>(fr, n, l, d);
+        return;
+    }
+    const int i = blockIdx.x * TOOL_END_BS + threadIdx.x;
+    const bool node = i < t.n_nodes;
+    const int2 rs = node ? t.node_robin[i] : make_int2(-1, -1);
+    // the row's entries are loaded before the records are ordered (most rows have 5 to 8)
+    constexpr int ROW = 10;
+    const int r0 = node ? t.row_ptr[i] : 0, r1 = node ? t.row_ptr[i + 1] : 0;
+    const int dg = node ? t.diag[i] : 0;
+    double kv[ROW], Tv[ROW];
+#pragma unroll
+    for (int q = 0; q < ROW; q++) {
+        kv[q] = r0 + q < r1 ? t.K[r0 + q] : 0.;
+        Tv[q] = r0 + q < r1 ? t.T_half[t.col_ind[r0 + q]] : 0.;
+    }
+    if (__syncthreads_or(n > 0 && rs.x >= 0)) {
+        seg_order<TOOL_END_BS>(fr, n, l);
+        double *vbuf = reinterpret_cast<double *>(l.sk);
+        for (int k = threadIdx.x; k < n; k += TOOL_END_BS) vbuf[k] = fr.vals[l.sl[k]];
+        __syncthreads();
+    }
+    const ToolKin kin = *t.kin;
+    if (node) {
+        double f = t.f[i];
+        double kd = t.K[dg];
+        const int seg[2] = {rs.x, rs.y};
+        for (int q = 0; q < 2; q++) {
+            if (seg[q] < 0) continue;
+            const sphfem_double2 rb = t.robin[seg[q]];
+            if (rb.y == -1.) continue;                   // no contact at the step's start
+            double fric = t.fric_heat[seg[q]];
+            if (n > 0) {
+                int lo = 0, hi = n;
+                while (lo < hi) {
+                    const int mid = (lo + hi) >> 1;
+                    if (l.sseg[mid] < seg[q]) lo = mid + 1;
+                    else hi = mid;
+                }
+                const double *vbuf = reinterpret_cast<const double *>(l.sk);
+                for (; lo < n && l.sseg[lo] == seg[q]; lo++) fric += vbuf[lo];
+            }
+            robin_add(c, rb.x, rb.y, fric, f, kd);
+        }
+        double buffer = 0.;
+#pragma unroll
+        for (int q = 0; q < ROW; q++)
+            if (r0 + q < r1) buffer += (r0 + q == dg ? kd : kv[q]) * Tv[q];
+        for (int k = r0 + ROW; k < r1; k++) buffer += (k == dg ? kd : t.K[k]) * t.T_half[t.col_ind[k]];
+        const double rate = t.Minv[i] * (f - buffer);
+        t.k[i] = rate;
+        t.T[i] = dt * rate + t.T_old[i];
+        if constexpr (!WEAR) node_move(t, kin, dt, i, t.pos[i]);
+    }
+    if constexpr (WEAR) {
+        if (i < t.n_layer) {
+            double m[10];
+            element_matrices(c, t, t.layer_elems[i], m);
+            for (int q = 0; q < 10; q++) t.layer_old[(long)i * 10 + q] = m[q];
+        }
+    } else {
+        if (i < t.n_seg) segment_move(t, kin, dt, i, t.left[i], t.right[i]);
+        if (i == 0) tool_move_kinematics(t, kin, dt);
     }
 }
 
@@ -774,7 +881,7 @@ static SegSink host_sink(sphfem_ctx *ctx, sphfem_tool *t, bool s2) {
     return SegSink{ctx->d_flags + SPHFEM_FLAG_SINK_FRIC, t->sink_keys, t->sink_vals, SPHFEM_SEG_SINK_CAP};
 }
 
-void launch_fric_heat_sums(sphfem_ctx *ctx, sphfem_tool *t) {
+static SegDst fric_dst(sphfem_tool *t) {
     SegDst d{};
     d.p[0] = t->fric_heat;
     d.p[1] = &t->physical_para[0].x;
@@ -784,17 +891,46 @@ void launch_fric_heat_sums(sphfem_ctx *ctx, sphfem_tool *t) {
     d.p[5] = t->sliding_force;
     const int st[6] = {1, 4, 4, 4, 4, 1};
     for (int q = 0; q < 6; q++) d.stride[q] = st[q];
+    return d;
+}
+
+__host__ __device__ static inline SegDst s2_dst(const sphfem_tool &t) {
+    SegDst d{};
+    d.p[0] = &t.heat_exchange[0].x;
+    d.p[1] = &t.heat_exchange[0].y;
+    d.stride[0] = d.stride[1] = 2;
+    return d;
+}
+
+static void launch_fric_heat_sums(sphfem_ctx *ctx, sphfem_tool *t) {
     KTimer tm(ctx, "fric_heat_sums");
-    k_segment_reduce<6><<<1, SEG_REDUCE_BS, 0, ctx->stream>>>(host_sink(ctx, t, false), d);
+    k_segment_reduce<6><<<1, SEG_REDUCE_BS, 0, ctx->stream>>>(host_sink(ctx, t, false), fric_dst(t));
 }
 
 static void launch_s2_sums(sphfem_ctx *ctx, sphfem_tool *t) {
-    SegDst d{};
-    d.p[0] = &t->heat_exchange[0].x;
-    d.p[1] = &t->heat_exchange[0].y;
-    d.stride[0] = d.stride[1] = 2;
     KTimer tm(ctx, "contact_s2_sums");
-    k_segment_reduce<2><<<1, SEG_REDUCE_BS, 0, ctx->stream>>>(host_sink(ctx, t, true), d);
+    k_segment_reduce<2><<<1, SEG_REDUCE_BS, 0, ctx->stream>>>(host_sink(ctx, t, true), s2_dst(*t));
+}
+
+void launch_tool_end(sphfem_ctx *ctx, sphfem_tool *t) {
+    const double dt = ctx->c.dt;
+    const bool wear = ctx->c.wear_pro != 0;
+    {
+        KTimer tm(ctx, "tool_end");
+        const int n = std::max(std::max(t->n_nodes, wear ? t->n_layer : t->n_seg), 1);
+        const int blocks = nblk(n, TOOL_END_BS) + 1;
+        if (wear)
+            k_tool_end<true><<<blocks, TOOL_END_BS, 0, ctx->stream>>>(ctx->c, *t, host_sink(ctx, t, false), fric_dst(t),
+                                                                      dt);
+        else
+            k_tool_end<false><<<blocks, TOOL_END_BS, 0, ctx->stream>>>(ctx->c, *t, host_sink(ctx, t, false),
+                                                                       fric_dst(t), dt);
+    }
+    if (!wear) return;
+    KTimer tm(ctx, "wear");
+    const int n = std::max(std::max(t->n_nodes, t->n_seg), t->n_layer);
+    k_wear_shift<<<nblk(n, 256) + 1, 256, 0, ctx->stream>>>(ctx->c, *t);
+    k_wear_finish_move<<<nblk(std::max(std::max(t->nnz, t->n_nodes), t->n_seg), 256), 256, 0, ctx->stream>>>(*t, dt);
 }
 
 void launch_contact(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_tool *t) {
@@ -815,10 +951,19 @@ void launch_contact(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_tool *t) 
 // the tool's temperatures, so it follows s1 in the same lane), and the thermal boundary condition
 // and the invalidation.
 // use32: the rates are the FP32 derivative carry r32 of the FP32C form (the particle arrays' FP64
-// rates are not maintained by its steps)
-__global__ void __launch_bounds__(256) k_near_contact(DevConsts c, sphfem_particles P, sphfem_tool t,
+// rates are not maintained by its steps).
+// The workgroup that finishes last adds the heat exchange's ordered segment sums (a launch of its own,
+// 6 us, before); workgroups without records only count themselves.  The friction heat, whose sums
+// k_tool_end has used, is cleared here.
+constexpr int NEAR_BS = 512;
+__global__ void __launch_bounds__(NEAR_BS) k_near_contact(DevConsts c, sphfem_particles P, sphfem_tool t,
                                                       const int *__restrict__ near_list, int *counters,
                                                       RateView r32, int use32) {
+    __shared__ SegLds l;
+    __shared__ int s_records, s_last;
+    if (threadIdx.x == 0) s_records = 0;
+    __syncthreads();
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < t.n_seg; i += gridDim.x * blockDim.x) t.fric_heat[i] = 0.;
     // one particle of the near list per wavefront (wave-uniform loop); the segment loops of
     // contact s1 run over the lanes
     const int count = counters[1];
@@ -882,6 +1027,7 @@ __global__ void __launch_bounds__(256) k_near_contact(DevConsts c, sphfem_partic
             // contact s2 (actions_gpu.cu:585-617; one lane, its sink record slot from a one-lane ballot)
             double T = P.T[i];
             contact_s2_one(c, t, s2_sink(t, counters), i, seg, P.rho[i], T);
+            s_records = 1;
             if (c.thermal_bc && P.fixed[i] == 1.) T = c.trml_wp.T_init;
             P.T[i] = T;
         } else if (c.thermal_bc && P.fixed[i] == 1.) {
@@ -890,18 +1036,31 @@ __global__ void __launch_bounds__(256) k_near_contact(DevConsts c, sphfem_partic
         if (bad) blanked = 1.;
         if (blanked == 1.) P.blanked[i] = 1.;
     }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (s_records) __threadfence();               // this workgroup's records, before it counts
+        s_last = atomicAdd(&counters[SPHFEM_FLAG_NEAR_DONE], 1) == (int)gridDim.x - 1;
+        if (s_last) __threadfence();                  // the other workgroups' records
+    }
+    __syncthreads();
+    if (__builtin_amdgcn_readfirstlane(s_last) == 0) return;
+    const SegSink sink = s2_sink(t, counters);
+    const int n = min(__hip_atomic_load(sink.count, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), sink.cap);
+    if (threadIdx.x == 0) counters[SPHFEM_FLAG_NEAR_DONE] = 0;
+    if (n > 0) seg_sums<0, 2, NEAR_BS>(sink, n, l, s2_dst(t));
 }
 
 void launch_near_contact(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_tool *t, sphfem_leap_frog *lf) {
-    int blocks = std::max(1, std::min(nblk(p.N, 256), 1024));
+    // about a wavefront per near particle (some 200 of 6,400 particles, 1,000 of 160k, 2,000 of 4M lie near
+    // the tool); more workgroups than that only keep other streams' work off the CUs
+    const int blocks = std::max(32, std::min(nblk(p.N, 1024), 256));
     {
         KTimer tm(ctx, "near_contact");
         const bool use32 = lf->rates_fp32;
         const RateView r32 = use32 ? rate_view(lf->rate32[lf->rate_cur], lf->num_part) : RateView{};
-        k_near_contact<<<blocks, 256, 0, ctx->stream>>>(ctx->c, p, *t, lf->near_list, ctx->d_flags, r32,
+        k_near_contact<<<blocks, NEAR_BS, 0, ctx->stream>>>(ctx->c, p, *t, lf->near_list, ctx->d_flags, r32,
                                                         use32 ? 1 : 0);
     }
-    launch_s2_sums(ctx, t);
 }
 
 }  // namespace sphfem
