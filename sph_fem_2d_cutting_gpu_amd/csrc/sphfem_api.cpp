@@ -1654,9 +1654,7 @@ int sphfem_leap_frog_set_precision(sphfem_ctx *ctx, sphfem_leap_frog *lf, int pr
             // neighbour records are addressed by 32-bit byte offsets (16 B each)
             if (lf->num_part >= (1u << 28)) return fail(ctx, SPHFEM_ERR_RANGE, "FP32C supports < 2^28 particles");
             if (!lf->rec) {
-                // record blocks r0 [N + 4], r1, r2, r3 [N]; the padding of r0 is zeroed once
-                lf->rec = dalloc<float4>(4ul * lf->num_part + 4);
-                SPHFEM_HIP_CHECK(hipMemsetAsync(lf->rec + lf->num_part, 0, 4 * sizeof(float4), ctx->stream));
+                lf->rec = dalloc<float4>(sphfem::rec_float4s(lf->num_part));
             }
             if (!lf->psum) lf->psum = dalloc<float4>(2ul * lf->num_part);
             if (!lf->psum_T) lf->psum_T = dalloc<float>(lf->num_part);

@@ -20,8 +20,13 @@
 #define SPHFEM_RESORT_SYNC 16
 // blocks of the bounding-box reduction of an unlocked grid
 #define SPHFEM_BBOX_BLOCKS 1024
-// d_flags slot set by the reorder when a live particle carries a non-finite pair input (the pair
-// kernels then use the reference's full 5x5-cell window) and cleared by the update kernel
+// d_flags slot set by the reorder and cleared by the update kernel: the form of the pair sums.  WINDOW: a
+// live particle carries a non-finite pair input, the pair kernels use the reference's full 5x5-cell
+// window.  FP32C only: WIDTH, one has a kernel width other than the cell size; AWAY, one is neither near
+// the cell that it is sorted into nor one column height above or below it
+#define SPHFEM_FORM_WINDOW 1
+#define SPHFEM_FORM_WIDTH 2
+#define SPHFEM_FORM_AWAY 4
 #define SPHFEM_FLAG_NONFINITE 5
 // densities whose sums, reciprocals and quotients are normal numbers; a live particle outside them
 // switches the FP64 pair sums to the window form and its plain divisions
@@ -99,6 +104,34 @@ inline RateView rate_view(float *base, size_t n) {
     r.rho_t = base + 8 * n;
     r.T_t = base + 9 * n;
     return r;
+}
+
+// FP32C neighbour records (written by the reorder kernel) of n sorted particles, SoA blocks so that a
+// wavefront's gather of one field stays within few cache lines:
+//   pos[j] = position in units of cell / 2^SPHFEM_POS_BITS from the grid's corner, modulo 2^32 (padded by
+//            4 records); 8 cells aside for blanked particles and outside the grid's rows (write_records)
+//   r1[j] = {vx, vy, (Sxx - p)/rho^2, Sxy/rho^2}     r2[j] = {(Syy - p)/rho^2, Rxx, Rxy, Ryy}
+//   r3[j] = {+-mass/rho, rho, sqrt(K/rho), T - T_init}
+//   h[j]    = kernel width (read where it is not the cell size)
+//   away[j] = position in the units of pos, unwrapped (written for live particles whose pos lies aside)
+// The volume is stored negative for tool particles, the sound speed of blanked ones is -1.
+#define SPHFEM_POS_BITS 28
+struct RecView {
+    float4 *r1, *r2, *r3;
+    int2 *pos;
+    float *h;
+    double2 *away;
+};
+inline size_t rec_float4s(size_t n) { return 4 * n + (n + 5) / 2 + (n + 3) / 4; }
+inline RecView rec_view(float4 *base, size_t n) {
+    RecView v;
+    v.r1 = base;
+    v.r2 = base + n;
+    v.r3 = base + 2 * n;
+    v.away = reinterpret_cast<double2 *>(base + 3 * n);
+    v.pos = reinterpret_cast<int2 *>(base + 4 * n);
+    v.h = reinterpret_cast<float *>(base + 4 * n + (n + 5) / 2);
+    return v;
 }
 
 // FP64 pair sums of one particle (interactions_gpu.cu:143-379 outputs, T as the Laplacian)
@@ -257,9 +290,7 @@ struct sphfem_leap_frog {
     sphfem::PairSums *psum64 = nullptr;   // FP64 form: pair sums of the sorted particles
     int *near_list = nullptr;      // [num_part] particles near the tool
     bool intermediates = false;    // also write S_der / v_der in the fused step
-    // FP32C neighbour records of the sorted predicted state, SoA blocks r0 [num_part + 4],
-    // r1, r2, r3 [num_part]: {x, y relative to the cell corner, cell row, h},
-    // {vx, vy, (Sxx-p)/rho^2, Sxy/rho^2}, {(Syy-p)/rho^2, R}, {+-mass/rho, rho, sqrt(K/rho), T - T_init}
+    // FP32C neighbour records of the sorted predicted state (rec_view)
     float4 *rec = nullptr;
     // FP32C pair sums of the sorted particles: [0] velocity gradient (xx, xy, yx, yy),
     // [1] stress-divergence + viscous acceleration (x, y), XSPH velocity (x, y); psum_T: Laplacian of T
@@ -366,7 +397,7 @@ void launch_reorder_full(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles
 // sorted order comes from launch_resort, not from p.hash and p.idx
 void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, sphfem_leap_frog *lf,
                             const RateView *rates, bool resorted);
-void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, float4 *rec);
+void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, const RecView &rec);
 
 // particles (sphfem_particles.hip)
 void launch_actions(sphfem_ctx *ctx, int which, const sphfem_particles &p);

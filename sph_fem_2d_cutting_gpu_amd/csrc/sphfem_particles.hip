@@ -173,51 +173,50 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
 // FP32-compensated form
 // ---------------------------------------------------------------------------------------------
 
-// FP32C neighbour records (written by the reorder kernel), four SoA blocks of float4:
-//   r0[j] = {x - cell corner x, y - cell corner y, cell row, h}   (block padded by 4 records)
-//   r1[j] = {vx, vy, (Sxx - p)/rho^2, Sxy/rho^2}     r2[j] = {(Syy - p)/rho^2, Rxx, Rxy, Ryy}
-//   r3[j] = {+-mass/rho, rho, sqrt(K/rho), T - T_init}
-// The volume is stored negative for tool particles; blanked particles have x = 1e30.  SoA keeps a
-// wavefront's gather of one field within few cache lines.
-struct RecView {
-    const float4 *__restrict__ r0;
-    const float4 *__restrict__ r1;
-    const float4 *__restrict__ r2;
-    const float4 *__restrict__ r3;
-};
-
-// record load at a 32-bit byte offset from a uniform base (one VGPR offset, no 64-bit address math)
+// the record at a 32-bit byte offset from a uniform base (one VGPR offset, no 64-bit address math)
 __device__ __forceinline__ float4 ldrec(const float4 *__restrict__ base, unsigned byte_off) {
     return *reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(base) + byte_off);
 }
+__device__ __forceinline__ int2 ldpos(const int2 *__restrict__ base, unsigned byte_off) {
+    return *reinterpret_cast<const int2 *>(reinterpret_cast<const char *>(base) + byte_off);
+}
+// two position records from an 8-byte-aligned address
+typedef int sphfem_v4i __attribute__((ext_vector_type(4), aligned(8)));
 
-// Where the pair loops read the neighbours' position records (r0) from: HBM through L1 (the list
-// kernel), or a wavefront's copy of its five columns' windows in LDS (the staged kernel).  Both give
-// the same float4 values, so the sums do not depend on the source.
-// A neighbour-list entry names the candidate's column d (0..4) and where its records are.
+// Where the pair loops read the neighbours' positions from: HBM through L1 (the list kernel), or a
+// wavefront's copy of its five columns' windows in LDS (the staged kernel).  Both give the same values,
+// so the sums do not depend on the source.  A neighbour-list entry names where its records are.
 struct GlobalPos {
-    using Entry = int;                                      // sorted index | column << 29
-    const float4 *__restrict__ r0;
-    // candidate j of column d during the scan
-    __device__ __forceinline__ float4 scan(int, int j) const { return ldrec(r0, (unsigned)j << 4); }
-    __device__ __forceinline__ Entry encode(int d, int j) const { return j | (d << 29); }
-    __device__ __forceinline__ int column(Entry e) const { return (int)((unsigned)e >> 29); }
-    __device__ __forceinline__ unsigned index(Entry e) const { return (unsigned)(e & 0x0fffffff); }
-    __device__ __forceinline__ float4 entry(Entry e) const { return ldrec(r0, index(e) << 4); }
+    using Entry = int;                                      // sorted index
+    const int2 *__restrict__ pos;
+    // candidates j .. j + 3 of column d during the scan
+    __device__ __forceinline__ void scan4(int, int j, int2 *b) const {
+        const char *at = reinterpret_cast<const char *>(pos) + ((unsigned)j << 3);
+        const sphfem_v4i u = *reinterpret_cast<const sphfem_v4i *>(at);
+        const sphfem_v4i v = *reinterpret_cast<const sphfem_v4i *>(at + 16);
+        b[0] = make_int2(u.x, u.y);
+        b[1] = make_int2(u.z, u.w);
+        b[2] = make_int2(v.x, v.y);
+        b[3] = make_int2(v.z, v.w);
+    }
+    __device__ __forceinline__ Entry encode(int, int j) const { return j; }
+    __device__ __forceinline__ unsigned index(Entry e) const { return (unsigned)e; }
+    __device__ __forceinline__ int2 entry(Entry e) const { return ldpos(pos, (unsigned)e << 3); }
     // the range a lane scans in column d, limited to what the source holds (everything here)
     __device__ __forceinline__ bool clip(int, int &, int &) const { return true; }
 };
 
 struct StagedPos {
     using Entry = unsigned short;                           // LDS slot | column << 12
-    const float4 *spos;       // LDS: the union windows of columns 0..4, one after the other
+    const int2 *spos;         // LDS: the union windows of columns 0..4, one after the other
     const int *sdelta;        // LDS: per column, sorted index minus LDS slot
     int F[5], L[5], delta[5]; // per column: staged sorted range [F, L) and its delta (uniform)
-    __device__ __forceinline__ float4 scan(int d, int j) const { return spos[j - delta[d]]; }
+    __device__ __forceinline__ void scan4(int d, int j, int2 *b) const {
+        for (int u = 0; u < 4; u++) b[u] = spos[j + u - delta[d]];
+    }
     __device__ __forceinline__ Entry encode(int d, int j) const { return (Entry)((j - delta[d]) | (d << 12)); }
-    __device__ __forceinline__ int column(Entry e) const { return (int)(e >> 12); }
     __device__ __forceinline__ unsigned index(Entry e) const { return (unsigned)((e & 0xfff) + sdelta[e >> 12]); }
-    __device__ __forceinline__ float4 entry(Entry e) const { return spos[e & 0xfff]; }
+    __device__ __forceinline__ int2 entry(Entry e) const { return spos[e & 0xfff]; }
     // a lane's window lies inside the wavefront's union by construction when the hashes are sorted;
     // otherwise the range is cut to the staged part (no access outside the LDS copy) and false
     // reports the inconsistent table
@@ -230,88 +229,119 @@ struct StagedPos {
     }
 };
 
-struct PairI {            // particle i and the per-i kernel constants
-    float fxi, fyi, rowi, hi, vxi, vyi, sxi, syi, szi, Rxi, Ryi, Rzi, rhoi, ci, Ti;
-    float h1, fac, c_out_w, c_out_g, c_in_g;
-    float fourh2, rr2min;     // the support test (used by the window form)
+// Particle i and the per-i kernel constants.  Distances D = x_i - x_j are in units u = cell / 2^28; the
+// kernel is evaluated in the dimensionless q = |D| ku, ku = u / h_i, and its dimensional factors multiply
+// the finished sums.
+struct PairI {
+    int xi, yi;
+    float vxi, vyi, sxi, syi, szi, Rxi, Ryi, Rzi, rhoi, ci, Ti;
+    float kf;                   // W (kernel / its value factor) to the artificial stress's w / wdeltap
+    float D2max, D2min;         // the support test on |D|^2
+    float beta2, alpha, eta2;   // 2 beta, alpha, eta^2 of the viscosity
     bool thermal;
-    bool mech;            // i is not a tool particle
+    bool mech;                  // i is not a tool particle
+    // general form only
+    float ku, H, D2heat;        // u / h_i, h_i / u, the heat term's least |D|^2
+    double xd, yd;              // the position where D is taken in FP64
 };
 
-struct PairAcc {          // FP32 block sums
+struct PairAcc {                // FP32 block sums
     float v0, v1, v2, v3, ax, ay, p0, p1, T;
 };
 
-template <bool WIN = false>
-__device__ __forceinline__ void pair_term(const PairI &I, float hf, float inv_wdp, float alpha, float beta,
-                                          float eta2, const float4 q0, const float4 q1, const float4 q2,
-                                          const float4 q3, int d, PairAcc &a) {
+constexpr float KU = 1.f / (float)(1 << SPHFEM_POS_BITS);      // ku where the kernel width is the cell size
+
+// one pair at distance D.  GEN: any kernel widths (h_j / u in Hj), and (win) window candidates outside the
+// support with the kernel set to 0 as in the reference; otherwise h_i = h_j = the cell size and every
+// entry lies in the support
+template <bool GEN>
+__device__ __forceinline__ void pair_term(const PairI &I, float dx, float dy, const float4 q1, const float4 q2,
+                                          const float4 q3, float Hj, bool win, PairAcc &a) {
 #pragma clang fp contract(fast)
-    const float dcol = (float)(d - 2);                          // column of j minus column of i
-    const float xij = (I.fxi - q0.x) - dcol * hf;
-    const float yij = (I.fyi - q0.y) + (I.rowi - q0.z) * hf;
-    const float rr2 = xij * xij + yij * yij;
-    const float rinv = __builtin_amdgcn_rsqf(rr2);
-    const float q = rr2 * rinv * I.h1;
-    float w, g;
-    if (q > 1.f) {
-        const float tq = 2.f - q;
-        const float tq2 = tq * tq;
-        w = I.c_out_w * (tq2 * tq2 * tq2);
-        g = I.c_out_g * tq2 * rinv;
-    } else {
-        w = I.fac * (1.f - 1.5f * q * q * (1.f - 0.5f * q));
-        g = I.c_in_g * (1.f - 0.75f * q);
-    }
-    if constexpr (WIN) {
-        // a window candidate outside the support: the reference's kernel value and gradient are 0
-        if (!(rr2 < I.fourh2 && rr2 >= I.rr2min)) {
+    const float D2 = dx * dx + dy * dy;
+    const float rinv = __builtin_amdgcn_rsqf(D2);
+    const float ku = GEN ? I.ku : KU;
+    const float q = D2 * rinv * ku;
+    const float u = 1.f - 0.5f * q;
+    const float s = u * u;
+    // value w (over fac) and radial factor g: gradient = fac / h_i * g * D
+    const bool outer = q > 1.f;
+    float w = outer ? 16.f * (s * s) * s : 1.f - 1.5f * (q * q) * u;
+    float g = outer ? (-3.f * s) * rinv : (2.25f * ku) * q - 3.f * ku;
+    if constexpr (GEN) {
+        if (win && !(D2 < I.D2max && D2 >= I.D2min)) {
             w = 0.f;
             g = 0.f;
         }
     }
-    const float wx = g * xij, wy = g * yij;
     const float volj = fabsf(q3.x);
-    if (I.thermal && rr2 > 1e-16f) a.T += volj * (I.Ti - q3.w) * g;
+    const float heat = volj * (I.Ti - q3.w) * g;
+    if constexpr (GEN) {
+        if (I.thermal && D2 > I.D2heat) a.T += heat;
+    } else {
+        a.T += heat;                                     // used only where the thermal block is set
+    }
     if (I.mech && q3.x > 0.f) {                          // neither i nor j is a tool particle
+        const float wx = g * dx, wy = g * dy;
         const float dvx = q1.x - I.vxi, dvy = q1.y - I.vyi;
         const float gx = dvx * volj, gy = dvy * volj;
         a.v0 += gx * wx;
         a.v1 += gx * wy;
         a.v2 += gy * wx;
         a.v3 += gy * wy;
-        float f = w * inv_wdp;
+        float f = w * I.kf;
         f *= f;
         f *= f;
         float Ax = (I.sxi + q1.z) + f * (I.Rxi + q2.y);
         const float Ay = (I.syi + q1.w) + f * (I.Ryi + q2.z);
         float Az = (I.szi + q2.x) + f * (I.Rzi + q2.w);
-        const float inv_rhoij = 2.f * __builtin_amdgcn_rcpf(I.rhoi + q3.y);
-        const float vp = -(dvx * xij + dvy * yij);          // (v_i - v_j) . x_ij
-        if (vp < 0.f) {
-            const float cij = 0.5f * (I.ci + q3.z);
-            const float hij = 0.5f * (I.hi + q0.w);
-            const float mu = hij * vp * __builtin_amdgcn_rcpf(rr2 + eta2 * hij * hij);
-            const float piij = mu * (beta * mu - alpha * cij) * inv_rhoij;
+        const float half_inv_rhoij = __builtin_amdgcn_rcpf(I.rhoi + q3.y);
+        const float vp = -(dvx * dx + dvy * dy);         // (v_i - v_j) . D
+        if constexpr (GEN) {
+            if (vp < 0.f) {
+                const float H = 0.5f * (I.H + Hj);
+                const float mu = H * vp * __builtin_amdgcn_rcpf(D2 + I.eta2 * H * H);
+                const float piij = mu * (I.beta2 * mu - I.alpha * (I.ci + q3.z)) * half_inv_rhoij;
+                Ax -= piij;
+                Az -= piij;
+            }
+        } else {
+            // receding pairs take mu = 0 and with it no viscous term
+            const float mu = fminf(vp, 0.f) * __builtin_amdgcn_rcpf(D2 * KU + I.eta2);
+            const float piij = mu * (I.beta2 * mu - I.alpha * (I.ci + q3.z)) * half_inv_rhoij;
             Ax -= piij;
             Az -= piij;
         }
         a.ax += Ax * wx + Ay * wy;
         a.ay += Ay * wx + Az * wy;
-        const float wr = w * inv_rhoij;
-        a.p0 -= wr * dvx;                                   // sum w / rho_ij * (v_i - v_j)
+        const float wr = w * half_inv_rhoij;
+        a.p0 -= wr * dvx;                                // sum w / (rho_i + rho_j) * (v_i - v_j)
         a.p1 -= wr * dvy;
     }
 }
 
+// the position, in units u from the grid's corner, of live record j of cell `hash` (general form)
+__device__ __forceinline__ double2 wide_pos(const RecView &rv, int ny, int j, int hash) {
+    const int2 p = rv.pos[j];
+    const int ix = hash / ny, iy = hash - ix * ny;
+    const int half = 1 << (SPHFEM_POS_BITS - 1);
+    const int rx = (int)((unsigned)p.x - ((unsigned)ix << SPHFEM_POS_BITS) - half);
+    const int ry = (int)((unsigned)p.y - ((unsigned)iy << SPHFEM_POS_BITS) - half);
+    const unsigned two = 2u << SPHFEM_POS_BITS;
+    if ((unsigned)rx + two > 2 * two || (unsigned)ry + two > 2 * two) return rv.away[j];   // not in its cell
+    const double unit = (double)(1 << SPHFEM_POS_BITS);
+    return make_double2((ix + 0.5) * unit + rx, (iy + 0.5) * unit + ry);
+}
+
 // FP32-compensated pair sums (same physics as pair_sums_fp64, different arithmetic), one lane per
 // sorted particle:
-//  * positions are cell-relative FP32 (x_ij = dx_rel + (cell_i - cell_j) * h): the pair distance
-//    carries ~1e-7 of the cell size whatever the absolute coordinates;
-//  * one v_rsq per pair (the distance), one v_rcp (2 / (rho_i + rho_j)) and one v_rcp for the
-//    viscosity denominator of approaching pairs;
-//  * the grad-T term uses e_ij . grad W / r_ij = g (the radial kernel-derivative factor): the
-//    reference's algebra without its extra sqrt and divisions;
+//  * positions are 32-bit integers in units of cell / 2^28 that wrap every 16 cells: the difference of
+//    any two particles near the cells of a 5x5 window is exact, and rounded once to FP32;
+//  * one v_rsq per pair (the distance), one v_rcp (rho_i + rho_j) and one v_rcp for the viscosity
+//    denominator; the kernel's dimensional factors and those of the equations multiply the finished sums
+//    in FP64;
+//  * the grad-T term uses e_ij . grad W / r_ij = the radial kernel-derivative factor: the reference's
+//    algebra without its extra sqrt and divisions;
 //  * each lane compacts its in-support candidates (columns in order, sorted index within a
 //    column: the reference order) into an LDS list of CHUNK entries, loading candidates four
 //    at a time, then evaluates the dense list with the records of the next entry in flight;
@@ -320,8 +350,15 @@ __device__ __forceinline__ void pair_term(const PairI &I, float hf, float inv_wd
 //    rounding on output.
 // Outputs (FP32): psum[i] = velocity gradient (xx, xy, yx, yy); psum[N + i] = (mass * stress
 // divergence - mass * viscous term) per axis, XSPH velocity per axis; psum_T[i] = Laplacian of T.
-// WIN: every non-blanked record of the 5x5 cells (blanked records sit at x = 1e30) is evaluated with
-// the kernel set to 0 outside the support, as the reference does; see pair_sums_fp64.
+// Bound by the L1's rate of cache lines per gather (a wavefront's 64 lists drift apart: some 36 lines
+// per 16-byte record, 20 per 8-byte position) and close behind by VALU issue.  Positions of 16 bytes
+// (cell-relative FP32 and the cell row, with the column in the list entry) and kernel factors applied
+// per pair took 868 us (with the update) on 4 M particles and 3337 us (sums alone) on 16 M, against 797
+// and 3010 us.
+// General form (form != 0; the SPHFEM_FORM_ bits): kernel widths other than the cell size; positions that
+// the wrapped ones cannot tell apart, taken in FP64; and the window form, where every non-blanked record
+// of the 5x5 cells is evaluated with the kernel set to 0 outside the support, as the reference does (see
+// pair_sums_fp64).
 __device__ __forceinline__ double interaction_alpha(const DevConsts &c, double is_tool) {
     // interactions_gpu.cu:164: the tool block (interactions_gpu.cu:19) is zero unless
     // interactions_setup_thermal_constants_tool set it (the rigid-tool setup does, benchmarks.cpp:518;
@@ -617,13 +654,14 @@ struct PairOut {           // one particle's FP32C sums: psum[i], psum[N + i], p
     float T;
 };
 
-template <int BS, int CHUNK, bool WIN, class Pos = GlobalPos>
-__device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const double *__restrict__ blanked,
-                                                   const int *__restrict__ hash, int N, const RecView &rv,
+template <int BS, int CHUNK, bool GEN, class Pos = GlobalPos>
+__device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int *__restrict__ hash, int N,
+                                                   const RecView &rv,
                                                    const int *__restrict__ cs, const int *__restrict__ ce, int i,
                                                    typename Pos::Entry *__restrict__ list, const Pos &pos,
-                                                   int *__restrict__ flags) {
+                                                   int *__restrict__ flags, int form) {
 #pragma clang fp contract(fast)
+    const bool win = GEN && (form & SPHFEM_FORM_WINDOW), wide = GEN && (form & ~SPHFEM_FORM_WIDTH);
     double d_v0 = 0., d_v1 = 0., d_v2 = 0., d_v3 = 0.;
     double d_ax = 0., d_ay = 0., d_p0 = 0., d_p1 = 0., d_T = 0.;
     const float4 a3 = rv.r3[i];
@@ -632,7 +670,9 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const dou
     // particles are skipped
     const bool tool_i = a3.x < 0.f;
     const double alpha_i = tool_i ? c.trml_itool.alpha : c.trml_wp.alpha;
-    if (blanked[i] != 1. && (!tool_i || alpha_i != 0.)) {
+    const double dxc = c.geom.dx;
+    const double hi = GEN ? (double)rv.h[i] : dxc;
+    if (a3.z != -1.f && (!tool_i || alpha_i != 0.)) {
         const int nx = c.geom.nx, ny = c.geom.ny;
         const int hashi = hash[i];
         const int gi = hashi / ny;
@@ -651,32 +691,57 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const dou
             cs_hi[d] = ok ? cs[c0 + high_j - 1] : -1;
             ce_hi[d] = ok ? ce[c0 + high_j - 1] : -1;
         }
-        const float4 a0 = rv.r0[i], a1 = rv.r1[i], a2 = rv.r2[i];
+        const int2 a0 = rv.pos[i];
+        const float4 a1 = rv.r1[i], a2 = rv.r2[i];
         PairI I;
-        I.fxi = a0.x; I.fyi = a0.y; I.rowi = a0.z; I.hi = a0.w;
+        I.xi = a0.x; I.yi = a0.y;
         I.vxi = a1.x; I.vyi = a1.y; I.sxi = a1.z; I.syi = a1.w;
         I.szi = a2.x; I.Rxi = a2.y; I.Ryi = a2.z; I.Rzi = a2.w;
         I.rhoi = a3.y; I.ci = a3.z; I.Ti = a3.w;
-        I.h1 = 1.f / I.hi;
-        I.fac = (float)SPHFEM_PI_FAC * I.h1 * I.h1;
-        I.c_out_w = 0.25f * I.fac;
-        I.c_out_g = -0.75f * I.h1 * I.fac;
-        I.c_in_g = -3.f * I.h1 * I.h1 * I.fac;
         I.thermal = alpha_i != 0.;
         I.mech = !tool_i;
-        const float fourh2 = 4.f * I.hi * I.hi;
-        const float rr2min = (float)c.rr2_min;
-        I.fourh2 = fourh2;
-        I.rr2min = rr2min;
-        const float hf = (float)c.geom.dx;
-        const float inv_wdp = (float)(1. / c.corr.wdeltap);
-        const float alpha = (float)c.corr.alpha, beta = (float)c.corr.beta;
-        const float eta2 = (float)(c.corr.eta * c.corr.eta);
+        I.kf = (float)(SPHFEM_PI_FAC / (hi * hi * c.corr.wdeltap));
+        const double inv_u = (double)(1 << SPHFEM_POS_BITS) / dxc;
+        I.D2min = (float)(c.rr2_min * inv_u * inv_u);
+        I.beta2 = (float)(2. * c.corr.beta);
+        I.alpha = (float)c.corr.alpha;
+        if constexpr (GEN) {
+            I.H = (float)(hi * inv_u);
+            I.ku = 1.f / I.H;
+            I.D2max = 4.f * I.H * I.H;
+            I.D2heat = (float)(1e-16 * inv_u * inv_u);
+            I.eta2 = (float)(c.corr.eta * c.corr.eta);
+            if (wide) {
+                const double2 x = wide_pos(rv, ny, i, hashi);
+                I.xd = x.x;
+                I.yd = x.y;
+            }
+        } else {
+            I.D2max = 4.f / (KU * KU);
+            I.eta2 = (float)(c.corr.eta * c.corr.eta / (double)KU);      // on the scale of D2 * KU
+        }
 
         auto flush = [&](PairAcc &a) {
             d_v0 += a.v0; d_v1 += a.v1; d_v2 += a.v2; d_v3 += a.v3;
             d_ax += a.ax; d_ay += a.ay; d_p0 += a.p0; d_p1 += a.p1; d_T += a.T;
             a = PairAcc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+        };
+        auto distance = [&](unsigned j, int2 p, float &dx, float &dy) {
+            if (GEN && wide) {
+                const double2 x = wide_pos(rv, ny, (int)j, hash[j]);
+                dx = (float)(I.xd - x.x);
+                dy = (float)(I.yd - x.y);
+            } else {
+                dx = (float)(int)((unsigned)I.xi - (unsigned)p.x);       // modulo 2^32
+                dy = (float)(int)((unsigned)I.yi - (unsigned)p.y);
+            }
+        };
+        auto term = [&](typename Pos::Entry e, const int2 q0, const float4 q1, const float4 q2, const float4 q3,
+                        PairAcc &acc) {
+            float dx, dy, Hj = 0.f;
+            distance(pos.index(e), q0, dx, dy);
+            if constexpr (GEN) Hj = (float)((double)rv.h[pos.index(e)] * inv_u);
+            pair_term<GEN>(I, dx, dy, q1, q2, q3, Hj, win, acc);
         };
         // dense list: two entries per iteration, the records of the next entry loaded before the
         // current one is evaluated (ping-pong registers, no copies); each list entry is read from LDS
@@ -687,19 +752,21 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const dou
             typename Pos::Entry eA = list[0];
             typename Pos::Entry eB = list[(1 < n ? 1 : n - 1) * BS];
             unsigned oA = pos.index(eA) << 4;
-            float4 A0 = pos.entry(eA), A1 = ldrec(rv.r1, oA), A2 = ldrec(rv.r2, oA), A3 = ldrec(rv.r3, oA);
+            int2 A0 = pos.entry(eA);
+            float4 A1 = ldrec(rv.r1, oA), A2 = ldrec(rv.r2, oA), A3 = ldrec(rv.r3, oA);
             for (int k = 0; k < n; k += 2) {
                 const typename Pos::Entry eA_next = list[(k + 2 < n ? k + 2 : n - 1) * BS];
                 const unsigned oB = pos.index(eB) << 4;
-                const float4 B0 = pos.entry(eB), B1 = ldrec(rv.r1, oB), B2 = ldrec(rv.r2, oB),
-                             B3 = ldrec(rv.r3, oB);
-                pair_term<WIN>(I, hf, inv_wdp, alpha, beta, eta2, A0, A1, A2, A3, pos.column(eA), acc);
+                const int2 B0 = pos.entry(eB);
+                const float4 B1 = ldrec(rv.r1, oB), B2 = ldrec(rv.r2, oB), B3 = ldrec(rv.r3, oB);
+                term(eA, A0, A1, A2, A3, acc);
                 if (k + 1 < n) {
                     const typename Pos::Entry eB_next = list[(k + 3 < n ? k + 3 : n - 1) * BS];
                     eA = eA_next;
                     oA = pos.index(eA) << 4;
-                    A0 = pos.entry(eA); A1 = ldrec(rv.r1, oA); A2 = ldrec(rv.r2, oA); A3 = ldrec(rv.r3, oA);
-                    pair_term<WIN>(I, hf, inv_wdp, alpha, beta, eta2, B0, B1, B2, B3, pos.column(eB), acc);
+                    A0 = pos.entry(eA);
+                    A1 = ldrec(rv.r1, oA); A2 = ldrec(rv.r2, oA); A3 = ldrec(rv.r3, oA);
+                    term(eB, B0, B1, B2, B3, acc);
                     eB = eB_next;
                 }
                 if (((k + 2) & 7) == 0) flush(acc);
@@ -721,19 +788,17 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const dou
                 if (cs[c0 + jr] != -1) last = ce[c0 + jr];
             if (last > N || first < 0) continue;                        // inconsistent cell table
             if (!pos.clip(d, first, last)) atomicOr(&flags[0], 4);
-            const float cofs = (float)(gi - col) * hf;
             for (int j = first; j < last; j += 4) {
-                // four scan records; up to three past `last` are read (both sources are padded)
-                const float4 b0 = pos.scan(d, j), b1 = pos.scan(d, j + 1), b2 = pos.scan(d, j + 2),
-                             b3 = pos.scan(d, j + 3);
-                const float4 bb[4] = {b0, b1, b2, b3};
+                // four positions; up to three past `last` are read (both sources are padded)
+                int2 b[4];
+                pos.scan4(d, j, b);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    const float xij = (I.fxi - bb[u].x) + cofs;
-                    const float yij = (I.fyi - bb[u].y) + (I.rowi - bb[u].z) * hf;
-                    const float rr2 = xij * xij + yij * yij;
-                    const bool take = WIN ? rr2 < 1e30f : (rr2 < fourh2 && rr2 >= rr2min);
-                    if (j + u < last && take) {
+                    if (GEN && (j + u >= last || rv.r3[j + u].z == -1.f)) continue;
+                    float dx, dy;
+                    distance((unsigned)(j + u), b[u], dx, dy);
+                    const float D2 = dx * dx + dy * dy;
+                    if (j + u < last && (win || (D2 < I.D2max && D2 >= I.D2min))) {
                         list[n * BS] = pos.encode(d, j + u);
                         n++;
                     }
@@ -748,12 +813,16 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const dou
         }
         run_list(n);
     }
+    // the kernel's factors fac / h (gradient), fac (value), and fac / h^2 (radial over distance: the sums
+    // hold its g in units of u / h)
     const double mass = c.phys.mass;
+    const double h1 = 1. / hi, fac = SPHFEM_PI_FAC * h1 * h1, grad = fac * h1;
+    const double ma = mass * grad, xs = -2. * c.corr.xspheps * mass * fac;
+    const double heat = 2. * grad * (double)(1 << SPHFEM_POS_BITS) / dxc;
     PairOut o;
-    o.g = make_float4((float)d_v0, (float)d_v1, (float)d_v2, (float)d_v3);
-    o.a = make_float4((float)(mass * d_ax), (float)(mass * d_ay), (float)(-c.corr.xspheps * mass * d_p0),
-                      (float)(-c.corr.xspheps * mass * d_p1));
-    o.T = (float)(2. * d_T);
+    o.g = make_float4((float)(grad * d_v0), (float)(grad * d_v1), (float)(grad * d_v2), (float)(grad * d_v3));
+    o.a = make_float4((float)(ma * d_ax), (float)(ma * d_ay), (float)(xs * d_p0), (float)(xs * d_p1));
+    o.T = (float)(heat * d_T);
     return o;
 }
 
@@ -771,25 +840,27 @@ __device__ __forceinline__ void emit_pairs(const DevConsts &c, const UpdateArgs 
     }
 }
 
-// in-support pair sums, one lane per sorted particle; when nonfinite[0] is set (a live particle
-// with a non-finite input), the window form: every record of the 5x5 cells, the kernel zeroed
-// outside the support, so the non-finite values spread as in the reference.  FUSE: each lane then
-// runs its particle's update (u) instead of writing psum.
+// in-support pair sums, one lane per sorted particle, in the form that nonfinite[0] asks for.  FUSE: each lane
+// then runs its particle's update (u) instead of writing psum.
+__device__ __forceinline__ int pairs_form(const DevConsts &c, const int *__restrict__ nonfinite) {
+    // a support that reaches below the heat term's least distance needs the test of the general form
+    return *nonfinite | (c.rr2_min > 1e-16 ? 0 : SPHFEM_FORM_WIDTH);
+}
+
 template <int BS, int CHUNK, bool FUSE = false, bool RIGID = false>
-__global__ void __launch_bounds__(BS) k_pairs_fp32c(DevConsts c, const double *__restrict__ blanked,
-                                                         const int *__restrict__ hash, int N, RecView rv,
+__global__ void __launch_bounds__(BS) k_pairs_fp32c(DevConsts c, const int *__restrict__ hash, int N, RecView rv,
                                                          const int *__restrict__ cs, const int *__restrict__ ce,
                                                          float4 *__restrict__ psum, float *__restrict__ psum_T,
                                                          const int *__restrict__ nonfinite, UpdateArgs u) {
     __shared__ int nb_list[CHUNK * BS];
-    const int win = *nonfinite;
+    const int form = pairs_form(c, nonfinite);
     const int i = xcd_logical_block() * BS + threadIdx.x;
     if (i >= N) return;
     const PairOut o =
-        win != 0 ? pairs_fp32c_one<BS, CHUNK, true>(c, blanked, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
-                                                    GlobalPos{rv.r0}, nullptr)
-                 : pairs_fp32c_one<BS, CHUNK, false>(c, blanked, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
-                                                     GlobalPos{rv.r0}, nullptr);
+        form != 0 ? pairs_fp32c_one<BS, CHUNK, true>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
+                                                     GlobalPos{rv.pos}, nullptr, form)
+                  : pairs_fp32c_one<BS, CHUNK, false>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
+                                                      GlobalPos{rv.pos}, nullptr, 0);
     emit_pairs<FUSE, RIGID>(c, u, psum, psum_T, N, i, o);
 }
 
@@ -806,33 +877,25 @@ __global__ void __launch_bounds__(BS) k_pairs_fp32c(DevConsts c, const double *_
 // last particles, read by every lane from memory, so no lane depends on another lane's registers.
 #define SPHFEM_STAGE_ROW_SCAN 64
 template <int CHUNK, int CAP, bool FUSE = false, bool RIGID = false>
-__global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const double *__restrict__ blanked,
-                                                           const int *__restrict__ hash, int N, RecView rv,
+__global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const int *__restrict__ hash, int N, RecView rv,
                                                            const int *__restrict__ cs, const int *__restrict__ ce,
                                                            float4 *__restrict__ psum, float *__restrict__ psum_T,
                                                            const int *__restrict__ nonfinite, int *__restrict__ flags,
                                                            UpdateArgs u) {
     // LDS: staged -- positions [CAP + 4] (+4: the scan reads up to three records past a range) and
     // 16-bit list entries; list path -- 32-bit list entries in the same bytes
-    constexpr int POS_BYTES = (CAP + 4) * 16, LIST16 = CHUNK * 64 * 2, LIST32 = CHUNK * 64 * 4;
+    constexpr int POS_BYTES = (CAP + 4) * 8, LIST16 = CHUNK * 64 * 2, LIST32 = CHUNK * 64 * 4;
     constexpr int LDS_BYTES = POS_BYTES + LIST16 > LIST32 ? POS_BYTES + LIST16 : LIST32;
     __shared__ __align__(16) unsigned char lds[LDS_BYTES];
     __shared__ int sdelta[8];
-    float4 *spos = reinterpret_cast<float4 *>(lds);
+    int2 *spos = reinterpret_cast<int2 *>(lds);
     unsigned short *list16 = reinterpret_cast<unsigned short *>(lds + POS_BYTES);
     int *list32 = reinterpret_cast<int *>(lds);
-    const int win = *nonfinite;
+    const int form = pairs_form(c, nonfinite);
     const int base = xcd_logical_block() * 64;
     if (base >= N) return;                              // the whole wavefront
     const int lane = (int)threadIdx.x;
     const int i = base + lane;
-    if (win != 0) {                                     // the window form, as k_pairs_fp32c
-        if (i < N)
-            emit_pairs<FUSE, RIGID>(c, u, psum, psum_T, N, i,
-                                    pairs_fp32c_one<64, CHUNK, true>(c, blanked, hash, N, rv, cs, ce, i,
-                                                                     list32 + lane, GlobalPos{rv.r0}, nullptr));
-        return;
-    }
     const int last_i = base + 63 < N ? base + 63 : N - 1;
     const int nx = c.geom.nx, ny = c.geom.ny;
     const int h0 = hash[base], h1 = hash[last_i];
@@ -840,7 +903,7 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const do
     StagedPos sp;
     sp.spos = spos;
     sp.sdelta = sdelta;
-    bool staged = h0 >= 0 && h1 >= h0 && h1 / ny == col0 && col0 < nx;
+    bool staged = form == 0 && h0 >= 0 && h1 >= h0 && h1 / ny == col0 && col0 < nx;
     int total = 0;
     if (staged) {
         const int r_lo = h0 - col0 * ny - 2 < 0 ? 0 : h0 - col0 * ny - 2;
@@ -890,20 +953,22 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const do
         for (int d = 0; d < 5; d++) {
             if (lane == d) sdelta[d] = sp.delta[d];
             const int n = sp.L[d] - sp.F[d], off = sp.F[d] - sp.delta[d];
-            for (int k = lane; k < n; k += 64) spos[off + k] = rv.r0[sp.F[d] + k];
+            for (int k = lane; k < n; k += 64) spos[off + k] = rv.pos[sp.F[d] + k];
         }
         __syncthreads();
-        if (i < N)
-            emit_pairs<FUSE, RIGID>(c, u, psum, psum_T, N, i,
-                                    pairs_fp32c_one<64, CHUNK, false, StagedPos>(c, blanked, hash, N, rv, cs, ce, i,
-                                                                                 list16 + lane, sp, flags));
-    } else if (i < N) {
-        emit_pairs<FUSE, RIGID>(c, u, psum, psum_T, N, i,
-                                pairs_fp32c_one<64, CHUNK, false>(c, blanked, hash, N, rv, cs, ce, i, list32 + lane,
-                                                                  GlobalPos{rv.r0}, nullptr));
     }
+    if (i >= N) return;
+    PairOut o;
+    if (staged)
+        o = pairs_fp32c_one<64, CHUNK, false, StagedPos>(c, hash, N, rv, cs, ce, i, list16 + lane, sp, flags, 0);
+    else if (form == 0)
+        o = pairs_fp32c_one<64, CHUNK, false>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
+                                              nullptr, 0);
+    else
+        o = pairs_fp32c_one<64, CHUNK, true>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
+                                             nullptr, form);
+    emit_pairs<FUSE, RIGID>(c, u, psum, psum_T, N, i, o);
 }
-
 
 // interactions_gpu.cu:143-379 for the drop-in entry point, first kernel: the neighbour factors of
 // k_pairs_fp64's pair loop from the arrays as they stand (the same operations the reference repeats
@@ -1167,7 +1232,7 @@ __global__ void __launch_bounds__(BS) k_pairs_fp64(DevConsts c, sphfem_particles
     if (i >= N || B.blanked[i] == 1.) return;
     const double thermal_alpha = interaction_alpha(c, B.tool_particle[i]);
     // the window form when a live particle carries a non-finite input (see pair_sums_fp64)
-    if (*nonfinite != 0)
+    if ((*nonfinite & SPHFEM_FORM_WINDOW) != 0)
         psum64[i] = pair_sums_fp64<BS, CHUNK, true>(c, B, i, thermal_alpha, cs, ce, pre_vol, pre_s,
                                                           nb_list + threadIdx.x);
     else
@@ -1220,18 +1285,18 @@ template <int BSZ, int CH, bool FUSE, bool RIGID>
 static void launch_pairs_fp32c(sphfem_ctx *ctx, const sphfem_particles &B, sphfem_leap_frog *lf, const int *cs,
                                const int *ce, const UpdateArgs &u) {
     const size_t n = B.N;
-    RecView rv{lf->rec, lf->rec + n + 4, lf->rec + 2 * n + 4, lf->rec + 3 * n + 4};
+    const RecView rv = rec_view(lf->rec, n);
     k_pairs_fp32c<BSZ, CH, FUSE, RIGID><<<nblk(B.N, BSZ), BSZ, 0, ctx->stream>>>(
-        ctx->c, B.blanked, B.hash, (int)B.N, rv, cs, ce, lf->psum, lf->psum_T, ctx->d_flags + SPHFEM_FLAG_NONFINITE, u);
+        ctx->c, B.hash, (int)B.N, rv, cs, ce, lf->psum, lf->psum_T, ctx->d_flags + SPHFEM_FLAG_NONFINITE, u);
 }
 
 template <int CH, bool FUSE, bool RIGID>
 static void launch_pairs_fp32c_staged(sphfem_ctx *ctx, const sphfem_particles &B, sphfem_leap_frog *lf, const int *cs,
                                       const int *ce, const UpdateArgs &u) {
     const size_t n = B.N;
-    RecView rv{lf->rec, lf->rec + n + 4, lf->rec + 2 * n + 4, lf->rec + 3 * n + 4};
+    const RecView rv = rec_view(lf->rec, n);
     k_pairs_fp32c_staged<CH, SPHFEM_STAGE_CAP, FUSE, RIGID><<<nblk(B.N, 64), 64, 0, ctx->stream>>>(
-        ctx->c, B.blanked, B.hash, (int)B.N, rv, cs, ce, lf->psum, lf->psum_T, ctx->d_flags + SPHFEM_FLAG_NONFINITE,
+        ctx->c, B.hash, (int)B.N, rv, cs, ce, lf->psum, lf->psum_T, ctx->d_flags + SPHFEM_FLAG_NONFINITE,
         ctx->d_flags, u);
 }
 
@@ -1268,7 +1333,7 @@ static void launch_pairs_fp32c_tuned(sphfem_ctx *ctx, const sphfem_particles &B,
 
 void launch_interactions_fp32c(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_leap_frog *lf, const int *cs,
                                const int *ce, int num_cell) {
-    launch_records_state(ctx, p, num_cell, lf->rec);
+    launch_records_state(ctx, p, num_cell, rec_view(lf->rec, p.N));
     launch_pairs_fp32c_tuned(ctx, p, lf, cs, ce);
     KTimer t(ctx, "psum_expand");
     k_psum_expand<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, lf->psum, lf->psum_T,

@@ -1026,26 +1026,53 @@ __device__ __forceinline__ void flag_nonfinite(int *__restrict__ flags, double b
         atomicOr(&flags[SPHFEM_FLAG_NONFINITE], 1);
 }
 
-// FP32C neighbour records of one sorted particle: positions relative to the cell corner keep ~1e-7
-// of the cell size; the stress terms are the per-particle factors of the pair sum, (S - p)/rho^2 and
-// S_xy/rho^2; the temperature is stored as T - T_init, so that the FP32 differences T_i - T_j of a
-// nearly uniform field keep ~1e-7 of the deviation instead of ~1e-7 of T; four SoA blocks; the
-// first has 4 padding records that absorb four-wide scan loads
-__device__ __forceinline__ void write_records(const DevConsts &c, float4 *__restrict__ rec, int N, int i, int h,
-                                             sphfem_double2 pos, sphfem_double2 vel, sphfem_double4 S, double rho,
-                                             double T, double blanked, double tool, double hh, double pr,
-                                             sphfem_double4 R) {
+// FP32C neighbour records (RecView) of one sorted particle.  The position is rounded to cell / 2^28 from
+// FP64 and wrapped (finer than FP32 relative to the cell corner); the stress terms are the per-particle
+// factors of the pair sum, (S - p)/rho^2 and S_xy/rho^2; the temperature is stored as T - T_init, so
+// that the FP32 differences T_i - T_j of a nearly uniform field keep ~1e-7 of the deviation instead of
+// ~1e-7 of T.
+__device__ __forceinline__ void write_records(const DevConsts &c, const RecView &rec, double inv_dx, int *__restrict__ flags, int i, int h,
+                                             sphfem_double2 pos, sphfem_double2 vel, sphfem_double4 S, double rho, double T, double blanked,
+                                             double tool, double hh, double pr, sphfem_double4 R) {
     const int ny = c.geom.ny;
     const int ix = h / ny, iy = h - ix * ny;
-    const double ox = c.geom.bbmin_x + ix * c.geom.dx;
-    const double oy = c.geom.bbmin_y + iy * c.geom.dx;
-    const double rho21 = 1. / (rho * rho);
-    const float vol = (float)(c.phys.mass / rho);
-    float4 r0, r1, r2, r3;
-    r0.x = blanked == 1. ? 1e30f : (float)(pos.x - ox);     // blanked: never inside a support
-    r0.y = (float)(pos.y - oy);
-    r0.z = (float)iy;
-    r0.w = (float)hh;
+    // cell units from the centre of the particle's cell.  Blanked particles are put 8 cells from it along
+    // both axes, where no kernel reaches them from the 5x5 cells.  Above or below the grid a key names a
+    // cell of the next or the previous column: those particles see only each other, and keep their place
+    // relative to that cell, 8 cells aside in x or in y.  One that lies near neither is put with the blanked
+    // ones, and the general form reads its position elsewhere.
+    double cx = (pos.x - c.geom.bbmin_x) * inv_dx - (ix + 0.5);
+    double cy = (pos.y - c.geom.bbmin_y) * inv_dx - (iy + 0.5);
+    const bool live = blanked != 1.;
+    bool near = fabs(cx) <= 1.6 && fabs(cy) <= 1.6;
+    int turn = 0;
+    const double unit = (double)(1 << SPHFEM_POS_BITS);
+    if (live && !near) {
+        rec.away[i] = make_double2((cx + (ix + 0.5)) * unit, (cy + (iy + 0.5)) * unit);
+        turn = cy > 0. ? 1 : -1;
+        cx += turn;
+        cy -= turn * (double)ny;
+        near = fabs(cx) <= 1.6 && fabs(cy) <= 1.6 && ny >= 10;
+    }
+    const int half = 1 << (SPHFEM_POS_BITS - 1);
+    const bool put = live && near;
+    unsigned ux = ((unsigned)ix << SPHFEM_POS_BITS) + half, uy = ((unsigned)iy << SPHFEM_POS_BITS) + half;
+    if (!put || turn > 0) ux ^= 1u << 31;
+    if (!put || turn < 0) uy ^= 1u << 31;
+    if (put) {
+        ux += (unsigned)(int)rint(cx * unit);
+        uy += (unsigned)(int)rint(cy * unit);
+    }
+    const int2 r0 = make_int2((int)ux, (int)uy);
+    // the form of the pair sums: one flag write per wavefront, and none for bits that are seen set
+    const int form = (__any(live && !near) ? SPHFEM_FORM_AWAY : 0) |
+                     (__any(live && hh != c.geom.dx) ? SPHFEM_FORM_WIDTH : 0);
+    if (form != 0 && (int)__lane_id() == __ffsll((long long)__ballot(1)) - 1 &&
+        (form & ~flags[SPHFEM_FLAG_NONFINITE]) != 0)
+        atomicOr(&flags[SPHFEM_FLAG_NONFINITE], form);
+    const double inv_rho = 1. / rho, rho21 = inv_rho * inv_rho;
+    const float vol = (float)(c.phys.mass * inv_rho);
+    float4 r1, r2, r3;
     r1.x = (float)vel.x;
     r1.y = (float)vel.y;
     r1.z = tool == 0. ? (float)((S.x - pr) * rho21) : 0.f;
@@ -1056,20 +1083,21 @@ __device__ __forceinline__ void write_records(const DevConsts &c, float4 *__rest
     r2.w = (float)R.z;
     r3.x = tool == 1. ? -vol : vol;
     r3.y = (float)rho;
-    r3.z = (float)sqrtf_d(c.phys.K / rho);
+    r3.z = live ? (float)sqrtf_d(c.phys.K * inv_rho) : -1.f;
     r3.w = (float)(T - c.trml_wp.T_init);    // only differences enter the sums: offset from T_init
-    const size_t n4 = (size_t)N + 4;
-    rec[i] = r0;
-    rec[n4 + i] = r1;
-    rec[n4 + (size_t)N + i] = r2;
-    rec[n4 + 2 * (size_t)N + i] = r3;
+    rec.pos[i] = r0;
+    rec.r1[i] = r1;
+    rec.r2[i] = r2;
+    rec.r3[i] = r3;
+    rec.h[i] = (float)hh;
 }
 
 // FP32C records of an already sorted state as it stands (no predictor): the inputs of
 // interactions_monaghan, with p and R as material_eos and corrector_artificial_stress left them
 // (interactions_gpu.cu:143-379 reads them from the particle arrays)
 __global__ void __launch_bounds__(256) k_records_state(DevConsts c, const sphfem_particles p, int num_cell,
-                                                       int *__restrict__ flags, float4 *__restrict__ rec) {
+                                                       int *__restrict__ flags, const RecView rec,
+                                                       double inv_dx) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
     if (i >= N) return;
@@ -1085,12 +1113,13 @@ __global__ void __launch_bounds__(256) k_records_state(DevConsts c, const sphfem
     const sphfem_double4 S = p.S[i];
     const double rho = p.rho[i], T = p.T[i], blanked = p.blanked[i], hh = p.h[i];
     flag_nonfinite(flags, blanked, pos, vel, S, rho, T, hh, pr, R);
-    write_records(c, rec, N, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
+    write_records(c, rec, inv_dx, flags, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
 }
 
-void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, float4 *rec) {
+void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, const RecView &rec) {
     KTimer t(ctx, "records_state");
-    k_records_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, num_cell, ctx->d_flags, rec);
+    k_records_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, num_cell, ctx->d_flags, rec,
+                                                             1. / ctx->c.geom.dx);
 }
 
 // source and key of sorted position i (from the re-sort's lists, or the sorted arrays when there are
@@ -1204,7 +1233,7 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
 __global__ void __launch_bounds__(256) k_reorder_records(DevConsts c, const sphfem_particles p,
                                                          int *__restrict__ cell_start, int *__restrict__ cell_end,
                                                          int num_cell, int *__restrict__ flags,
-                                                         float4 *__restrict__ rec, const RateView rates,
+                                                         const RecView rec, double inv_dx, const RateView rates,
                                                          ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
@@ -1239,7 +1268,7 @@ __global__ void __launch_bounds__(256) k_reorder_records(DevConsts c, const sphf
     }
     const double hh = ld_stream(&p.h[s]);
     flag_nonfinite(flags, blanked, pos, vel, tool == 0. ? S : sphfem_double4{0., 0., 0., 0.}, rho, T, hh, pr, R);
-    write_records(c, rec, N, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
+    write_records(c, rec, inv_dx, flags, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
 }
 
 void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, sphfem_leap_frog *lf,
@@ -1249,7 +1278,8 @@ void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_partic
     if (lf->precision == SPHFEM_FP32C) {
         KTimer t(ctx, "reorder_records");
         k_reorder_records<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, g->cell_start, g->cell_end,
-                                                                   g->num_cell, ctx->d_flags, lf->rec, *rates, rs);
+                                                                   g->num_cell, ctx->d_flags, rec_view(lf->rec, p.N),
+                                                                   1. / ctx->c.geom.dx, *rates, rs);
         return;
     }
     KTimer t(ctx, "reorder_predict");
