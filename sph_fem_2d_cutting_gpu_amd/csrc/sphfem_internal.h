@@ -111,10 +111,10 @@ inline RateView rate_view(float *base, size_t n) {
 //   pos[j] = position in units of cell / 2^SPHFEM_POS_BITS from the grid's corner, modulo 2^32 (padded by
 //            4 records); 8 cells aside for blanked particles and outside the grid's rows (write_records)
 //   r1[j] = {vx, vy, (Sxx - p)/rho^2, Sxy/rho^2}     r2[j] = {(Syy - p)/rho^2, Rxx, Rxy, Ryy}
-//   r3[j] = {+-mass/rho, rho, sqrt(K/rho), T - T_init}
+//   r3[j] = {+-mass/rho, rho, alpha sqrt(K/rho), T - T_init}
 //   h[j]    = kernel width (read where it is not the cell size)
 //   away[j] = position in the units of pos, unwrapped (written for live particles whose pos lies aside)
-// The volume is stored negative for tool particles, the sound speed of blanked ones is -1.
+// The volume is stored negative for tool particles, the sound speed of blanked ones is -inf.
 #define SPHFEM_POS_BITS 28
 struct RecView {
     float4 *r1, *r2, *r3;

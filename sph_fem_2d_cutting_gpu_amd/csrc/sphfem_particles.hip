@@ -229,15 +229,14 @@ struct StagedPos {
     }
 };
 
-// Particle i and the per-i kernel constants.  Distances D = x_i - x_j are in units u = cell / 2^28; the
-// kernel is evaluated in the dimensionless q = |D| ku, ku = u / h_i, and its dimensional factors multiply
-// the finished sums.
+// Particle i and the per-i kernel constants.  Distances D = x_i - x_j are in units u = cell / 2^28, with
+// ku = u / h_i; the kernel's factors multiply the finished sums.
 struct PairI {
     int xi, yi;
     float vxi, vyi, sxi, syi, szi, Rxi, Ryi, Rzi, rhoi, ci, Ti;
-    float kf;                   // W (kernel / its value factor) to the artificial stress's w / wdeltap
+    float kf;                   // W to the artificial stress's w / wdeltap
     float D2max, D2min;         // the support test on |D|^2
-    float beta2, alpha, eta2;   // 2 beta, alpha, eta^2 of the viscosity
+    float beta2, eta2;          // 2 beta and eta^2 of the viscosity
     bool thermal;
     bool mech;                  // i is not a tool particle
     // general form only
@@ -261,13 +260,13 @@ __device__ __forceinline__ void pair_term(const PairI &I, float dx, float dy, co
     const float D2 = dx * dx + dy * dy;
     const float rinv = __builtin_amdgcn_rsqf(D2);
     const float ku = GEN ? I.ku : KU;
-    const float q = D2 * rinv * ku;
-    const float u = 1.f - 0.5f * q;
+    const float r = D2 * rinv;
+    const float u = 1.f - (0.5f * ku) * r;
     const float s = u * u;
-    // value w (over fac) and radial factor g: gradient = fac / h_i * g * D
-    const bool outer = q > 1.f;
-    float w = outer ? 16.f * (s * s) * s : 1.f - 1.5f * (q * q) * u;
-    float g = outer ? (-3.f * s) * rinv : (2.25f * ku) * q - 3.f * ku;
+    // W = kernel / (16 fac) and g: gradient = -3 fac / h_i * g * D
+    const bool outer = r > (GEN ? I.H : 1.f / KU);
+    float w = outer ? s * s * s : 0.0625f - (0.09375f * ku * ku) * D2 * u;
+    float g = outer ? s * rinv : ku - (0.75f * ku * ku) * r;
     if constexpr (GEN) {
         if (win && !(D2 < I.D2max && D2 >= I.D2min)) {
             w = 0.f;
@@ -301,21 +300,21 @@ __device__ __forceinline__ void pair_term(const PairI &I, float dx, float dy, co
             if (vp < 0.f) {
                 const float H = 0.5f * (I.H + Hj);
                 const float mu = H * vp * __builtin_amdgcn_rcpf(D2 + I.eta2 * H * H);
-                const float piij = mu * (I.beta2 * mu - I.alpha * (I.ci + q3.z)) * half_inv_rhoij;
+                const float piij = mu * (I.beta2 * mu - (I.ci + q3.z)) * half_inv_rhoij;
                 Ax -= piij;
                 Az -= piij;
             }
         } else {
             // receding pairs take mu = 0 and with it no viscous term
             const float mu = fminf(vp, 0.f) * __builtin_amdgcn_rcpf(D2 * KU + I.eta2);
-            const float piij = mu * (I.beta2 * mu - I.alpha * (I.ci + q3.z)) * half_inv_rhoij;
+            const float piij = mu * (I.beta2 * mu - (I.ci + q3.z)) * half_inv_rhoij;
             Ax -= piij;
             Az -= piij;
         }
-        a.ax += Ax * wx + Ay * wy;
-        a.ay += Ay * wx + Az * wy;
+        a.ax = Ay * wy + (Ax * wx + a.ax);
+        a.ay = Az * wy + (Ay * wx + a.ay);
         const float wr = w * half_inv_rhoij;
-        a.p0 -= wr * dvx;                                // sum w / (rho_i + rho_j) * (v_i - v_j)
+        a.p0 -= wr * dvx;                                // sum W / (rho_i + rho_j) * (v_i - v_j)
         a.p1 -= wr * dvy;
     }
 }
@@ -350,11 +349,15 @@ __device__ __forceinline__ double2 wide_pos(const RecView &rv, int ny, int j, in
 //    rounding on output.
 // Outputs (FP32): psum[i] = velocity gradient (xx, xy, yx, yy); psum[N + i] = (mass * stress
 // divergence - mass * viscous term) per axis, XSPH velocity per axis; psum_T[i] = Laplacian of T.
-// Bound by the L1's rate of cache lines per gather (a wavefront's 64 lists drift apart: some 36 lines
-// per 16-byte record, 20 per 8-byte position) and close behind by VALU issue.  Positions of 16 bytes
+// Bound by VALU issue (70 - 80 % busy; 64 instructions a pair, 12 a candidate) and close behind by the
+// L1's rate of cache lines per gather (a wavefront's 64 lists drift apart: some 30 lines per load).
+// ROLL: the columns in a loop, which leaves the kernel with 128 registers and four wavefronts per SIMD
+// where no update follows the sums (16 M particles: 3000 -> 2827 us); with the update's 166 registers there
+// are three either way, and the unrolled columns are the faster (4 M: 779 us against 796).  Copying all
+// records of 256-particle tiles to LDS cut the L1's accesses by five and cost as much in other issue.  Positions of 16 bytes
 // (cell-relative FP32 and the cell row, with the column in the list entry) and kernel factors applied
-// per pair took 868 us (with the update) on 4 M particles and 3337 us (sums alone) on 16 M, against 797
-// and 3010 us.
+// per pair took 868 us (with the update) on 4 M particles and 3337 us (sums alone) on 16 M, against 779
+// and 2827 us.
 // General form (form != 0; the SPHFEM_FORM_ bits): kernel widths other than the cell size; positions that
 // the wrapped ones cannot tell apart, taken in FP64; and the window form, where every non-blanked record
 // of the 5x5 cells is evaluated with the kernel set to 0 outside the support, as the reference does (see
@@ -654,7 +657,7 @@ struct PairOut {           // one particle's FP32C sums: psum[i], psum[N + i], p
     float T;
 };
 
-template <int BS, int CHUNK, bool GEN, class Pos = GlobalPos>
+template <int BS, int CHUNK, bool GEN, bool ROLL, class Pos = GlobalPos>
 __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int *__restrict__ hash, int N,
                                                    const RecView &rv,
                                                    const int *__restrict__ cs, const int *__restrict__ ce, int i,
@@ -672,25 +675,25 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
     const double alpha_i = tool_i ? c.trml_itool.alpha : c.trml_wp.alpha;
     const double dxc = c.geom.dx;
     const double hi = GEN ? (double)rv.h[i] : dxc;
-    if (a3.z != -1.f && (!tool_i || alpha_i != 0.)) {
+    if (a3.z != -INFINITY && (!tool_i || alpha_i != 0.)) {
         const int nx = c.geom.nx, ny = c.geom.ny;
         const int hashi = hash[i];
         const int gi = hashi / ny;
         const int gj = hashi - gi * ny;
         const int low_j = gj - 2 < 0 ? 0 : gj - 2;
         const int high_j = gj + 3 > ny ? ny : gj + 3;
-        // cell-table entries of the five columns, issued together: the lowest and highest row of
-        // each column's window decide its sorted range unless those cells are empty
-        int cs_lo[5], cs_hi[5], ce_hi[5];
-#pragma unroll
-        for (int d = 0; d < 5; d++) {
-            const int col = gi - 2 + d;
+        // cell-table entries of a column's window: its lowest and highest row decide the sorted range
+        // unless those cells are empty.  A column's are loaded while the one before it is scanned.
+        auto cells = [&](int col, int &lo_s, int &hi_s, int &hi_e) {
             const bool ok = col >= 0 && col < nx;
             const int c0 = (ok ? col : gi) * ny;
-            cs_lo[d] = ok ? cs[c0 + low_j] : -1;
-            cs_hi[d] = ok ? cs[c0 + high_j - 1] : -1;
-            ce_hi[d] = ok ? ce[c0 + high_j - 1] : -1;
-        }
+            lo_s = cs[c0 + low_j];
+            hi_s = cs[c0 + high_j - 1];
+            hi_e = ce[c0 + high_j - 1];
+            if (!ok) lo_s = hi_s = -1;
+        };
+        int lo_s, hi_s, hi_e;
+        cells(gi - 2, lo_s, hi_s, hi_e);
         const int2 a0 = rv.pos[i];
         const float4 a1 = rv.r1[i], a2 = rv.r2[i];
         PairI I;
@@ -700,11 +703,10 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
         I.rhoi = a3.y; I.ci = a3.z; I.Ti = a3.w;
         I.thermal = alpha_i != 0.;
         I.mech = !tool_i;
-        I.kf = (float)(SPHFEM_PI_FAC / (hi * hi * c.corr.wdeltap));
+        I.kf = (float)(16. * SPHFEM_PI_FAC / (hi * hi * c.corr.wdeltap));
         const double inv_u = (double)(1 << SPHFEM_POS_BITS) / dxc;
         I.D2min = (float)(c.rr2_min * inv_u * inv_u);
         I.beta2 = (float)(2. * c.corr.beta);
-        I.alpha = (float)c.corr.alpha;
         if constexpr (GEN) {
             I.H = (float)(hi * inv_u);
             I.ku = 1.f / I.H;
@@ -743,25 +745,28 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
             if constexpr (GEN) Hj = (float)((double)rv.h[pos.index(e)] * inv_u);
             pair_term<GEN>(I, dx, dy, q1, q2, q3, Hj, win, acc);
         };
-        // dense list: two entries per iteration, the records of the next entry loaded before the
-        // current one is evaluated (ping-pong registers, no copies); each list entry is read from LDS
-        // one pair term before its records are loaded, so the LDS latency passes under that term
-        auto run_list = [&](int n) {
-            if (n <= 0) return;
+        // dense list of the entries in front of list[end]: two per iteration, the records of the next
+        // entry loaded before the current one is evaluated (ping-pong registers, no copies); each list
+        // entry is read from LDS one pair term before its records are loaded, so the LDS latency passes
+        // under that term.  The two entries past the end, which are loaded and not evaluated, are i itself.
+        auto run_list = [&](int end) {
+            if (end <= 0) return;
             PairAcc acc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+            list[end] = pos.encode(2, i);
+            list[end + BS] = pos.encode(2, i);
             typename Pos::Entry eA = list[0];
-            typename Pos::Entry eB = list[(1 < n ? 1 : n - 1) * BS];
+            typename Pos::Entry eB = list[BS];
             unsigned oA = pos.index(eA) << 4;
             int2 A0 = pos.entry(eA);
             float4 A1 = ldrec(rv.r1, oA), A2 = ldrec(rv.r2, oA), A3 = ldrec(rv.r3, oA);
-            for (int k = 0; k < n; k += 2) {
-                const typename Pos::Entry eA_next = list[(k + 2 < n ? k + 2 : n - 1) * BS];
+            for (int k = 0; k < end; k += 2 * BS) {
+                const typename Pos::Entry eA_next = list[k + 2 * BS];
                 const unsigned oB = pos.index(eB) << 4;
                 const int2 B0 = pos.entry(eB);
                 const float4 B1 = ldrec(rv.r1, oB), B2 = ldrec(rv.r2, oB), B3 = ldrec(rv.r3, oB);
                 term(eA, A0, A1, A2, A3, acc);
-                if (k + 1 < n) {
-                    const typename Pos::Entry eB_next = list[(k + 3 < n ? k + 3 : n - 1) * BS];
+                if (k + BS < end) {
+                    const typename Pos::Entry eB_next = list[k + 3 * BS];
                     eA = eA_next;
                     oA = pos.index(eA) << 4;
                     A0 = pos.entry(eA);
@@ -769,21 +774,21 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
                     term(eB, B0, B1, B2, B3, acc);
                     eB = eB_next;
                 }
-                if (((k + 2) & 7) == 0) flush(acc);
+                if (((k + 2 * BS) & (8 * BS - 1)) == 0) flush(acc);
             }
             flush(acc);
         };
 
-        int n = 0;
-#pragma unroll
+        int end = 0;               // BS times the number of entries
+#pragma unroll (ROLL ? 1 : 5)
         for (int d = 0; d < 5; d++) {
             const int col = gi - 2 + d;
+            int first = lo_s, last = hi_s != -1 ? hi_e : -1;
+            if (d < 4) cells(col + 1, lo_s, hi_s, hi_e);
             if (col < 0 || col >= nx) continue;
             const int c0 = col * ny;
-            int first = cs_lo[d];
             for (int jr = low_j + 1; first == -1 && jr < high_j; jr++) first = cs[c0 + jr];
             if (first == -1) continue;                                   // empty window
-            int last = cs_hi[d] != -1 ? ce_hi[d] : -1;
             for (int jr = high_j - 2; last == -1 && jr >= low_j; jr--)
                 if (cs[c0 + jr] != -1) last = ce[c0 + jr];
             if (last > N || first < 0) continue;                        // inconsistent cell table
@@ -794,30 +799,30 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
                 pos.scan4(d, j, b);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    if (GEN && (j + u >= last || rv.r3[j + u].z == -1.f)) continue;
+                    if (GEN && (j + u >= last || rv.r3[j + u].z == -INFINITY)) continue;
                     float dx, dy;
                     distance((unsigned)(j + u), b[u], dx, dy);
                     const float D2 = dx * dx + dy * dy;
                     if (j + u < last && (win || (D2 < I.D2max && D2 >= I.D2min))) {
-                        list[n * BS] = pos.encode(d, j + u);
-                        n++;
+                        list[end] = pos.encode(d, j + u);
+                        end += BS;
                     }
                 }
                 // dense region: every active lane empties its list at once (a lane emptying its
                 // list alone runs it with the rest of the wavefront idle)
-                if (__any(n > CHUNK - 4)) {
-                    run_list(n);
-                    n = 0;
+                if (__any(end > (CHUNK - 4) * BS)) {
+                    run_list(end);
+                    end = 0;
                 }
             }
         }
-        run_list(n);
+        run_list(end);
     }
-    // the kernel's factors fac / h (gradient), fac (value), and fac / h^2 (radial over distance: the sums
-    // hold its g in units of u / h)
+    // the factors of the kernel gradient, -3 fac / h, and of its value, 16 fac; the heat term holds the
+    // gradient over the distance, in units of u
     const double mass = c.phys.mass;
-    const double h1 = 1. / hi, fac = SPHFEM_PI_FAC * h1 * h1, grad = fac * h1;
-    const double ma = mass * grad, xs = -2. * c.corr.xspheps * mass * fac;
+    const double h1 = 1. / hi, fac = SPHFEM_PI_FAC * h1 * h1, grad = -3. * fac * h1;
+    const double ma = mass * grad, xs = -32. * c.corr.xspheps * mass * fac;
     const double heat = 2. * grad * (double)(1 << SPHFEM_POS_BITS) / dxc;
     PairOut o;
     o.g = make_float4((float)(grad * d_v0), (float)(grad * d_v1), (float)(grad * d_v2), (float)(grad * d_v3));
@@ -852,14 +857,14 @@ __global__ void __launch_bounds__(BS) k_pairs_fp32c(DevConsts c, const int *__re
                                                          const int *__restrict__ cs, const int *__restrict__ ce,
                                                          float4 *__restrict__ psum, float *__restrict__ psum_T,
                                                          const int *__restrict__ nonfinite, UpdateArgs u) {
-    __shared__ int nb_list[CHUNK * BS];
+    __shared__ int nb_list[(CHUNK + 2) * BS];
     const int form = pairs_form(c, nonfinite);
     const int i = xcd_logical_block() * BS + threadIdx.x;
     if (i >= N) return;
     const PairOut o =
-        form != 0 ? pairs_fp32c_one<BS, CHUNK, true>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
+        form != 0 ? pairs_fp32c_one<BS, CHUNK, true, true>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
                                                      GlobalPos{rv.pos}, nullptr, form)
-                  : pairs_fp32c_one<BS, CHUNK, false>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
+                  : pairs_fp32c_one<BS, CHUNK, false, !FUSE>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
                                                       GlobalPos{rv.pos}, nullptr, 0);
     emit_pairs<FUSE, RIGID>(c, u, psum, psum_T, N, i, o);
 }
@@ -884,7 +889,7 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
                                                            UpdateArgs u) {
     // LDS: staged -- positions [CAP + 4] (+4: the scan reads up to three records past a range) and
     // 16-bit list entries; list path -- 32-bit list entries in the same bytes
-    constexpr int POS_BYTES = (CAP + 4) * 8, LIST16 = CHUNK * 64 * 2, LIST32 = CHUNK * 64 * 4;
+    constexpr int POS_BYTES = (CAP + 4) * 8, LIST16 = (CHUNK + 2) * 64 * 2, LIST32 = (CHUNK + 2) * 64 * 4;
     constexpr int LDS_BYTES = POS_BYTES + LIST16 > LIST32 ? POS_BYTES + LIST16 : LIST32;
     __shared__ __align__(16) unsigned char lds[LDS_BYTES];
     __shared__ int sdelta[8];
@@ -960,12 +965,12 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
     if (i >= N) return;
     PairOut o;
     if (staged)
-        o = pairs_fp32c_one<64, CHUNK, false, StagedPos>(c, hash, N, rv, cs, ce, i, list16 + lane, sp, flags, 0);
+        o = pairs_fp32c_one<64, CHUNK, false, false, StagedPos>(c, hash, N, rv, cs, ce, i, list16 + lane, sp, flags, 0);
     else if (form == 0)
-        o = pairs_fp32c_one<64, CHUNK, false>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
+        o = pairs_fp32c_one<64, CHUNK, false, !FUSE>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
                                               nullptr, 0);
     else
-        o = pairs_fp32c_one<64, CHUNK, true>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
+        o = pairs_fp32c_one<64, CHUNK, true, true>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
                                              nullptr, form);
     emit_pairs<FUSE, RIGID>(c, u, psum, psum_T, N, i, o);
 }

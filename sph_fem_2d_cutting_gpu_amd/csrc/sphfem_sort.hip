@@ -1083,7 +1083,7 @@ __device__ __forceinline__ void write_records(const DevConsts &c, const RecView 
     r2.w = (float)R.z;
     r3.x = tool == 1. ? -vol : vol;
     r3.y = (float)rho;
-    r3.z = live ? (float)sqrtf_d(c.phys.K * inv_rho) : -1.f;
+    r3.z = live ? (float)(c.corr.alpha * sqrtf_d(c.phys.K * inv_rho)) : -INFINITY;
     r3.w = (float)(T - c.trml_wp.T_init);    // only differences enter the sums: offset from T_init
     rec.pos[i] = r0;
     rec.r1[i] = r1;
