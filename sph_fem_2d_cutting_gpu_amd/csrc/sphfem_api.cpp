@@ -249,8 +249,7 @@ int sphfem_destroy(sphfem_ctx *ctx) {
     (void)hipStreamSynchronize(ctx->stream);
     timing_collect(ctx);
     dfree(ctx->d_flags);
-    dfree(ctx->pre_vol);
-    dfree(ctx->pre_s);
+    dfree(ctx->pre);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
     return SPHFEM_OK;
@@ -638,13 +637,11 @@ int sphfem_interactions_monaghan(sphfem_ctx *ctx, sphfem_particles *p, const int
     if (!ctx || !p || !cell_start || !cell_end || num_cell != ctx->c.geom.nx * ctx->c.geom.ny) return SPHFEM_ERR_ARG;
     return guarded(ctx, [&] {
         if (int rc = need(ctx, SET_PHYS | SET_CORR)) return rc;
-        if (p->N > ctx->pre_cap) {      // the factors' workspace grows to the largest particle count
+        if (p->N > ctx->pre_cap) {      // the neighbour fields' workspace grows to the largest particle count
             SPHFEM_HIP_CHECK(hipStreamSynchronize(ctx->stream));
             ctx->pre_cap = 0;
-            dfree(ctx->pre_vol);
-            dfree(ctx->pre_s);
-            ctx->pre_vol = dalloc<double>(p->N);
-            ctx->pre_s = dalloc<sphfem_double4>(p->N);
+            dfree(ctx->pre);
+            ctx->pre = dalloc<sphfem_double2>(sphfem::pre_double2s(p->N));
             ctx->pre_cap = p->N;
         }
         launch_interactions_ref(ctx, *p, cell_start, cell_end);
@@ -1622,8 +1619,7 @@ int sphfem_leap_frog_create(sphfem_ctx *ctx, unsigned int num_part, unsigned int
         lf->S_init = dalloc<sphfem_double4>(num_part);
         lf->rho_init = dalloc<double>(num_part);
         lf->T_init = dalloc<double>(num_part);
-        lf->pre_vol = dalloc<double>(num_part);
-        lf->pre_s = dalloc<sphfem_double4>(num_part);
+        lf->pre = dalloc<sphfem_double2>(sphfem::pre_double2s(num_part));
         lf->psum64 = dalloc<sphfem::PairSums>(num_part);
         lf->cell_start = dalloc<int>(std::max(num_cell, 1u));
         lf->cell_end = dalloc<int>(std::max(num_cell, 1u));
@@ -1639,7 +1635,7 @@ int sphfem_leap_frog_destroy(sphfem_ctx *ctx, sphfem_leap_frog *lf) {
         SPHFEM_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         dfree(lf->pos_init); dfree(lf->vel_init); dfree(lf->S_init); dfree(lf->rho_init); dfree(lf->T_init);
         dfree(lf->cell_start); dfree(lf->cell_end); dfree(lf->near_list);
-        dfree(lf->rec); dfree(lf->psum); dfree(lf->psum_T); dfree(lf->pre_vol); dfree(lf->pre_s); dfree(lf->psum64);
+        dfree(lf->rec); dfree(lf->psum); dfree(lf->psum_T); dfree(lf->pre); dfree(lf->psum64);
         dfree(lf->rate32[0]); dfree(lf->rate32[1]);
         delete lf;
         return SPHFEM_OK;

@@ -134,6 +134,18 @@ inline RecView rec_view(float4 *base, size_t n) {
     return v;
 }
 
+// FP64 neighbour fields of n sorted particles, 16 bytes each (an L1 line holds eight records of a field):
+//   pos (blanked: x = 1e300, outside every support; padded by 4), vr = {m/rho, rho} (rho negative for tool
+//   particles), s1 = {(Sxx-p)/rho^2, Sxy/rho^2}, s2 = {(Syy-p)/rho^2, sqrtf(K/rho)}, r1 = {Rxx, Rxy},
+//   r2 = {Ryy, T}
+struct PreView {
+    sphfem_double2 *pos, *vr, *s1, *s2, *r1, *r2;
+};
+inline size_t pre_double2s(size_t n) { return 6 * n + 4; }
+inline PreView pre_view(sphfem_double2 *base, size_t n) {
+    return PreView{base, base + n + 4, base + 2 * n + 4, base + 3 * n + 4, base + 4 * n + 4, base + 5 * n + 4};
+}
+
 // FP64 pair sums of one particle (interactions_gpu.cu:143-379 outputs, T as the Laplacian)
 struct PairSums {
     sphfem_double4 v_der, S_der;
@@ -163,10 +175,9 @@ struct sphfem_ctx {
                                   // [3]: re-sort mode (1 full, 2 incremental), [4]: changed count,
                                   // [5]: non-finite pair inputs present (SPHFEM_FLAG_NONFINITE)
     double *force_scratch = nullptr;  // this device's `scratch` array (sphfem_api.cpp)
-    // interactions_monaghan: the neighbour factors of k_pre_state for the largest particle count seen
-    // (pre_vol [pre_cap], pre_s [pre_cap]) and which of its two switches the next call uses
-    double *pre_vol = nullptr;
-    sphfem_double4 *pre_s = nullptr;
+    // interactions_monaghan: the neighbour fields of k_pre_state for the largest particle count seen
+    // (pre_view, pre_cap particles) and which of its two switches the next call uses
+    sphfem_double2 *pre = nullptr;
     unsigned pre_cap = 0;
     int monaghan_turn = 0;
     sphfem::Timing timing;
@@ -282,11 +293,9 @@ struct sphfem_leap_frog {
     sphfem_double4 *S_init = nullptr;
     double *rho_init = nullptr, *T_init = nullptr;
     int *cell_start = nullptr, *cell_end = nullptr;   // only used by the unfused path
-    // FP64 form: factors of each sorted particle's neighbour terms that depend on that particle
-    // alone, computed once by the reorder with the operations the pair loop would repeat per pair:
-    // pre_vol = m/rho, pre_s = {(Sxx-p)/rho^2, Sxy/rho^2, (Syy-p)/rho^2, sqrtf(K/rho)}
-    double *pre_vol = nullptr;
-    sphfem_double4 *pre_s = nullptr;
+    // FP64 form: the neighbour fields of the sorted particles (pre_view), with the factors that depend on
+    // one particle alone computed once by the reorder, by the operations the pair loop would repeat per pair
+    sphfem_double2 *pre = nullptr;
     sphfem::PairSums *psum64 = nullptr;   // FP64 form: pair sums of the sorted particles
     int *near_list = nullptr;      // [num_part] particles near the tool
     bool intermediates = false;    // also write S_der / v_der in the fused step

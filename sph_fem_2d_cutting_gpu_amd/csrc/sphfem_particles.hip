@@ -31,9 +31,14 @@ __device__ __forceinline__ void column_range(const int *__restrict__ cs, const i
     }
 }
 
-// The neighbour factors m/rho_j, (S_j - p_j)/rho_j^2, S_xy,j/rho_j^2 and sqrtf(K/rho_j) come from
-// pre_vol / pre_s, computed once per particle with the operations the reference repeats per pair, so
-// the sums are bit-identical.  The in-support neighbours go through a per-lane list of CHUNK entries in
+// The neighbour fields come from pre (PreView), with the factors m/rho_j, (S_j - p_j)/rho_j^2,
+// S_xy,j/rho_j^2 and sqrtf(K/rho_j) computed once per particle with the operations the reference repeats
+// per pair, so the sums are bit-identical.  Bound by the L1's rate of cache lines: a wavefront's 64 lists
+// drift apart, each load touches some 30 lines, and 2.3e8 of them filled 82 % of the cycles of the 1 M
+// particle step's kernel while a pair's fields took 13 loads of 8 to 32 byte records, and a candidate's
+// position and blanked flag two (503 us).  Eight loads of 16-byte records, and four candidates at a time:
+// 417 us; all eight issued before the first is used: 358 us.  Loading the next pair's fields ahead costs
+// a third of the wavefronts (188 registers): 392 us.  The in-support neighbours go through a per-lane list of CHUNK entries in
 // LDS (list = this lane's first entry, stride LIST_BS) before their terms are evaluated.
 // WIN: every non-blanked particle of the 5x5 cells is evaluated, as the reference does, instead of
 // the in-support ones only.  The kernel's zeros outside the support make the two the same sums for
@@ -42,8 +47,8 @@ __device__ __forceinline__ void column_range(const int *__restrict__ cs, const i
 template <int LIST_BS, int CHUNK, bool WIN>
 __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sphfem_particles &P, int pidx,
                                                    double thermal_alpha, const int *__restrict__ cs,
-                                                   const int *__restrict__ ce, const double *__restrict__ pre_vol,
-                                                   const sphfem_double4 *__restrict__ pre_s, int *__restrict__ list) {
+                                                   const int *__restrict__ ce, const PreView &pre,
+                                                   int *__restrict__ list) {
     const double mass = c.phys.mass;
     const double wdeltap = c.corr.wdeltap, alpha = c.corr.alpha, beta = c.corr.beta;
     const double eta = c.corr.eta, eps = c.corr.xspheps;
@@ -59,7 +64,7 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
     const double fourh2 = 4 * hi * hi;
     const double h1 = 1 / hi;
     const bool unit_wdp = wdeltap == 1.;      // w / 1 == w exactly
-    const double ci = pre_s[pidx].w;
+    const double ci = pre.s2[pidx].y;
     const int hashi = P.hash[pidx];
     const int gi = hashi / ny;
     const int gj = hashi - gi * ny;
@@ -75,7 +80,12 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
     r.T_lapl = 0.;
     // one in-support pair (xij, yij from the sorted positions); the order of the calls is the
     // reference's neighbour order, so the sums are the same whichever loop drives them
-    auto pair = [&](int iter, const sphfem_double2 pj, double xij, double yij) {
+    auto pair = [&](int iter) {
+        // every field of j is loaded before anything is computed from one
+        const sphfem_double2 pj = pre.pos[iter], vr = pre.vr[iter], r2T = pre.r2[iter], vj = P.vel[iter];
+        const sphfem_double2 s1 = pre.s1[iter], s2 = pre.s2[iter], Rj = pre.r1[iter];
+        const double hj = P.h[iter];
+        const double xij = pi.x - pj.x, yij = pi.y - pj.y;
         const bool heat = thermal_alpha != 0.;
         const double r2 = xij * xij + yij * yij;
         // the shared-reciprocal form (the 1M-particle step's k_pairs_fp64 529 -> 497 us) while the single-precision radius and the quotients by it are normal
@@ -84,15 +94,11 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
         if (!WIN && r2 > 1e-36 && r2 < 1e36) t = radial_terms(xij, yij, r2, hi, h1, heat);
         else t = radial_terms_plain(pi.x, pi.y, pj.x, pj.y, xij, yij, r2, hi, rr2_min, heat);
         const double w = t.w, w_x = t.w_x, w_y = t.w_y;
-        const double rhoj = P.rho[iter];
-        const double is_tool_j = P.tool_particle[iter];
-        if (!(is_tool_i == 1.) && !(is_tool_j == 1.)) {
-            const sphfem_double2 vj = P.vel[iter];
-            const sphfem_double4 Rj = P.R[iter];
-            const double hj = P.h[iter];
-            const double volj = pre_vol[iter];
-            const sphfem_double4 fj = pre_s[iter];
-            const double sjx = fj.x, sjy = fj.y, sjz = fj.z, cj = fj.w;
+        // the densities are positive where the window form is off (flag_nonfinite): the sign is free
+        const double volj = vr.x, rhoj = WIN ? P.rho[iter] : fabs(vr.y);
+        const bool tool_j = WIN ? P.tool_particle[iter] == 1. : vr.y < 0.;
+        if (!(is_tool_i == 1.) && !tool_j) {
+            const double sjx = s1.x, sjy = s1.y, sjz = s2.x, cj = s2.y, Rjz = r2T.x;
             r.v_der.x += (vj.x - vi.x) * w_x * volj;
             r.v_der.y += (vj.x - vi.x) * w_y * volj;
             r.v_der.z += (vj.y - vi.y) * w_x * volj;
@@ -102,7 +108,7 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
             fab *= fab;
             double Rx = fab * (Ri.x + Rj.x);
             double Ry = fab * (Ri.y + Rj.y);
-            double Rz = fab * (Ri.z + Rj.z);
+            double Rz = fab * (Ri.z + Rjz);
             r.S_der.x += mass * ((Si.x - prsi) * rhoi21 + sjx + Rx) * w_x;
             r.S_der.y += mass * (Si.y * rhoi21 + sjy + Ry) * w_y;
             r.S_der.z += mass * (Si.y * rhoi21 + sjy + Ry) * w_x;
@@ -131,8 +137,7 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
             r.pos_t.y += xsph * vijy;
         }
         if (heat && t.rij > 1e-8) {
-            const double Tj = P.T[iter];
-            r.T_lapl += 2.0 * pre_vol[iter] * (Ti - Tj) * t.rij1 * (t.ex * w_x + t.ey * w_y);
+            r.T_lapl += 2.0 * volj * (Ti - r2T.y) * t.rij1 * (t.ex * w_x + t.ey * w_y);
         }
     };
     // the in-support neighbours are listed first (in the same order) and the pair terms are
@@ -141,9 +146,7 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
     int n = 0;
     auto run = [&]() {
         for (int k = 0; k < n; k++) {
-            const int iter = list[k * LIST_BS];
-            const sphfem_double2 pj = P.pos[iter];
-            pair(iter, pj, pi.x - pj.x, pi.y - pj.y);
+            pair(list[k * LIST_BS]);
         }
         n = 0;
     };
@@ -151,18 +154,25 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
         int first, last;
         column_range(cs, ce, ii * ny, low_j, high_j, first, last);
         if (first < 0 || last > (int)P.N) continue;
-        for (int iter = first; iter < last; iter++) {
-            if (P.blanked[iter] == 1.) continue;
-            const sphfem_double2 pj = P.pos[iter];
-            double xij = pi.x - pj.x;
-            double yij = pi.y - pj.y;
-            double rr2 = xij * xij + yij * yij;
-            if (!WIN && (rr2 >= fourh2 || rr2 < rr2_min)) continue;
-            list[n * LIST_BS] = iter;
-            ++n;
+        for (int it4 = first; it4 < last; it4 += 4) {
+            // four positions, loaded together; up to three past `last` are read and not used
+            sphfem_double2 q[4];
+#pragma unroll
+            for (int k = 0; k < 4; k++) q[k] = pre.pos[it4 + k];
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                const int iter = it4 + k;
+                if (iter >= last) break;
+                double xij = pi.x - q[k].x;
+                double yij = pi.y - q[k].y;
+                double rr2 = xij * xij + yij * yij;
+                if (WIN ? P.blanked[iter] == 1. : (rr2 >= fourh2 || rr2 < rr2_min)) continue;
+                list[n * LIST_BS] = iter;
+                ++n;
+            }
             // a full list empties every active lane's list at once: lanes that flushed at
             // their own points would each run their list with the rest of the wavefront idle
-            if (__any(n == CHUNK)) run();
+            if (__any(n > CHUNK - 4)) run();
         }
     }
     run();
@@ -980,9 +990,8 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
 // per pair), and the switch to the reference's full window: a live particle with a non-finite input
 // or factor, or with a density out of the range of flag_nonfinite (a zero kernel value times such a
 // factor is not zero).
-__global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_particles P, double *__restrict__ pre_vol,
-                                                   sphfem_double4 *__restrict__ pre_s, int *__restrict__ window,
-                                                   int *__restrict__ next_window) {
+__global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_particles P, const PreView pre,
+                                                   int *__restrict__ window, int *__restrict__ next_window) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i == 0) *next_window = 0;
     if (i >= (int)P.N) return;
@@ -993,8 +1002,12 @@ __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_par
     const double vol = c.phys.mass / rho;
     const double rho21 = 1. / (rho * rho);
     const sphfem_double4 f = {(S.x - pr) * rho21, S.y * rho21, (S.z - pr) * rho21, sqrtf_d(c.phys.K / rho)};
-    pre_vol[i] = vol;
-    pre_s[i] = f;
+    pre.pos[i] = {blanked == 1. ? 1e300 : pos.x, pos.y};
+    pre.vr[i] = {vol, P.tool_particle[i] == 1. ? -rho : rho};
+    pre.s1[i] = {f.x, f.y};
+    pre.s2[i] = {f.z, f.w};
+    pre.r1[i] = {R.x, R.y};
+    pre.r2[i] = {R.z, T};
     const double s = ((pos.x + pos.y) + (vel.x + vel.y)) + ((T + h) + (R.x + R.y)) + (R.z + vol) +
                      ((f.x + f.y) + (f.z + f.w));
     if (blanked != 1. && !(isfinite(s) && rho > SPHFEM_RHO_MIN && rho < SPHFEM_RHO_MAX)) *window = 1;
@@ -1008,8 +1021,7 @@ __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_par
 // 2.07M particles of the chip domain, this and k_pre_state 2140 us, 2010 us with the shared reciprocals.
 __global__ void __launch_bounds__(256) k_interactions_ref(DevConsts c, sphfem_particles P, const int *__restrict__ cs,
                                                           const int *__restrict__ ce,
-                                                          const double *__restrict__ pre_vol,
-                                                          const sphfem_double4 *__restrict__ pre_s,
+                                                          const PreView pre,
                                                           const int *__restrict__ window) {
     __shared__ int nb_list[48 * 256];
     const int pidx = xcd_logical_block() * 256 + (int)threadIdx.x;
@@ -1018,10 +1030,10 @@ __global__ void __launch_bounds__(256) k_interactions_ref(DevConsts c, sphfem_pa
     const double thermal_alpha = interaction_alpha(c, P.tool_particle[pidx]);
     PairSums r;
     if (*window != 0)
-        r = pair_sums_fp64<256, 48, true>(c, P, pidx, thermal_alpha, cs, ce, pre_vol, pre_s,
+        r = pair_sums_fp64<256, 48, true>(c, P, pidx, thermal_alpha, cs, ce, pre,
                                                 nb_list + threadIdx.x);
     else
-        r = pair_sums_fp64<256, 48, false>(c, P, pidx, thermal_alpha, cs, ce, pre_vol, pre_s,
+        r = pair_sums_fp64<256, 48, false>(c, P, pidx, thermal_alpha, cs, ce, pre,
                                                  nb_list + threadIdx.x);
     P.S_der[pidx] = r.S_der;
     P.v_der[pidx] = r.v_der;
@@ -1082,10 +1094,11 @@ void launch_interactions_ref(sphfem_ctx *ctx, const sphfem_particles &p, const i
     int *next_window = ctx->d_flags + SPHFEM_FLAG_MONAGHAN + ctx->monaghan_turn;
     {
         KTimer t(ctx, "interactions_pre");
-        k_pre_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, ctx->pre_vol, ctx->pre_s, window, next_window);
+        k_pre_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, pre_view(ctx->pre, p.N), window, next_window);
     }
     KTimer t(ctx, "interactions_ref");
-    k_interactions_ref<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, cs, ce, ctx->pre_vol, ctx->pre_s, window);
+    k_interactions_ref<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, cs, ce, pre_view(ctx->pre, p.N),
+                                                                window);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1227,8 +1240,7 @@ void launch_leapfrog(sphfem_ctx *ctx, int which, const sphfem_particles &p, sphf
 // every particle is evaluated with the reference's full window.
 template <int BS>
 __global__ void __launch_bounds__(BS) k_pairs_fp64(DevConsts c, sphfem_particles B, const int *__restrict__ cs,
-                                                   const int *__restrict__ ce, const double *__restrict__ pre_vol,
-                                                   const sphfem_double4 *__restrict__ pre_s,
+                                                   const int *__restrict__ ce, const PreView pre,
                                                    PairSums *__restrict__ psum64, const int *__restrict__ nonfinite) {
     constexpr int CHUNK = 48;
     __shared__ int nb_list[CHUNK * BS];
@@ -1238,10 +1250,10 @@ __global__ void __launch_bounds__(BS) k_pairs_fp64(DevConsts c, sphfem_particles
     const double thermal_alpha = interaction_alpha(c, B.tool_particle[i]);
     // the window form when a live particle carries a non-finite input (see pair_sums_fp64)
     if ((*nonfinite & SPHFEM_FORM_WINDOW) != 0)
-        psum64[i] = pair_sums_fp64<BS, CHUNK, true>(c, B, i, thermal_alpha, cs, ce, pre_vol, pre_s,
+        psum64[i] = pair_sums_fp64<BS, CHUNK, true>(c, B, i, thermal_alpha, cs, ce, pre,
                                                           nb_list + threadIdx.x);
     else
-        psum64[i] = pair_sums_fp64<BS, CHUNK, false>(c, B, i, thermal_alpha, cs, ce, pre_vol, pre_s,
+        psum64[i] = pair_sums_fp64<BS, CHUNK, false>(c, B, i, thermal_alpha, cs, ce, pre,
                                                            nb_list + threadIdx.x);
 }
 
@@ -1404,10 +1416,10 @@ void launch_fused_update(sphfem_ctx *ctx, const sphfem_particles &B, const sphfe
         {
             KTimer tp(ctx, "pairs_fp64");
             if (lf->tuning.pair_block == 128)
-                k_pairs_fp64<128><<<nblk(B.N, 128), 128, 0, ctx->stream>>>(ctx->c, B, cs, ce, lf->pre_vol, lf->pre_s,
+                k_pairs_fp64<128><<<nblk(B.N, 128), 128, 0, ctx->stream>>>(ctx->c, B, cs, ce, pre_view(lf->pre, B.N),
                                                                             lf->psum64, nf);
             else
-                k_pairs_fp64<256><<<nblk(B.N, 256), 256, 0, ctx->stream>>>(ctx->c, B, cs, ce, lf->pre_vol, lf->pre_s,
+                k_pairs_fp64<256><<<nblk(B.N, 256), 256, 0, ctx->stream>>>(ctx->c, B, cs, ce, pre_view(lf->pre, B.N),
                                                                             lf->psum64, nf);
         }
         KTimer tm(ctx, "fused_update");

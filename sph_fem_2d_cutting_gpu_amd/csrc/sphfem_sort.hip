@@ -1161,8 +1161,7 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
                                                          sphfem_double4 *__restrict__ S_init,
                                                          double *__restrict__ rho_init, double *__restrict__ T_init,
                                                          int num_cell, int *__restrict__ flags,
-                                                         double *__restrict__ pre_vol,
-                                                         sphfem_double4 *__restrict__ pre_s, ResortView rs) {
+                                                         const PreView pre, ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
     int h, s;
@@ -1207,20 +1206,30 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
     b.eps_pl_dot[i] = p.eps_pl_dot[s];
     b.fixed[i] = p.fixed[s];
     b.on_seg[i] = p.on_seg[s];
-    // the neighbour factors of interactions_gpu.cu:247-252, 283-285 (m/rho_j in the heat term, :352)
-    pre_vol[i] = c.phys.mass / rho;
+    // the neighbour fields of interactions_gpu.cu:247-252, 283-285 (m/rho_j in the heat term, :352)
+    const bool tool_rec = tool == 1.;
+    pre.pos[i] = {blanked == 1. ? 1e300 : pos.x, pos.y};
+    pre.vr[i] = {c.phys.mass / rho, tool_rec ? -rho : rho};
     if (tool == 0.) {
         const double pr = eos_pressure(c, rho);
+        const sphfem_double4 R = artificial_stress(c, rho, pr, S);
         b.p[i] = pr;
-        b.R[i] = artificial_stress(c, rho, pr, S);
+        b.R[i] = R;
         const double rho21 = 1. / (rho * rho);
-        pre_s[i] = {(S.x - pr) * rho21, S.y * rho21, (S.z - pr) * rho21, sqrtf_d(c.phys.K / rho)};
-        flag_nonfinite(flags, blanked, pos, vel, S, rho, T, p.h[s], pr, b.R[i]);
+        pre.s1[i] = {(S.x - pr) * rho21, S.y * rho21};
+        pre.s2[i] = {(S.z - pr) * rho21, sqrtf_d(c.phys.K / rho)};
+        pre.r1[i] = {R.x, R.y};
+        pre.r2[i] = {R.z, T};
+        flag_nonfinite(flags, blanked, pos, vel, S, rho, T, p.h[s], pr, R);
     } else {
         // neither gathered nor computed for tool particles by the reference: they stay in place
+        const sphfem_double4 R = p.R[i];
         b.p[i] = p.p[i];
-        b.R[i] = p.R[i];
-        pre_s[i] = {0., 0., 0., 0.};   // the pair loop skips these terms for tool particles
+        b.R[i] = R;
+        pre.s1[i] = {0., 0.};   // the pair loop skips these terms for tool particles
+        pre.s2[i] = {0., 0.};
+        pre.r1[i] = {R.x, R.y};
+        pre.r2[i] = {R.z, T};
         flag_nonfinite(flags, blanked, pos, vel, sphfem_double4{0., 0., 0., 0.}, rho, T, p.h[s], 0.,
                        sphfem_double4{0., 0., 0., 0.});
     }
@@ -1286,7 +1295,7 @@ void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_partic
     k_reorder_predict<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, g->buf, g->cell_start, g->cell_end,
                                                                lf->pos_init, lf->vel_init, lf->S_init,
                                                                lf->rho_init, lf->T_init, g->num_cell,
-                                                               ctx->d_flags, lf->pre_vol, lf->pre_s, rs);
+                                                               ctx->d_flags, pre_view(lf->pre, p.N), rs);
 }
 
 }  // namespace sphfem
