@@ -55,8 +55,8 @@ def measured_traffic(kernel, workload_key):
     with open(path) as f:
         t = json.load(f)
     # (name prefix, template-argument tail) of the kernel's instantiations
-    sel = {"pairs_fp32c": ("sphfem::k_pairs_fp32c<", ", false, false>"),
-           "pairs_update_fp32c": ("sphfem::k_pairs_fp32c<", ", true, false>"),
+    sel = {"pairs_fp32c": ("sphfem::k_pairs_fp32c<", ", 0, false>"),
+           "pairs_update_fp32c": ("sphfem::k_pairs_fp32c<", ", 1, false>"),
            "pairs_fp64": ("sphfem::k_pairs_fp64<", ">"),
            "fused_update": ("sphfem::k_fused_update<false,", ", false>"),
            "update_fp32c": ("sphfem::k_fused_update<true,", ", false>")}.get(kernel)

@@ -42,7 +42,10 @@
 #define SPHFEM_FLAG_MONAGHAN 8
 // workgroups of the near-tool pass that are done; zero between launches
 #define SPHFEM_FLAG_NEAR_DONE 10
-#define SPHFEM_NUM_FLAGS 11
+// interactions_monaghan_fp32c's own two words of the pair sums' form, used in turn like those of
+// interactions_monaghan
+#define SPHFEM_FLAG_MONAGHAN_FP32C 11
+#define SPHFEM_NUM_FLAGS 13
 // position records a wavefront of the staged FP32C pair kernel copies into LDS (8 KiB)
 #define SPHFEM_STAGE_CAP 512
 // blocks of the report_force reduction (its partials: 2 doubles per block) and the largest particle
@@ -180,6 +183,7 @@ struct sphfem_ctx {
     sphfem_double2 *pre = nullptr;
     unsigned pre_cap = 0;
     int monaghan_turn = 0;
+    int fp32c_turn = 0;           // the same for interactions_monaghan_fp32c
     sphfem::Timing timing;
 };
 
@@ -406,7 +410,8 @@ void launch_reorder_full(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles
 // sorted order comes from launch_resort, not from p.hash and p.idx
 void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, sphfem_leap_frog *lf,
                             const RateView *rates, bool resorted);
-void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, const RecView &rec);
+void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, const RecView &rec, int *form,
+                          int *next_form);
 
 // particles (sphfem_particles.hip)
 void launch_actions(sphfem_ctx *ctx, int which, const sphfem_particles &p);

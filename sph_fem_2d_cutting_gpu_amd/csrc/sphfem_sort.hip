@@ -1017,13 +1017,13 @@ void launch_rothlin_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p) {
 // where such a neighbour turns the sums NaN even outside the kernel support.  A finite sum that
 // overflows, or a density outside [SPHFEM_RHO_MIN, SPHFEM_RHO_MAX], only sends the step down that
 // (exact, slower) path.
-__device__ __forceinline__ void flag_nonfinite(int *__restrict__ flags, double blanked, sphfem_double2 pos,
+__device__ __forceinline__ void flag_nonfinite(int *__restrict__ form, double blanked, sphfem_double2 pos,
                                                sphfem_double2 vel, sphfem_double4 S, double rho, double T, double h,
                                                double pr, sphfem_double4 R) {
     const double s = ((pos.x + pos.y) + (vel.x + vel.y)) + ((S.x + S.y) + (S.z + rho)) + ((T + h) + (pr + R.x)) +
                      (R.y + R.z);
     if (blanked != 1. && !(isfinite(s) && rho > SPHFEM_RHO_MIN && rho < SPHFEM_RHO_MAX))
-        atomicOr(&flags[SPHFEM_FLAG_NONFINITE], 1);
+        atomicOr(form, SPHFEM_FORM_WINDOW);
 }
 
 // FP32C neighbour records (RecView) of one sorted particle.  The position is rounded to cell / 2^28 from
@@ -1031,7 +1031,7 @@ __device__ __forceinline__ void flag_nonfinite(int *__restrict__ flags, double b
 // factors of the pair sum, (S - p)/rho^2 and S_xy/rho^2; the temperature is stored as T - T_init, so
 // that the FP32 differences T_i - T_j of a nearly uniform field keep ~1e-7 of the deviation instead of
 // ~1e-7 of T.
-__device__ __forceinline__ void write_records(const DevConsts &c, const RecView &rec, double inv_dx, int *__restrict__ flags, int i, int h,
+__device__ __forceinline__ void write_records(const DevConsts &c, const RecView &rec, double inv_dx, int *__restrict__ form_word, int i, int h,
                                              sphfem_double2 pos, sphfem_double2 vel, sphfem_double4 S, double rho, double T, double blanked,
                                              double tool, double hh, double pr, sphfem_double4 R) {
     const int ny = c.geom.ny;
@@ -1068,8 +1068,8 @@ __device__ __forceinline__ void write_records(const DevConsts &c, const RecView 
     const int form = (__any(live && !near) ? SPHFEM_FORM_AWAY : 0) |
                      (__any(live && hh != c.geom.dx) ? SPHFEM_FORM_WIDTH : 0);
     if (form != 0 && (int)__lane_id() == __ffsll((long long)__ballot(1)) - 1 &&
-        (form & ~flags[SPHFEM_FLAG_NONFINITE]) != 0)
-        atomicOr(&flags[SPHFEM_FLAG_NONFINITE], form);
+        (form & ~*form_word) != 0)
+        atomicOr(form_word, form);
     const double inv_rho = 1. / rho, rho21 = inv_rho * inv_rho;
     const float vol = (float)(c.phys.mass * inv_rho);
     float4 r1, r2, r3;
@@ -1097,9 +1097,11 @@ __device__ __forceinline__ void write_records(const DevConsts &c, const RecView 
 // (interactions_gpu.cu:143-379 reads them from the particle arrays)
 __global__ void __launch_bounds__(256) k_records_state(DevConsts c, const sphfem_particles p, int num_cell,
                                                        int *__restrict__ flags, const RecView rec,
-                                                       double inv_dx) {
+                                                       double inv_dx, int *__restrict__ form,
+                                                       int *__restrict__ next_form) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
+    if (i == 0) *next_form = 0;
     if (i >= N) return;
     int h = p.hash[i];
     if ((unsigned)h >= (unsigned)num_cell) {
@@ -1112,14 +1114,15 @@ __global__ void __launch_bounds__(256) k_records_state(DevConsts c, const sphfem
     const sphfem_double2 pos = p.pos[i], vel = p.vel[i];
     const sphfem_double4 S = p.S[i];
     const double rho = p.rho[i], T = p.T[i], blanked = p.blanked[i], hh = p.h[i];
-    flag_nonfinite(flags, blanked, pos, vel, S, rho, T, hh, pr, R);
-    write_records(c, rec, inv_dx, flags, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
+    flag_nonfinite(form, blanked, pos, vel, S, rho, T, hh, pr, R);
+    write_records(c, rec, inv_dx, form, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
 }
 
-void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, const RecView &rec) {
+void launch_records_state(sphfem_ctx *ctx, const sphfem_particles &p, int num_cell, const RecView &rec, int *form,
+                          int *next_form) {
     KTimer t(ctx, "records_state");
     k_records_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, num_cell, ctx->d_flags, rec,
-                                                             1. / ctx->c.geom.dx);
+                                                             1. / ctx->c.geom.dx, form, next_form);
 }
 
 // source and key of sorted position i (from the re-sort's lists, or the sorted arrays when there are
@@ -1164,6 +1167,7 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
                                                          const PreView pre, ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
+    int *form = flags + SPHFEM_FLAG_NONFINITE;
     int h, s;
     if (!cell_bounds(p, rs, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
     sphfem_double2 pos = p.pos[s], vel = p.vel[s];
@@ -1220,7 +1224,7 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
         pre.s2[i] = {(S.z - pr) * rho21, sqrtf_d(c.phys.K / rho)};
         pre.r1[i] = {R.x, R.y};
         pre.r2[i] = {R.z, T};
-        flag_nonfinite(flags, blanked, pos, vel, S, rho, T, p.h[s], pr, R);
+        flag_nonfinite(form, blanked, pos, vel, S, rho, T, p.h[s], pr, R);
     } else {
         // neither gathered nor computed for tool particles by the reference: they stay in place
         const sphfem_double4 R = p.R[i];
@@ -1230,7 +1234,7 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
         pre.s2[i] = {0., 0.};
         pre.r1[i] = {R.x, R.y};
         pre.r2[i] = {R.z, T};
-        flag_nonfinite(flags, blanked, pos, vel, sphfem_double4{0., 0., 0., 0.}, rho, T, p.h[s], 0.,
+        flag_nonfinite(form, blanked, pos, vel, sphfem_double4{0., 0., 0., 0.}, rho, T, p.h[s], 0.,
                        sphfem_double4{0., 0., 0., 0.});
     }
 }
@@ -1246,6 +1250,7 @@ __global__ void __launch_bounds__(256) k_reorder_records(DevConsts c, const sphf
                                                          ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
+    int *form = flags + SPHFEM_FLAG_NONFINITE;
     int h, s;
     if (!cell_bounds(p, rs, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
     sphfem_double2 pos = ld_stream(&p.pos[s]), vel = ld_stream(&p.vel[s]);
@@ -1276,8 +1281,8 @@ __global__ void __launch_bounds__(256) k_reorder_records(DevConsts c, const sphf
         R = artificial_stress(c, rho, pr, S);
     }
     const double hh = ld_stream(&p.h[s]);
-    flag_nonfinite(flags, blanked, pos, vel, tool == 0. ? S : sphfem_double4{0., 0., 0., 0.}, rho, T, hh, pr, R);
-    write_records(c, rec, inv_dx, flags, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
+    flag_nonfinite(form, blanked, pos, vel, tool == 0. ? S : sphfem_double4{0., 0., 0., 0.}, rho, T, hh, pr, R);
+    write_records(c, rec, inv_dx, form, i, h, pos, vel, S, rho, T, blanked, tool, hh, pr, R);
 }
 
 void launch_reorder_predict(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particles &p, sphfem_leap_frog *lf,
