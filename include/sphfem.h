@@ -186,7 +186,7 @@ int sphfem_interactions_setup_geometry_constants(sphfem_ctx *ctx, const sphfem_g
 int sphfem_interactions_monaghan(sphfem_ctx *ctx, sphfem_particles *p, const int *cell_start,
                                  const int *cell_end, int num_cell);
 /* interactions_gpu.cu:466-474 in the FP32-compensated form (the pair sums of
- * sphfem_leap_frog_step with SPHFEM_FP32C, lf set to that precision): FP32 terms on cell-relative
+ * sphfem_leap_frog_step with SPHFEM_FP32C, lf set to that precision): FP32 terms on wrapped integer
  * positions, FP32 blocks of 8 terms accumulated in FP64, from the sorted state p (p and R as left
  * by material_eos and corrector_artificial_stress).  Writes v_der, pos_t and T_t as the reference
  * does; the stress-divergence and viscous accelerations come summed per axis as S_der = {ax, 0,

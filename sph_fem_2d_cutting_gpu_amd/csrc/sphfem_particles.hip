@@ -1033,7 +1033,8 @@ __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_par
 // particle of the 5x5 cells is evaluated, as the reference visits them.  Bound by the neighbour gathers
 // and the FP64 arithmetic of the in-support pairs: evaluating the whole window instead (about twice
 // the pairs, with each neighbour's factors divided out again per pair) took 3106 us per launch at
-// 2.07M particles of the chip domain, this and k_pre_state 2140 us, 2010 us with the shared reciprocals.
+// 2.07M particles of the chip domain, this and k_pre_state 2140 us, 2010 us with the shared reciprocals,
+// 1320 us with the fields in 16-byte records (pair_sums_fp64).
 __global__ void __launch_bounds__(256) k_interactions_ref(DevConsts c, sphfem_particles P, const int *__restrict__ cs,
                                                           const int *__restrict__ ce,
                                                           const PreView pre,
