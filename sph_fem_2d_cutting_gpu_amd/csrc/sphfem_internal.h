@@ -138,12 +138,17 @@ inline RecView rec_view(float4 *base, size_t n) {
 }
 
 // FP64 neighbour fields of n sorted particles, 16 bytes each (an L1 line holds eight records of a field):
-//   pos (blanked: x = 1e300, outside every support; padded by 4), vr = {m/rho, rho} (rho negative for tool
+//   pos (blanked: scan_pos, outside every support; padded by 4), vr = {m/rho, rho} (rho negative for tool
 //   particles), s1 = {(Sxx-p)/rho^2, Sxy/rho^2}, s2 = {(Syy-p)/rho^2, sqrtf(K/rho)}, r1 = {Rxx, Rxy},
 //   r2 = {Ryy, T}
 struct PreView {
     sphfem_double2 *pos, *vr, *s1, *s2, *r1, *r2;
 };
+// the pos field: a blanked particle is put out of every support, both coordinates, as its own may be NaN and
+// a NaN distance fails every comparison
+__device__ __forceinline__ sphfem_double2 scan_pos(double blanked, sphfem_double2 pos) {
+    return blanked == 1. ? sphfem_double2{1e300, 1e300} : pos;
+}
 inline size_t pre_double2s(size_t n) { return 6 * n + 4; }
 inline PreView pre_view(sphfem_double2 *base, size_t n) {
     return PreView{base, base + n + 4, base + 2 * n + 4, base + 3 * n + 4, base + 4 * n + 4, base + 5 * n + 4};

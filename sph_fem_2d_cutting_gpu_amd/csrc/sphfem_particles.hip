@@ -1017,7 +1017,7 @@ __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_par
     const double vol = c.phys.mass / rho;
     const double rho21 = 1. / (rho * rho);
     const sphfem_double4 f = {(S.x - pr) * rho21, S.y * rho21, (S.z - pr) * rho21, sqrtf_d(c.phys.K / rho)};
-    pre.pos[i] = {blanked == 1. ? 1e300 : pos.x, pos.y};
+    pre.pos[i] = scan_pos(blanked, pos);
     pre.vr[i] = {vol, P.tool_particle[i] == 1. ? -rho : rho};
     pre.s1[i] = {f.x, f.y};
     pre.s2[i] = {f.z, f.w};

@@ -1212,7 +1212,7 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
     b.on_seg[i] = p.on_seg[s];
     // the neighbour fields of interactions_gpu.cu:247-252, 283-285 (m/rho_j in the heat term, :352)
     const bool tool_rec = tool == 1.;
-    pre.pos[i] = {blanked == 1. ? 1e300 : pos.x, pos.y};
+    pre.pos[i] = scan_pos(blanked, pos);
     pre.vr[i] = {c.phys.mass / rho, tool_rec ? -rho : rho};
     if (tool == 0.) {
         const double pr = eos_pressure(c, rho);
