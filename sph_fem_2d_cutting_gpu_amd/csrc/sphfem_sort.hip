@@ -616,9 +616,7 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
                 vo[dst] = val[q];
             }
         }
-        // this item's writes before it counts as done: the barrier orders the workgroup's before lane 0's
-        // fence (a fence by every wavefront writes the L2 back sixteen times)
-        __syncthreads();
+        stores_done_barrier();                        // this item's writes before it counts as done
         if (tid == 0) {
             __threadfence();
             atomicAdd(&sync[RS_DONE + phase], 1);
