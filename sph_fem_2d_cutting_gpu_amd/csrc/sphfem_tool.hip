@@ -1036,7 +1036,7 @@ __global__ void __launch_bounds__(NEAR_BS) k_near_contact(DevConsts c, sphfem_pa
         if (bad) blanked = 1.;
         if (blanked == 1.) P.blanked[i] = 1.;
     }
-    __syncthreads();
+    stores_done_barrier();
     if (threadIdx.x == 0) {
         if (s_records) __threadfence();               // this workgroup's records, before it counts
         s_last = atomicAdd(&counters[SPHFEM_FLAG_NEAR_DONE], 1) == (int)gridDim.x - 1;

@@ -31,7 +31,7 @@ def _body(asm, kernel):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="no hipcc")
-@pytest.mark.parametrize("source,kernel", [("sphfem_sort.hip", "k_resort")])
+@pytest.mark.parametrize("source,kernel", [("sphfem_sort.hip", "k_resort"), ("sphfem_tool.hip", "k_near_contact")])
 def test_every_wavefront_waits_for_its_stores(source, kernel, tmp_path):
     lines = _body(_assembly(source, tmp_path), kernel)
     found = 0
