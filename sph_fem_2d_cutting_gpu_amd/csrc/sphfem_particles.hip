@@ -685,9 +685,11 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
     const double alpha_i = tool_i ? c.trml_itool.alpha : c.trml_wp.alpha;
     const double dxc = c.geom.dx;
     const double hi = GEN ? (double)rv.h[i] : dxc;
-    if (a3.z != -INFINITY && (!tool_i || alpha_i != 0.)) {
-        const int nx = c.geom.nx, ny = c.geom.ny;
-        const int hashi = hash[i];
+    // nor does one whose key names no cell (the records' kernel reported it): its window's entries are read
+    // before their columns are known to exist
+    const int nx = c.geom.nx, ny = c.geom.ny;
+    const int hashi = hash[i];
+    if (a3.z != -INFINITY && (!tool_i || alpha_i != 0.) && (unsigned)hashi < (unsigned)(nx * ny)) {
         const int gi = hashi / ny;
         const int gj = hashi - gi * ny;
         const int low_j = gj - 2 < 0 ? 0 : gj - 2;
