@@ -760,12 +760,12 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
         // dense list of the entries in front of list[end]: two per iteration, the records of the next
         // entry loaded before the current one is evaluated (ping-pong registers, no copies); each list
         // entry is read from LDS one pair term before its records are loaded, so the LDS latency passes
-        // under that term.  The two entries past the end, which are loaded and not evaluated, are i itself.
+        // under that term.  The two entries past the end, which are loaded and not evaluated, repeat the
+        // last one (i itself need not be among the records that Pos holds, if the cell table leaves it out).
         auto run_list = [&](int end) {
             if (end <= 0) return;
             PairAcc acc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-            list[end] = pos.encode(2, i);
-            list[end + BS] = pos.encode(2, i);
+            list[end] = list[end + BS] = list[end - BS];
             typename Pos::Entry eA = list[0];
             typename Pos::Entry eB = list[BS];
             unsigned oA = pos.index(eA) << 4;

@@ -63,3 +63,24 @@ def test_keys_outside_the_grid_are_reported(kernel):
     for f in OUT:
         assert_equal(f, got[f], want[f])
     s.close()
+
+
+@pytest.mark.parametrize("chunk", [16, 32, 48])
+def test_cell_tables_that_leave_particles_out(chunk):
+    """Every third column missing from the table, and some cells of the others: a particle's own column may
+    have no records.  The staged kernel's sums equal the list kernel's bit for bit."""
+    s = Pass(50_000)
+    geo, start = s.sim.grid.geom, s.sim.ctx.dtoh(s.cells[0].value, s.nc, np.int32)
+    cell = np.arange(s.nc)
+    start[((cell // geo.ny) % 3 == 1) | (cell % 11 == 4)] = -1
+    s.sim.ctx.htod(s.cells[0].value, start)
+    out = []
+    for kernel in (_lib.PAIRS_LIST, _lib.PAIRS_STAGED):
+        s.sim.set_tuning(pair_kernel=kernel, pair_chunk=chunk)
+        print("partial table", kernel, chunk, flush=True)
+        out.append(s.sums())
+        s.sim.ctx.check_error()
+    for f in OUT:
+        assert np.all(np.isfinite(out[0][f])), f
+        assert_equal(f, out[1][f], out[0][f])
+    s.close()
