@@ -20,8 +20,9 @@ namespace sphfem {
 #define SPHFEM_HD inline
 #endif
 
-// a divisor and its reciprocal, correctly rounded but (by an ulp) for some of the divisors in the last
-// 2^-46 below a power of two; the quotients by such a divisor are correctly rounded all the same
+// a divisor and its reciprocal, by recip_from within an ulp of the correctly rounded one.  With that
+// reciprocal the quotients are correctly rounded, but for dividends that are powers of two by a divisor
+// whose fraction bits are all ones (where 1 / b lies 2^-106 beyond the middle of two numbers).
 struct Recip {
     double b, y;
 };
@@ -30,6 +31,17 @@ struct Recip {
 SPHFEM_HD Recip recip_from(double b, double y0) {
     const double y = std::fma(std::fma(-b, y0, 1.), y0, y0);
     return {b, std::fma(std::fma(-b, y, 1.), y, y)};
+}
+
+// the correctly rounded reciprocal, from a seed of at least 40 good bits: the first step ends within an ulp,
+// and the second then rounds correctly for every divisor but one with all ones (Markstein), which is divided
+// out.  The upper fraction bits select a few divisors more.
+SPHFEM_HD Recip recip_rounded(double b, double y0) {
+    Recip r = recip_from(b, y0);
+    unsigned long long bits;
+    __builtin_memcpy(&bits, &b, 8);
+    if (((bits >> 32) & 0xfffff) == 0xfffff) r.y = 1. / b;
+    return r;
 }
 
 SPHFEM_HD double quot(double a, const Recip &r) {

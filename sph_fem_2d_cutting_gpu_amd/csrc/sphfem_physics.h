@@ -86,7 +86,7 @@ __device__ __forceinline__ RadialTerms radial_terms(double xij, double yij, doub
     t.w_y = der * yij * fac;
     if (heat) {
         t.rij = sqrt_from(rr2, y0, h);
-        const Recip r = recip_from(t.rij, 2. * h);
+        const Recip r = recip_rounded(t.rij, 2. * h);
         t.rij1 = r.y;
         t.ex = quot(xij, r);
         t.ey = quot(yij, r);

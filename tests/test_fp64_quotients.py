@@ -52,3 +52,46 @@ def test_quotients_and_roots_are_correctly_rounded(tmp_path):
     exe = tmp_path / "q"
     subprocess.run(["g++", "-O2", "-mfma", "-ffp-contract=off", "-std=c++17", str(src), "-o", str(exe)], check=True)
     assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.strip() == "0"
+
+
+ROUNDED = r"""
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <random>
+#include "%s/sph_fem_2d_cutting_gpu_amd/csrc/sphfem_fpmath.h"
+using namespace sphfem;
+int main() {
+    std::mt19937_64 g(4);
+    std::uniform_real_distribution<double> u(-1, 1);
+    long bad = 0, plain = 0;
+    for (long k = 0; k < 4000000; k++) {
+        // roots whose fraction bits are random, or all ones but for up to 63 units
+        unsigned long long m = (1ull << 52) - 1 - (k %% 2 ? g() %% 64 : g() >> 12);
+        m |= (unsigned long long)(1023 + (int)(60 * u(g))) << 52;
+        double b, h;
+        std::memcpy(&b, &m, 8);
+        const double x = b * b;
+        const double q = sqrt_from(x, 1 / std::sqrt(x) * (1 + u(g) * std::ldexp(1, -20)), h);
+        bad += q != std::sqrt(x);
+        const Recip r = recip_rounded(q, 2 * h);
+        const double a = k %% 3 ? q * u(g) : std::ldexp(1, (int)(60 * u(g)));
+        bad += r.y != 1 / q;
+        bad += quot(a, r) != a / q;
+        plain += recip_from(q, 2 * h).y != 1 / q;
+    }
+    std::printf("%%ld %%d\n", bad, plain > 0);
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_reciprocals_of_double_roots_are_correctly_rounded(tmp_path):
+    """1 / distance of the heat term, which is used itself and not only in quotients; the unrounded form
+    differs at the divisors of all ones that the test holds."""
+    src = tmp_path / "r.cpp"
+    src.write_text(ROUNDED % ROOT)
+    exe = tmp_path / "r"
+    subprocess.run(["g++", "-O2", "-mfma", "-ffp-contract=off", "-std=c++17", str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split() == ["0", "1"]
