@@ -4,8 +4,9 @@
 // and q within an ulp or two of a / b, q + (a - b q) y rounded once is the correctly rounded quotient.
 // A pair of the FP64 sums divides three times by its distance and twice by its mean density; one
 // reciprocal serves each, where a division of its own per quotient repeats the reciprocal and adds the
-// scaling of extreme operands.  Valid for divisors and radicands whose reciprocal, square and remainder
-// are normal numbers; the callers keep others on the plain operators.
+// scaling of extreme operands.  Valid for operands whose reciprocal, square, quotient and remainder are
+// normal numbers; the callers keep others on the plain operators (quot_holds; a coordinate difference below
+// 1e-290 in a unit vector may round the other way).
 //
 // y0 is a seed of at least 20 good bits: the hardware's approximation, or any other in a host test.
 #pragma once
@@ -47,6 +48,14 @@ SPHFEM_HD Recip recip_rounded(double b, double y0) {
 SPHFEM_HD double quot(double a, const Recip &r) {
     const double q = a * r.y;
     return std::fma(std::fma(-r.b, q, a), r.y, q);
+}
+
+// whether quot() holds for dividend a by a divisor of 1e-100 to 1e100: a has an exponent of 2^-600 to 2^600,
+// so that quotient and remainder are normal numbers (it is not zero, subnormal, near overflow or non-finite)
+SPHFEM_HD bool quot_holds(double a) {
+    unsigned long long bits;
+    __builtin_memcpy(&bits, &a, 8);
+    return ((unsigned)(bits >> 52) & 0x7ff) - (1023u - 600u) <= 1200u;
 }
 
 // square root of x and the half reciprocal root the iteration carries (h = 1 / (2 sqrt(x)) to 40 bits)

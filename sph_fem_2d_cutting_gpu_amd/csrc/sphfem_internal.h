@@ -28,10 +28,13 @@
 #define SPHFEM_FORM_WIDTH 2
 #define SPHFEM_FORM_AWAY 4
 #define SPHFEM_FLAG_NONFINITE 5
-// densities whose sums, reciprocals and quotients are normal numbers; a live particle outside them
-// switches the FP64 pair sums to the window form and its plain divisions
-#define SPHFEM_RHO_MIN 1e-290
-#define SPHFEM_RHO_MAX 1e290
+// densities whose sums, reciprocals and quotients (quot_holds) are normal numbers; a live particle outside
+// them switches the FP64 pair sums to the window form and its plain divisions
+#define SPHFEM_RHO_MIN 1e-100
+#define SPHFEM_RHO_MAX 1e100
+// velocities whose viscous terms are finite for every pair of a window; a live particle beyond switches to the
+// window form (0 times an infinite term is not zero outside the support either)
+#define SPHFEM_VEL_MAX 1e100
 // records per step of each ordered segment sum (friction heat, contact heat exchange); the
 // reduction sorts them in LDS
 #define SPHFEM_SEG_SINK_CAP 4096

@@ -122,7 +122,7 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
             if constexpr (!WIN) by_rhoij = recip_from(rhoij, __builtin_amdgcn_rcp(rhoij));
             auto over_rhoij = [&](double a) {
                 if constexpr (WIN) return a / rhoij;
-                else return quot(a, by_rhoij);
+                else return quot_holds(a) ? quot(a, by_rhoij) : a / rhoij;
             };
             if (vijposij < 0.) {
                 double cij = 0.5 * (ci + cj);
@@ -1005,8 +1005,8 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
 // interactions_gpu.cu:143-379 for the drop-in entry point, first kernel: the neighbour factors of
 // k_pairs_fp64's pair loop from the arrays as they stand (the same operations the reference repeats
 // per pair), and the switch to the reference's full window: a live particle with a non-finite input
-// or factor, or with a density out of the range of flag_nonfinite (a zero kernel value times such a
-// factor is not zero).
+// or factor, or out of the range of pair_inputs_in_range (a zero kernel value times such a factor is not
+// zero).
 __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_particles P, const PreView pre,
                                                    int *__restrict__ window, int *__restrict__ next_window) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1027,7 +1027,7 @@ __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_par
     pre.r2[i] = {R.z, T};
     const double s = ((pos.x + pos.y) + (vel.x + vel.y)) + ((T + h) + (R.x + R.y)) + (R.z + vol) +
                      ((f.x + f.y) + (f.z + f.w));
-    if (blanked != 1. && !(isfinite(s) && rho > SPHFEM_RHO_MIN && rho < SPHFEM_RHO_MAX)) *window = 1;
+    if (blanked != 1. && !(isfinite(s) && pair_inputs_in_range(rho, vel))) *window = 1;
 }
 
 // second kernel: the pair sums in the reference's arithmetic and neighbour order.  With finite inputs

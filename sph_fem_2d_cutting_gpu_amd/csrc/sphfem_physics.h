@@ -56,6 +56,11 @@ __device__ __forceinline__ bool cubic_spline(double pix, double piy, double pjx,
     return true;
 }
 
+// density and velocity of a live particle that the in-support pair sums take (see SPHFEM_RHO_MIN, SPHFEM_VEL_MAX)
+__device__ __forceinline__ bool pair_inputs_in_range(double rho, sphfem_double2 vel) {
+    return rho > SPHFEM_RHO_MIN && rho < SPHFEM_RHO_MAX && fabs(vel.x) < SPHFEM_VEL_MAX && fabs(vel.y) < SPHFEM_VEL_MAX;
+}
+
 // The distance terms of one in-support pair: the kernel's value and gradient (cubic_spline above, the
 // same operations and roundings) and, for the heat term, the distance and 1 / distance and the unit
 // vector (interactions_gpu.cu:340-352), the quotients by shared reciprocals (sphfem_fpmath.h)

@@ -1013,15 +1013,14 @@ void launch_rothlin_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p) {
 // a live particle with a non-finite pair input (interactions_gpu.cu:143-379 reads pos, vel, h, rho, p,
 // S, R and T of both particles): the pair kernels then evaluate the reference's full 5x5-cell window,
 // where such a neighbour turns the sums NaN even outside the kernel support.  A finite sum that
-// overflows, or a density outside [SPHFEM_RHO_MIN, SPHFEM_RHO_MAX], only sends the step down that
-// (exact, slower) path.
+// overflows, or a density or velocity out of the range of pair_inputs_in_range, only sends the step down
+// that (exact, slower) path.
 __device__ __forceinline__ void flag_nonfinite(int *__restrict__ form, double blanked, sphfem_double2 pos,
                                                sphfem_double2 vel, sphfem_double4 S, double rho, double T, double h,
                                                double pr, sphfem_double4 R) {
     const double s = ((pos.x + pos.y) + (vel.x + vel.y)) + ((S.x + S.y) + (S.z + rho)) + ((T + h) + (pr + R.x)) +
                      (R.y + R.z);
-    if (blanked != 1. && !(isfinite(s) && rho > SPHFEM_RHO_MIN && rho < SPHFEM_RHO_MAX))
-        atomicOr(form, SPHFEM_FORM_WINDOW);
+    if (blanked != 1. && !(isfinite(s) && pair_inputs_in_range(rho, vel))) atomicOr(form, SPHFEM_FORM_WINDOW);
 }
 
 // FP32C neighbour records (RecView) of one sorted particle.  The position is rounded to cell / 2^28 from

@@ -95,3 +95,43 @@ def test_reciprocals_of_double_roots_are_correctly_rounded(tmp_path):
     exe = tmp_path / "r"
     subprocess.run(["g++", "-O2", "-mfma", "-ffp-contract=off", "-std=c++17", str(src), "-o", str(exe)], check=True)
     assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split() == ["0", "1"]
+
+
+RANGE = r"""
+#include <cmath>
+#include <cstdio>
+#include <cstring>
+#include <random>
+#include "%s/sph_fem_2d_cutting_gpu_amd/csrc/sphfem_fpmath.h"
+using namespace sphfem;
+int main() {
+    std::mt19937_64 g(6);
+    std::uniform_real_distribution<double> u(-1, 1);
+    long bad = 0, held = 0, n = 4000000;
+    for (long k = 0; k < n; k++) {
+        unsigned long long m = g();                        // every exponent: subnormal, infinite, NaN
+        if (k %% 64 == 0) m &= 1ull << 63;                 // zeros
+        double a;
+        std::memcpy(&a, &m, 8);
+        const double b = std::pow(10., 100 * u(g));
+        if (!quot_holds(a)) continue;
+        held++;
+        bad += quot(a, recip_from(b, 1 / b * (1 + u(g) * std::ldexp(1, -20)))) != a / b;
+    }
+    const double end[] = {0., -0., 5e-324, 1e-308, 1e-200, 1e200, 1.7e308, INFINITY, -INFINITY, NAN};
+    for (double a : end) bad += quot_holds(a);
+    std::printf("%%ld %%d\n", bad, held > n / 2);
+    return 0;
+}
+"""
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="no host compiler")
+def test_dividends_that_the_quotient_is_used_for(tmp_path):
+    """Dividends of any exponent by the densities that the in-support sums take: those that quot_holds lets
+    through are divided correctly, and zeros, subnormal, infinite and NaN ones are not let through."""
+    src = tmp_path / "d.cpp"
+    src.write_text(RANGE % ROOT)
+    exe = tmp_path / "d"
+    subprocess.run(["g++", "-O2", "-mfma", "-ffp-contract=off", "-std=c++17", str(src), "-o", str(exe)], check=True)
+    assert subprocess.run([str(exe)], check=True, capture_output=True, text=True).stdout.split() == ["0", "1"]

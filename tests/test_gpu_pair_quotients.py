@@ -1,5 +1,6 @@
 """The FP64 pair sums' quotients by shared reciprocals against the oracle's plain operators, bit for bit, at
-operands where the reciprocal alone is not enough."""
+operands where the reciprocal alone is not enough: viscous terms that overflow or lie among the subnormal
+numbers (velocities of finite but extreme size)."""
 import ctypes as C
 import dataclasses
 
@@ -56,6 +57,17 @@ def _against_oracle(case, label):
         sim.ctx.call("sphfem_free", q)
     sim.close()
     return o
+
+
+@pytest.mark.parametrize("scale", [1e170, 1e-300, 1e-310, 1e-316])
+def test_viscous_terms_at_the_ends_of_the_range(scale):
+    case = _columns(60)
+    rng = np.random.default_rng(7)
+    o = _against_oracle(dataclasses.replace(case, vel=rng.standard_normal((case.N, 2)) * scale), f"velocities {scale}")
+    if scale > 1:
+        assert np.isinf(o.P["vel_t"]).any()
+    else:
+        assert np.any(o.P["vel_t"] != 0.0)
 
 
 def test_distances_just_below_a_power_of_two():
