@@ -303,7 +303,8 @@ int sphfem_material_fric_heat_gen(sphfem_ctx *ctx, sphfem_particles *p, sphfem_d
  * at zero (tool particles then conduct no heat). */
 int sphfem_interactions_setup_thermal_constants_tool(sphfem_ctx *ctx, const sphfem_trml_constants *c);
 
-/* ---- time integration (leap_frog.h:46-49, leap_frog.cu:25-96, 162-248) */
+/* ---- time integration (leap_frog.h:46-49, leap_frog.cu:25-96, 162-248).  The first FP64 step of a
+ * stepper (or graph of FP64 steps) allocates 200 B per particle that FP32C steps do without. */
 int sphfem_leap_frog_create(sphfem_ctx *ctx, unsigned int num_part, unsigned int num_cell, int node_num,
                             sphfem_leap_frog **out);
 int sphfem_leap_frog_destroy(sphfem_ctx *ctx, sphfem_leap_frog *lf);

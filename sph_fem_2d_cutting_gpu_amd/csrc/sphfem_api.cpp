@@ -1619,8 +1619,6 @@ int sphfem_leap_frog_create(sphfem_ctx *ctx, unsigned int num_part, unsigned int
         lf->S_init = dalloc<sphfem_double4>(num_part);
         lf->rho_init = dalloc<double>(num_part);
         lf->T_init = dalloc<double>(num_part);
-        lf->pre = dalloc<sphfem_double2>(sphfem::pre_double2s(num_part));
-        lf->psum64 = dalloc<sphfem::PairSums>(num_part);
         lf->cell_start = dalloc<int>(std::max(num_cell, 1u));
         lf->cell_end = dalloc<int>(std::max(num_cell, 1u));
         lf->near_list = dalloc<int>(num_part);
@@ -1740,8 +1738,17 @@ static void sync_rate_form(sphfem_ctx *ctx, sphfem_leap_frog *lf, const sphfem_p
     lf->rates_fp32 = f32c;
 }
 
+// the arrays that only FP64 steps use, 200 B per particle, from the first of them on (before a capture: a
+// graph keeps their addresses, so they stay until the stepper goes)
+static void fp64_workspace(sphfem_leap_frog *lf) {
+    if (lf->precision != SPHFEM_FP64) return;
+    if (!lf->pre) lf->pre = dalloc<sphfem_double2>(sphfem::pre_double2s(lf->num_part));
+    if (!lf->psum64) lf->psum64 = dalloc<sphfem::PairSums>(lf->num_part);
+}
+
 static int step_body(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_particles *p, sphfem_grid *g, sphfem_tool *t,
                      sphfem_rigid_tool *rt = nullptr) {
+    fp64_workspace(lf);
     // leap_frog.cu:175 (a no-op for a locked grid)
     if (int rc = update_geometry(ctx, g, *p, 2.)) return rc;
     ctx->c.geom = g->geom;
@@ -1882,6 +1889,7 @@ static int graph_create(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_particles 
         if (!g->locked)
             return fail(ctx, SPHFEM_ERR_STATE, "graphs need a locked grid (the geometry update reads back to the host)");
         if (g->first_sort) return fail(ctx, SPHFEM_ERR_STATE, "run one step before capturing (first sort)");
+        fp64_workspace(lf);
         sync_rate_form(ctx, lf, *p);      // eagerly: the graph records the steady state only
         const bool timing = ctx->timing.enabled;
         ctx->timing.enabled = false;
@@ -1944,7 +1952,10 @@ int sphfem_batch_graph_create(sphfem_ctx *const *ctxs, sphfem_leap_frog *const *
                         "batch graph: every case needs a locked grid and one eager step before capture");
     }
     return guarded(ctx0, [&] {
-        for (int k = 0; k < n; k++) sync_rate_form(ctxs[k], lfs[k], *ps[k]);
+        for (int k = 0; k < n; k++) {
+            fp64_workspace(lfs[k]);
+            sync_rate_form(ctxs[k], lfs[k], *ps[k]);
+        }
         std::vector<bool> timing((size_t)n);
         for (int k = 0; k < n; k++) {
             timing[(size_t)k] = ctxs[k]->timing.enabled;
