@@ -183,6 +183,9 @@ int sphfem_grid_get_cells(sphfem_ctx *ctx, sphfem_grid *g, const sphfem_particle
 
 /* ---- pair interactions (interactions_gpu.cu:381-432, 466-474) */
 int sphfem_interactions_setup_geometry_constants(sphfem_ctx *ctx, const sphfem_grid *g);
+/* interactions_monaghan keeps 96 B per particle of workspace in the context, for the largest particle count
+ * it has been called with; growing it waits for the stream.  sphfem_particles_free of that many particles
+ * gives it back. */
 int sphfem_interactions_monaghan(sphfem_ctx *ctx, sphfem_particles *p, const int *cell_start,
                                  const int *cell_end, int num_cell);
 /* interactions_gpu.cu:466-474 in the FP32-compensated form (the pair sums of

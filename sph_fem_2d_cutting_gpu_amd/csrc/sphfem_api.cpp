@@ -380,6 +380,11 @@ int sphfem_particles_free(sphfem_ctx *ctx, sphfem_particles *p) {
     return guarded(ctx, [&] {
         SPHFEM_HIP_CHECK(hipStreamSynchronize(ctx->stream));
         free_particles(*p);
+        // interactions_monaghan's workspace goes with the particles that it was sized for
+        if (p->N >= ctx->pre_cap) {
+            ctx->pre_cap = 0;
+            dfree(ctx->pre);
+        }
         return SPHFEM_OK;
     });
 }

@@ -60,3 +60,40 @@ def test_forms_switched_between_steps_and_graphs():
         assert_equal(f, got[f], want[f])
     for f in ("pos", "vel", "S", "T"):
         assert np.max(np.abs(got[f] - want[f])) <= 1e-6 * np.max(np.abs(want[f])), f
+
+
+def test_interactions_workspace_goes_with_the_particles():
+    """interactions_monaghan's workspace in the context: given back with the particles that it was sized for,
+    there again for the next ones."""
+    small, large = cases.chip_case(n_target=40_000), cases.chip_case(n_target=2_000_000)
+    keep = S.Simulation(small)
+    ctx = keep.ctx
+
+    def sums(case, p, g):
+        cells = [C.c_void_p(), C.c_void_p()]
+        for q in cells:
+            ctx.call("sphfem_malloc", C.byref(q), 4 * g.num_cell)
+        g.assign_hashes(p)
+        g.sort(p)
+        g.get_cells(p, cells[0].value, cells[1].value)
+        S.interactions_setup_geometry_constants(g)
+        S.material_eos(p)
+        S.corrector_artificial_stress(p)
+        S.interactions_monaghan(p, cells[0].value, cells[1].value, g.num_cell)
+        out = p.download("S_der")
+        for q in cells:
+            ctx.call("sphfem_free", q)
+        return out
+
+    print("workspace of", small.N, "then", large.N, "particles", flush=True)
+    want = sums(small, keep.p, keep.grid)
+    before = _free(ctx)
+    init = cases.initial_particles(large)
+    p = S.particle_gpu(ctx, large.N, **{f: init[f] for f in ("pos", "vel", "rho", "T", "h", "S")})
+    g = S.grid_gpu_green(ctx, large.N, large.grid_bbmin, large.grid_bbmax, large.h)
+    sums(large, p, g)
+    ctx.call("sphfem_grid_destroy", g.h)
+    p.free()
+    assert before - _free(ctx) < 16 * large.N
+    assert_equal("S_der", sums(small, keep.p, keep.grid), want)
+    keep.close()
