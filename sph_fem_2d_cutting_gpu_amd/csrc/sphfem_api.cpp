@@ -1761,7 +1761,7 @@ static int step_body(sphfem_ctx *ctx, sphfem_leap_frog *lf, sphfem_particles *p,
     const bool green = g->kind != SPHFEM_GRID_ROTHLIN;
     if (!green) {
         if (t) launch_tool_begin(ctx, t);
-        else launch_fill_int(ctx, ctx->d_flags + 1, SPHFEM_FLAG_NONFINITE, 0);   // [1] .. [5]
+        else launch_fill_int(ctx, ctx->d_flags + 1, SPHFEM_FLAG_FORM + SPHFEM_FORM_WORDS - 1, 0);   // all but the error
         if (rt) launch_rigid_advance(ctx, rt);
     }
     // the source of each sorted position: the permutation of the sort (Green), or the identity

@@ -20,14 +20,19 @@
 #define SPHFEM_RESORT_SYNC 16
 // blocks of the bounding-box reduction of an unlocked grid
 #define SPHFEM_BBOX_BLOCKS 1024
-// d_flags slot set by the reorder and cleared by the update kernel: the form of the pair sums.  WINDOW: a
-// live particle carries a non-finite pair input, the pair kernels use the reference's full 5x5-cell
-// window.  FP32C only: WIDTH, one has a kernel width other than the cell size; AWAY, one is neither near
-// the cell that it is sorted into nor one column height above or below it
+// The form of the pair sums: SPHFEM_FORM_WORDS words, word k nonzero for bit 2^k, written by the reorder or the
+// stage calls' first kernels with plain stores of 1 (an atomic on one word by every wavefront of a state with
+// narrower kernels took 35 us at 204k particles).  WINDOW: a live particle carries a non-finite pair input, the
+// pair kernels use the reference's full 5x5-cell window.  FP32C only: WIDTH, one has a kernel width other than
+// the cell size; AWAY, one is neither near the cell that it is sorted into nor one column height above or below
+// it; REACH, one has a kernel width above twice the cell size
 #define SPHFEM_FORM_WINDOW 1
 #define SPHFEM_FORM_WIDTH 2
 #define SPHFEM_FORM_AWAY 4
-#define SPHFEM_FLAG_NONFINITE 5
+#define SPHFEM_FORM_REACH 8
+#define SPHFEM_FORM_WORDS 4
+// the step's form words in d_flags, cleared at its start
+#define SPHFEM_FLAG_FORM 10
 // densities whose sums, reciprocals and quotients (quot_holds) are normal numbers; a live particle outside
 // them switches the FP64 pair sums to the window form and its plain divisions
 #define SPHFEM_RHO_MIN 1e-100
@@ -40,15 +45,14 @@
 #define SPHFEM_SEG_SINK_CAP 4096
 #define SPHFEM_FLAG_SINK_FRIC 6
 #define SPHFEM_FLAG_SINK_S2 7
-// interactions_monaghan's own two switches of the same kind, used in turn by its calls: a call's first
-// kernel sets one and clears the other for the next call (each is read by the call's second kernel)
-#define SPHFEM_FLAG_MONAGHAN 8
 // workgroups of the near-tool pass that are done; zero between launches
-#define SPHFEM_FLAG_NEAR_DONE 10
-// interactions_monaghan_fp32c's own two words of the pair sums' form, used in turn like those of
-// interactions_monaghan
-#define SPHFEM_FLAG_MONAGHAN_FP32C 11
-#define SPHFEM_NUM_FLAGS 13
+#define SPHFEM_FLAG_NEAR_DONE 8
+// interactions_monaghan's and interactions_monaghan_fp32c's own two sets of form words each, used in turn by
+// their calls: a call's first kernel sets one and clears the other for the next call (each is read by the
+// call's second kernel)
+#define SPHFEM_FLAG_MONAGHAN (SPHFEM_FLAG_FORM + SPHFEM_FORM_WORDS)
+#define SPHFEM_FLAG_MONAGHAN_FP32C (SPHFEM_FLAG_MONAGHAN + 2 * SPHFEM_FORM_WORDS)
+#define SPHFEM_NUM_FLAGS (SPHFEM_FLAG_MONAGHAN_FP32C + 2 * SPHFEM_FORM_WORDS)
 // position records a wavefront of the staged FP32C pair kernel copies into LDS (8 KiB)
 #define SPHFEM_STAGE_CAP 512
 // blocks of the report_force reduction (its partials: 2 doubles per block) and the largest particle
@@ -118,7 +122,7 @@ inline RateView rate_view(float *base, size_t n) {
 //            4 records); 8 cells aside for blanked particles and outside the grid's rows (write_records)
 //   r1[j] = {vx, vy, (Sxx - p)/rho^2, Sxy/rho^2}     r2[j] = {(Syy - p)/rho^2, Rxx, Rxy, Ryy}
 //   r3[j] = {+-mass/rho, rho, alpha sqrt(K/rho), T - T_init}
-//   h[j]    = kernel width (read where it is not the cell size)
+//   h[j]    = kernel width in the units of pos (read where one is not the cell size)
 //   away[j] = position in the units of pos, unwrapped (written for live particles whose pos lies aside)
 // The volume is stored negative for tool particles, the sound speed of blanked ones is -inf.
 #define SPHFEM_POS_BITS 28
@@ -184,7 +188,7 @@ struct sphfem_ctx {
     std::string err;
     int *d_flags = nullptr;       // [0]: error bits, [1]: near-list count, [2]: unused,
                                   // [3]: re-sort mode (1 full, 2 incremental), [4]: changed count,
-                                  // [5]: non-finite pair inputs present (SPHFEM_FLAG_NONFINITE)
+                                  // then the SPHFEM_FLAG_ slots
     double *force_scratch = nullptr;  // this device's `scratch` array (sphfem_api.cpp)
     // interactions_monaghan: the neighbour fields of k_pre_state for the largest particle count seen
     // (pre_view, pre_cap particles) and which of its two switches the next call uses
@@ -461,7 +465,7 @@ void launch_tool_begin(sphfem_ctx *ctx, sphfem_tool *t);
 // the step's counters: the near list's length and the window-form switch of the pair kernels
 __device__ __forceinline__ void step_counters_clear(int *counters) {
     counters[1] = 0;
-    counters[SPHFEM_FLAG_NONFINITE] = 0;
+    for (int k = 0; k < SPHFEM_FORM_WORDS; k++) counters[SPHFEM_FLAG_FORM + k] = 0;
 }
 
 // the start of a step for the FEM tool, item i of max(nodes, segments): reset_FEM_server's T_old = T and

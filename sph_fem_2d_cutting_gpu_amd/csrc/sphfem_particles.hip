@@ -260,9 +260,8 @@ struct PairAcc {                // FP32 block sums
 
 constexpr float KU = 1.f / (float)(1 << SPHFEM_POS_BITS);      // ku where the kernel width is the cell size
 
-// one pair at distance D.  GEN: any kernel widths (h_j / u in Hj), and (win) window candidates outside the
-// support with the kernel set to 0 as in the reference; otherwise h_i = h_j = the cell size and every
-// entry lies in the support
+// one pair at distance D.  GEN: any kernel widths (h_j / u in Hj), else h_i = h_j = the cell size; win: window
+// candidates outside the support are among the entries, with the kernel set to 0 as in the reference
 template <bool GEN>
 __device__ __forceinline__ void pair_term(const PairI &I, float dx, float dy, const float4 q1, const float4 q2,
                                           const float4 q3, float Hj, bool win, PairAcc &a) {
@@ -285,11 +284,8 @@ __device__ __forceinline__ void pair_term(const PairI &I, float dx, float dy, co
     }
     const float volj = fabsf(q3.x);
     const float heat = volj * (I.Ti - q3.w) * g;
-    if constexpr (GEN) {
-        if (I.thermal && D2 > I.D2heat) a.T += heat;
-    } else {
-        a.T += heat;                                     // used only where the thermal block is set
-    }
+    // used only where the thermal block is set
+    a.T += GEN && !(D2 > I.D2heat) ? 0.f : heat;
     if (I.mech && q3.x > 0.f) {                          // neither i nor j is a tool particle
         const float wx = g * dx, wy = g * dy;
         const float dvx = q1.x - I.vxi, dvy = q1.y - I.vyi;
@@ -307,13 +303,11 @@ __device__ __forceinline__ void pair_term(const PairI &I, float dx, float dy, co
         const float half_inv_rhoij = __builtin_amdgcn_rcpf(I.rhoi + q3.y);
         const float vp = -(dvx * dx + dvy * dy);         // (v_i - v_j) . D
         if constexpr (GEN) {
-            if (vp < 0.f) {
-                const float H = 0.5f * (I.H + Hj);
-                const float mu = H * vp * __builtin_amdgcn_rcpf(D2 + I.eta2 * H * H);
-                const float piij = mu * (I.beta2 * mu - (I.ci + q3.z)) * half_inv_rhoij;
-                Ax -= piij;
-                Az -= piij;
-            }
+            const float H = 0.5f * (I.H + Hj);
+            const float mu = H * vp * __builtin_amdgcn_rcpf(D2 + I.eta2 * H * H);
+            const float piij = vp < 0.f ? mu * (I.beta2 * mu - (I.ci + q3.z)) * half_inv_rhoij : 0.f;
+            Ax -= piij;
+            Az -= piij;
         } else {
             // receding pairs take mu = 0 and with it no viscous term
             const float mu = fminf(vp, 0.f) * __builtin_amdgcn_rcpf(D2 * KU + I.eta2);
@@ -368,10 +362,13 @@ __device__ __forceinline__ double2 wide_pos(const RecView &rv, int ny, int j, in
 // (cell-relative FP32 and the cell row, with the column in the list entry) and kernel factors applied
 // per pair took 868 us (with the update) on 4 M particles and 3337 us (sums alone) on 16 M, against 779
 // and 2827 us.
-// General form (form != 0; the SPHFEM_FORM_ bits): kernel widths other than the cell size; positions that
-// the wrapped ones cannot tell apart, taken in FP64; and the window form, where every non-blanked record
-// of the 5x5 cells is evaluated with the kernel set to 0 outside the support, as the reference does (see
-// pair_sums_fp64).
+// General form (GEN; the SPHFEM_FORM_ bits): kernel widths other than the cell size, at a fifth load per pair and
+// the factors of h_i; and (SPECIAL), with a test of every candidate's record, widths that reach the place of
+// blanked records, positions that the wrapped ones cannot tell apart, taken in FP64, and the window form, where
+// every non-blanked record of the 5x5 cells is evaluated with the kernel set to 0 outside the support, as the
+// reference does (see pair_sums_fp64).  With a third of the widths at 0.9 of the cell size the stage call takes
+// 165 us at 204k and 580 us at 2M particles, a 1M-particle step 296 us; 178, 663 and 322 us with the 16-byte
+// records, 302, 897 and 390 us while every state other than the first form's took the whole of the tests.
 __device__ __forceinline__ double interaction_alpha(const DevConsts &c, double is_tool) {
     // interactions_gpu.cu:164: the tool block (interactions_gpu.cu:19) is zero unless
     // interactions_setup_thermal_constants_tool set it (the rigid-tool setup does, benchmarks.cpp:518;
@@ -667,14 +664,14 @@ struct PairOut {           // one particle's FP32C sums: psum[i], psum[N + i], p
     float T;
 };
 
-template <int BS, int CHUNK, bool GEN, bool ROLL, class Pos = GlobalPos>
+template <int BS, int CHUNK, bool GEN, bool SPECIAL, bool ROLL, class Pos = GlobalPos>
 __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int *__restrict__ hash, int N,
                                                    const RecView &rv,
                                                    const int *__restrict__ cs, const int *__restrict__ ce, int i,
                                                    typename Pos::Entry *__restrict__ list, const Pos &pos,
                                                    int *__restrict__ flags, int form) {
 #pragma clang fp contract(fast)
-    const bool win = GEN && (form & SPHFEM_FORM_WINDOW), wide = GEN && (form & ~SPHFEM_FORM_WIDTH);
+    const bool win = SPECIAL && (form & SPHFEM_FORM_WINDOW), wide = SPECIAL && (form & ~SPHFEM_FORM_WIDTH);
     double d_v0 = 0., d_v1 = 0., d_v2 = 0., d_v3 = 0.;
     double d_ax = 0., d_ay = 0., d_p0 = 0., d_p1 = 0., d_T = 0.;
     const float4 a3 = rv.r3[i];
@@ -684,7 +681,7 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
     const bool tool_i = a3.x < 0.f;
     const double alpha_i = tool_i ? c.trml_itool.alpha : c.trml_wp.alpha;
     const double dxc = c.geom.dx;
-    const double hi = GEN ? (double)rv.h[i] : dxc;
+    const double hi = GEN ? (double)rv.h[i] * (dxc / (double)(1 << SPHFEM_POS_BITS)) : dxc;
     // nor does one whose key names no cell (the records' kernel reported it): its window's entries are read
     // before their columns are known to exist
     const int nx = c.geom.nx, ny = c.geom.ny;
@@ -720,7 +717,7 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
         I.D2min = (float)(c.rr2_min * inv_u * inv_u);
         I.beta2 = (float)(2. * c.corr.beta);
         if constexpr (GEN) {
-            I.H = (float)(hi * inv_u);
+            I.H = rv.h[i];
             I.ku = 1.f / I.H;
             I.D2max = 4.f * I.H * I.H;
             I.D2heat = (float)(1e-16 * inv_u * inv_u);
@@ -741,7 +738,7 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
             a = PairAcc{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         };
         auto distance = [&](unsigned j, int2 p, float &dx, float &dy) {
-            if (GEN && wide) {
+            if (SPECIAL && wide) {
                 const double2 x = wide_pos(rv, ny, (int)j, hash[j]);
                 dx = (float)(I.xd - x.x);
                 dy = (float)(I.yd - x.y);
@@ -751,11 +748,14 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
             }
         };
         auto term = [&](typename Pos::Entry e, const int2 q0, const float4 q1, const float4 q2, const float4 q3,
-                        PairAcc &acc) {
-            float dx, dy, Hj = 0.f;
+                        float Hj, PairAcc &acc) {
+            float dx, dy;
             distance(pos.index(e), q0, dx, dy);
-            if constexpr (GEN) Hj = (float)((double)rv.h[pos.index(e)] * inv_u);
             pair_term<GEN>(I, dx, dy, q1, q2, q3, Hj, win, acc);
+        };
+        auto width = [&](unsigned byte_off) {      // of the record at this offset of a block of 16-byte ones
+            if constexpr (!GEN) return 0.f;
+            else return *reinterpret_cast<const float *>(reinterpret_cast<const char *>(rv.h) + (byte_off >> 2));
         };
         // dense list of the entries in front of list[end]: two per iteration, the records of the next
         // entry loaded before the current one is evaluated (ping-pong registers, no copies); each list
@@ -771,19 +771,22 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
             unsigned oA = pos.index(eA) << 4;
             int2 A0 = pos.entry(eA);
             float4 A1 = ldrec(rv.r1, oA), A2 = ldrec(rv.r2, oA), A3 = ldrec(rv.r3, oA);
+            float Ah = width(oA);
             for (int k = 0; k < end; k += 2 * BS) {
                 const typename Pos::Entry eA_next = list[k + 2 * BS];
                 const unsigned oB = pos.index(eB) << 4;
                 const int2 B0 = pos.entry(eB);
                 const float4 B1 = ldrec(rv.r1, oB), B2 = ldrec(rv.r2, oB), B3 = ldrec(rv.r3, oB);
-                term(eA, A0, A1, A2, A3, acc);
+                const float Bh = width(oB);
+                term(eA, A0, A1, A2, A3, Ah, acc);
                 if (k + BS < end) {
                     const typename Pos::Entry eB_next = list[k + 3 * BS];
                     eA = eA_next;
                     oA = pos.index(eA) << 4;
                     A0 = pos.entry(eA);
                     A1 = ldrec(rv.r1, oA); A2 = ldrec(rv.r2, oA); A3 = ldrec(rv.r3, oA);
-                    term(eB, B0, B1, B2, B3, acc);
+                    Ah = width(oA);
+                    term(eB, B0, B1, B2, B3, Bh, acc);
                     eB = eB_next;
                 }
                 if (((k + 2 * BS) & (8 * BS - 1)) == 0) flush(acc);
@@ -811,7 +814,7 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
                 pos.scan4(d, j, b);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    if (GEN && (j + u >= last || rv.r3[j + u].z == -INFINITY)) continue;
+                    if (SPECIAL && wide && (j + u >= last || rv.r3[j + u].z == -INFINITY)) continue;
                     float dx, dy;
                     distance((unsigned)(j + u), b[u], dx, dy);
                     const float D2 = dx * dx + dy * dy;
@@ -872,27 +875,41 @@ __device__ __forceinline__ void emit_pairs(const DevConsts &c, const UpdateArgs 
     }
 }
 
-// in-support pair sums, one lane per sorted particle, in the form that nonfinite[0] asks for.  TO: what
+// in-support pair sums, one lane per sorted particle, in the form that the form words ask for.  TO: what
 // each lane does with its particle's sums (emit_pairs).
-__device__ __forceinline__ int pairs_form(const DevConsts &c, const int *__restrict__ nonfinite) {
+__device__ __forceinline__ int pairs_form(const DevConsts &c, const int *__restrict__ form) {
     // a support that reaches below the heat term's least distance needs the test of the general form
-    return *nonfinite | (c.rr2_min > 1e-16 ? 0 : SPHFEM_FORM_WIDTH);
+    int f = c.rr2_min > 1e-16 ? 0 : SPHFEM_FORM_WIDTH;
+    for (int k = 0; k < SPHFEM_FORM_WORDS; k++) f |= form[k] != 0 ? 1 << k : 0;
+    return f;
+}
+
+// the list kernel's sums of particle i, in the given form.  Fused with the update there are two forms in the
+// kernel, the tests switched by uniform branches: a third one takes it from 166 to 168 registers and costs the
+// first form 3 % (1 M particles: 260 -> 269 us a step)
+template <int BS, int CHUNK, int TO>
+__device__ __forceinline__ PairOut pairs_fp32c_list(const DevConsts &c, const int *__restrict__ hash, int N,
+                                                    const RecView &rv, const int *__restrict__ cs,
+                                                    const int *__restrict__ ce, int i, int *__restrict__ list,
+                                                    int form) {
+    const GlobalPos pos{rv.pos};
+    if (form == 0)
+        return pairs_fp32c_one<BS, CHUNK, false, false, TO != TO_UPDATE>(c, hash, N, rv, cs, ce, i, list, pos, nullptr, 0);
+    if (TO != TO_UPDATE && form == SPHFEM_FORM_WIDTH)
+        return pairs_fp32c_one<BS, CHUNK, true, false, true>(c, hash, N, rv, cs, ce, i, list, pos, nullptr, form);
+    return pairs_fp32c_one<BS, CHUNK, true, true, true>(c, hash, N, rv, cs, ce, i, list, pos, nullptr, form);
 }
 
 template <int BS, int CHUNK, int TO = TO_PSUM, bool RIGID = false>
 __global__ void __launch_bounds__(BS) k_pairs_fp32c(DevConsts c, const int *__restrict__ hash, int N, RecView rv,
                                                          const int *__restrict__ cs, const int *__restrict__ ce,
                                                          float4 *__restrict__ psum, float *__restrict__ psum_T,
-                                                         const int *__restrict__ nonfinite, UpdateArgs u) {
+                                                         const int *__restrict__ form_words, UpdateArgs u) {
     __shared__ int nb_list[(CHUNK + 2) * BS];
-    const int form = pairs_form(c, nonfinite);
+    const int form = pairs_form(c, form_words);
     const int i = xcd_logical_block() * BS + threadIdx.x;
     if (i >= N) return;
-    const PairOut o =
-        form != 0 ? pairs_fp32c_one<BS, CHUNK, true, true>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
-                                                     GlobalPos{rv.pos}, nullptr, form)
-                  : pairs_fp32c_one<BS, CHUNK, false, TO != TO_UPDATE>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x,
-                                                      GlobalPos{rv.pos}, nullptr, 0);
+    const PairOut o = pairs_fp32c_list<BS, CHUNK, TO>(c, hash, N, rv, cs, ce, i, nb_list + threadIdx.x, form);
     emit_pairs<TO, RIGID>(c, u, psum, psum_T, N, i, o);
 }
 
@@ -912,7 +929,7 @@ template <int CHUNK, int CAP, int TO = TO_PSUM, bool RIGID = false>
 __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const int *__restrict__ hash, int N, RecView rv,
                                                            const int *__restrict__ cs, const int *__restrict__ ce,
                                                            float4 *__restrict__ psum, float *__restrict__ psum_T,
-                                                           const int *__restrict__ nonfinite, int *__restrict__ flags,
+                                                           const int *__restrict__ form_words, int *__restrict__ flags,
                                                            UpdateArgs u) {
     // LDS: staged -- positions [CAP + 4] (+4: the scan reads up to three records past a range) and
     // 16-bit list entries; list path -- 32-bit list entries in the same bytes
@@ -923,7 +940,7 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
     int2 *spos = reinterpret_cast<int2 *>(lds);
     unsigned short *list16 = reinterpret_cast<unsigned short *>(lds + POS_BYTES);
     int *list32 = reinterpret_cast<int *>(lds);
-    const int form = pairs_form(c, nonfinite);
+    const int form = pairs_form(c, form_words);
     const int base = xcd_logical_block() * 64;
     if (base >= N) return;                              // the whole wavefront
     const int lane = (int)threadIdx.x;
@@ -992,13 +1009,10 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
     if (i >= N) return;
     PairOut o;
     if (staged)
-        o = pairs_fp32c_one<64, CHUNK, false, false, StagedPos>(c, hash, N, rv, cs, ce, i, list16 + lane, sp, flags, 0);
-    else if (form == 0)
-        o = pairs_fp32c_one<64, CHUNK, false, TO != TO_UPDATE>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
-                                              nullptr, 0);
+        o = pairs_fp32c_one<64, CHUNK, false, false, false, StagedPos>(c, hash, N, rv, cs, ce, i, list16 + lane, sp, flags,
+                                                                       0);
     else
-        o = pairs_fp32c_one<64, CHUNK, true, true>(c, hash, N, rv, cs, ce, i, list32 + lane, GlobalPos{rv.pos},
-                                             nullptr, form);
+        o = pairs_fp32c_list<64, CHUNK, TO>(c, hash, N, rv, cs, ce, i, list32 + lane, form);
     emit_pairs<TO, RIGID>(c, u, psum, psum_T, N, i, o);
 }
 
@@ -1010,7 +1024,7 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
 __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_particles P, const PreView pre,
                                                    int *__restrict__ window, int *__restrict__ next_window) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i == 0) *next_window = 0;
+    if (i == 0) *next_window = 0;         // the first form word; this call knows no others
     if (i >= (int)P.N) return;
     const double rho = P.rho[i], pr = P.p[i];
     const sphfem_double4 S = P.S[i], R = P.R[i];
@@ -1107,9 +1121,9 @@ void launch_interactions_pse(sphfem_ctx *ctx, const sphfem_particles &p, const i
 }
 
 void launch_interactions_ref(sphfem_ctx *ctx, const sphfem_particles &p, const int *cs, const int *ce) {
-    int *window = ctx->d_flags + SPHFEM_FLAG_MONAGHAN + ctx->monaghan_turn;
+    int *window = ctx->d_flags + SPHFEM_FLAG_MONAGHAN + ctx->monaghan_turn * SPHFEM_FORM_WORDS;
     ctx->monaghan_turn ^= 1;
-    int *next_window = ctx->d_flags + SPHFEM_FLAG_MONAGHAN + ctx->monaghan_turn;
+    int *next_window = ctx->d_flags + SPHFEM_FLAG_MONAGHAN + ctx->monaghan_turn * SPHFEM_FORM_WORDS;
     {
         KTimer t(ctx, "interactions_pre");
         k_pre_state<<<nblk(p.N, 256), 256, 0, ctx->stream>>>(ctx->c, p, pre_view(ctx->pre, p.N), window, next_window);
@@ -1267,7 +1281,7 @@ __global__ void __launch_bounds__(BS) k_pairs_fp64(DevConsts c, sphfem_particles
     if (i >= N || B.blanked[i] == 1.) return;
     const double thermal_alpha = interaction_alpha(c, B.tool_particle[i]);
     // the window form when a live particle carries a non-finite input (see pair_sums_fp64)
-    if ((*nonfinite & SPHFEM_FORM_WINDOW) != 0)
+    if (*nonfinite != 0)
         psum64[i] = pair_sums_fp64<BS, CHUNK, true>(c, B, i, thermal_alpha, cs, ce, pre,
                                                           nb_list + threadIdx.x);
     else
@@ -1334,7 +1348,7 @@ static void launch_pairs_fp32c_shape(sphfem_ctx *ctx, const sphfem_particles &B,
 // arguments (the rigid-tool update when fuse->rt is set)
 static void launch_pairs_fp32c_tuned(sphfem_ctx *ctx, const sphfem_particles &B, sphfem_leap_frog *lf, const int *cs,
                                      const int *ce, const UpdateArgs *fuse = nullptr) {
-    const int *form = ctx->d_flags + SPHFEM_FLAG_NONFINITE;
+    const int *form = ctx->d_flags + SPHFEM_FLAG_FORM;
     if (fuse) {
         KTimer tm(ctx, "pairs_update_fp32c");
         if (fuse->rt) launch_pairs_fp32c_shape<TO_UPDATE, true>(ctx, B, lf, cs, ce, form, *fuse);
@@ -1349,9 +1363,9 @@ static void launch_pairs_fp32c_tuned(sphfem_ctx *ctx, const sphfem_particles &B,
 // 442 us for a second kernel that read them back and spread them into the outputs.
 void launch_interactions_fp32c(sphfem_ctx *ctx, const sphfem_particles &p, sphfem_leap_frog *lf, const int *cs,
                                const int *ce, int num_cell) {
-    int *form = ctx->d_flags + SPHFEM_FLAG_MONAGHAN_FP32C + ctx->fp32c_turn;
+    int *form = ctx->d_flags + SPHFEM_FLAG_MONAGHAN_FP32C + ctx->fp32c_turn * SPHFEM_FORM_WORDS;
     ctx->fp32c_turn ^= 1;
-    int *next_form = ctx->d_flags + SPHFEM_FLAG_MONAGHAN_FP32C + ctx->fp32c_turn;
+    int *next_form = ctx->d_flags + SPHFEM_FLAG_MONAGHAN_FP32C + ctx->fp32c_turn * SPHFEM_FORM_WORDS;
     launch_records_state(ctx, p, num_cell, rec_view(lf->rec, p.N), form, next_form);
     KTimer tm(ctx, "pairs_fp32c");
     UpdateArgs u{};
@@ -1392,7 +1406,7 @@ void launch_fused_update(sphfem_ctx *ctx, const sphfem_particles &B, const sphfe
     u.rt = rtd;
     u.r_old = r_old;
     u.r_new = r_new;
-    int *nf = ctx->d_flags + SPHFEM_FLAG_NONFINITE;
+    int *nf = ctx->d_flags + SPHFEM_FLAG_FORM;      // the WINDOW word
     if (lf->precision == SPHFEM_FP32C) {
         u.skip_contact = skip;
         // the fused pair kernels run the update themselves

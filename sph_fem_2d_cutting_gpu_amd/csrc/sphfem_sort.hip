@@ -1020,7 +1020,7 @@ __device__ __forceinline__ void flag_nonfinite(int *__restrict__ form, double bl
                                                double pr, sphfem_double4 R) {
     const double s = ((pos.x + pos.y) + (vel.x + vel.y)) + ((S.x + S.y) + (S.z + rho)) + ((T + h) + (pr + R.x)) +
                      (R.y + R.z);
-    if (blanked != 1. && !(isfinite(s) && pair_inputs_in_range(rho, vel))) atomicOr(form, SPHFEM_FORM_WINDOW);
+    if (blanked != 1. && !(isfinite(s) && pair_inputs_in_range(rho, vel))) form[0] = 1;      // WINDOW
 }
 
 // FP32C neighbour records (RecView) of one sorted particle.  The position is rounded to cell / 2^28 from
@@ -1028,7 +1028,7 @@ __device__ __forceinline__ void flag_nonfinite(int *__restrict__ form, double bl
 // factors of the pair sum, (S - p)/rho^2 and S_xy/rho^2; the temperature is stored as T - T_init, so
 // that the FP32 differences T_i - T_j of a nearly uniform field keep ~1e-7 of the deviation instead of
 // ~1e-7 of T.
-__device__ __forceinline__ void write_records(const DevConsts &c, const RecView &rec, double inv_dx, int *__restrict__ form_word, int i, int h,
+__device__ __forceinline__ void write_records(const DevConsts &c, const RecView &rec, double inv_dx, int *__restrict__ form, int i, int h,
                                              sphfem_double2 pos, sphfem_double2 vel, sphfem_double4 S, double rho, double T, double blanked,
                                              double tool, double hh, double pr, sphfem_double4 R) {
     const int ny = c.geom.ny;
@@ -1061,12 +1061,13 @@ __device__ __forceinline__ void write_records(const DevConsts &c, const RecView 
         uy += (unsigned)(int)rint(cy * unit);
     }
     const int2 r0 = make_int2((int)ux, (int)uy);
-    // the form of the pair sums: one flag write per wavefront, and none for bits that are seen set
-    const int form = (__any(live && !near) ? SPHFEM_FORM_AWAY : 0) |
-                     (__any(live && hh != c.geom.dx) ? SPHFEM_FORM_WIDTH : 0);
-    if (form != 0 && (int)__lane_id() == __ffsll((long long)__ballot(1)) - 1 &&
-        (form & ~*form_word) != 0)
-        atomicOr(form_word, form);
+    // the form of the pair sums: one store per wavefront and bit
+    const int bits = (__any(live && hh != c.geom.dx) ? SPHFEM_FORM_WIDTH : 0) |
+                     (__any(live && !near) ? SPHFEM_FORM_AWAY : 0) |
+                     (__any(live && hh > 2. * c.geom.dx) ? SPHFEM_FORM_REACH : 0);
+    if (bits != 0 && (int)__lane_id() == __ffsll((long long)__ballot(1)) - 1)
+        for (int k = 1; k < SPHFEM_FORM_WORDS; k++)
+            if (bits >> k & 1) form[k] = 1;
     const double inv_rho = 1. / rho, rho21 = inv_rho * inv_rho;
     const float vol = (float)(c.phys.mass * inv_rho);
     float4 r1, r2, r3;
@@ -1086,7 +1087,7 @@ __device__ __forceinline__ void write_records(const DevConsts &c, const RecView 
     rec.r1[i] = r1;
     rec.r2[i] = r2;
     rec.r3[i] = r3;
-    rec.h[i] = (float)hh;
+    rec.h[i] = (float)(hh * inv_dx * unit);
 }
 
 // FP32C records of an already sorted state as it stands (no predictor): the inputs of
@@ -1098,7 +1099,7 @@ __global__ void __launch_bounds__(256) k_records_state(DevConsts c, const sphfem
                                                        int *__restrict__ next_form) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
-    if (i == 0) *next_form = 0;
+    if (i < SPHFEM_FORM_WORDS) next_form[i] = 0;
     if (i >= N) return;
     int h = p.hash[i];
     if ((unsigned)h >= (unsigned)num_cell) {
@@ -1164,7 +1165,7 @@ __global__ void __launch_bounds__(256) k_reorder_predict(DevConsts c, const sphf
                                                          const PreView pre, ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
-    int *form = flags + SPHFEM_FLAG_NONFINITE;
+    int *form = flags + SPHFEM_FLAG_FORM;
     int h, s;
     if (!cell_bounds(p, rs, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
     sphfem_double2 pos = p.pos[s], vel = p.vel[s];
@@ -1247,7 +1248,7 @@ __global__ void __launch_bounds__(256) k_reorder_records(DevConsts c, const sphf
                                                          ResortView rs) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     const int N = (int)p.N;
-    int *form = flags + SPHFEM_FLAG_NONFINITE;
+    int *form = flags + SPHFEM_FLAG_FORM;
     int h, s;
     if (!cell_bounds(p, rs, i, N, num_cell, cell_start, cell_end, flags, h, s)) return;
     sphfem_double2 pos = ld_stream(&p.pos[s]), vel = ld_stream(&p.vel[s]);

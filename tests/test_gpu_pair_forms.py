@@ -1,7 +1,7 @@
 """FP32C pair sums where the fast form's assumptions fail, against the FP64 pair sums of the same state:
 particles above and below the grid's rows (their keys name cells of the next or previous column: they
 meet only each other), two column heights away, on the grid's edge and clustered near coincidence; kernel
-widths other than the cell size (smaller, and wide enough to reach the blanked records' place); a support
+widths other than the cell size (smaller, larger, and wide enough to reach the blanked records' place); a support
 that starts at 0; grids of few rows.  One step's derivatives agree within 1e-5 of each field's largest
 magnitude, the bound of the ordinary form: the general form does the same FP32 terms in the same blocks."""
 import ctypes as C
@@ -38,13 +38,16 @@ def _moved(kind, P, geom):
     elif kind == "wide":
         h[::5] *= 1.9
         blanked[1::7] = 1.0
+    elif kind == "reach":
+        h[::5] *= 2.6
+        blanked[1::7] = 1.0
     elif kind == "close":
         pos[1:-1:9] = pos[:-2:9] + 9e-5 * np.array([1.0, -1.0])
     return {"pos": pos, "h": h, "blanked": blanked}
 
 
 @pytest.mark.parametrize("nx,ny", [(48, 16), (96, 7)])
-@pytest.mark.parametrize("kind", ["above", "below", "two_heights", "edge", "narrow", "wide", "close", "cutoff"])
+@pytest.mark.parametrize("kind", ["above", "below", "two_heights", "edge", "narrow", "wide", "reach", "close", "cutoff"])
 def test_pair_forms(kind, nx, ny):
     case = cases.perturbed(cases.small_cutting_case(nx=nx, ny=ny))
     out = []
