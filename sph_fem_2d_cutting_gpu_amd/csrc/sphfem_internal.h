@@ -15,7 +15,7 @@
 // largest N for which the tuning resort_one_block is accepted
 #define SPHFEM_SORT_ONE_BLOCK_MAX (1 << 19)
 // largest N for which a step known to sort in full does so inside the re-sort's one launch
-#define SPHFEM_SORT_ONE_LAUNCH_MAX (1 << 18)
+#define SPHFEM_SORT_ONE_LAUNCH_MAX (1 << 19)
 // counters of the re-sort (sphfem_grid::sync)
 #define SPHFEM_RESORT_SYNC 16
 // blocks of the bounding-box reduction of an unlocked grid
@@ -406,11 +406,10 @@ template <bool NT, class T> __device__ __forceinline__ void st_maybe_stream(T *p
     else *p = v;
 }
 
-// Workgroup barrier before one lane announces the workgroup's results to other workgroups (an agent fence,
-// then a counter).  A barrier does not wait for the global stores that other wavefronts have in flight and
-// the lane's fence waits for its own wavefront's only, so every wavefront waits for its stores here; the
-// lane's fence then writes the L2 back once (a fence by every wavefront does so sixteen times: 131k-particle
-// impact 507 us against 294).
+// Workgroup barrier before one lane announces the workgroup's results to other workgroups by a counter.  A
+// barrier does not wait for the global stores that other wavefronts have in flight, and a fence by the lane
+// waits for its own wavefront's only, so every wavefront waits for its stores here.  Plain stores then need
+// the lane's agent fence, which writes the L2 back; written-through ones (agent scope) do not.
 __device__ __forceinline__ void stores_done_barrier() {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();

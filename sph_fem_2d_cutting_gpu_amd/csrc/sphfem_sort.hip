@@ -250,7 +250,8 @@ void launch_radix_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, int
 // key or index array is written and read back in between.  The full sort runs on the first step and
 // whenever more than `cap` particles changed cells: k_resort's workgroups run it in that one launch.
 // Where the host knows of it before (force) and N is above SPHFEM_SORT_ONE_LAUNCH_MAX it is the
-// multi-block radix sort, whose launches beat the queue's waits there.  (Per step with the incremental
+// multi-block radix sort, whose launches beat the queue's waits there (steps of 131k, 400k, 550k, 750k and 1M
+// particles 199, 303, 366, 443 and 549 us by the queue; 314, 362, 428 and 511 us by launches from 400k on).  (Per step with the incremental
 // path before: the hash pass, scan, three idle launches per radix pass, compaction, ranking and
 // scatter, each a dependent launch of about 4.5 us.)
 // Sorted keys and permutation end in (g->keys_alt, p.idx); the caller swaps keys_alt and p.hash.
@@ -266,9 +267,9 @@ constexpr int HASH_BS = 1024;                       // 16 wavefronts per tile, 4
 constexpr int HASH_ITEMS = SORT_TILE / HASH_BS;
 // slots of sphfem_grid::sync: changed particles of this step, then the work queue of k_resort
 enum { RS_COUNT = 0, RS_TICKET = 1, RS_DONE = 2 };   // RS_DONE + phase: finished items of a phase
-constexpr int RS_USED = RS_DONE + 3 * 4;             // at most four passes of three phases
+constexpr int RS_USED = RS_DONE + 2 * 4;             // at most four passes of two phases
 static_assert(RS_USED <= SPHFEM_RESORT_SYNC, "counters");
-constexpr int RS_SCAN_TILES = 64;                    // above, a phase of its own scans the tiles' counts
+constexpr int RS_ITEMS = 256;                        // work items of a phase at most, of whole tiles
 
 struct StepStart {            // what else begins with the step (see k_hash_mark)
     sphfem_tool tool;
@@ -378,6 +379,19 @@ __device__ __forceinline__ int insert_position(const int *__restrict__ old_keys,
     return lo;
 }
 
+__device__ __forceinline__ int wave_inclusive(int v) {
+    for (int o = 1; o < WAVE; o <<= 1) {
+        const int u = __shfl_up(v, o);
+        if ((int)__lane_id() >= o) v += u;
+    }
+    return v;
+}
+
+// a store that other workgroups of the same launch read: written through to where every XCD sees it
+__device__ __forceinline__ void st_agent(int *p, int v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
 // waits until `want` items of a phase are done; false (with the error bit set) if that never comes,
 // which a queue in order cannot do: an item only waits for items taken before it, by running workgroups
 __device__ __forceinline__ bool wait_done(int *counter, int want, int *flags) {
@@ -391,13 +405,18 @@ __device__ __forceinline__ bool wait_done(int *counter, int want, int *flags) {
 
 // The ranking of the changed particles by the first workgroup, or (more than cap of them, or force) the
 // full stable LSD radix sort by all of them.  The sort is a queue of items handed out in order by one
-// counter: per pass the tiles' digit counts, above RS_SCAN_TILES tiles the digits' scans over the tiles,
-// then the tiles' scatter (tile order, and within a tile wavefront, row and lane order, as k_downsweep
-// ranks them, so the permutation is the same).  Items of a phase wait for every item of the phase
-// before, all of which were taken by workgroups that are running: the queue needs no co-resident grid.
-// Latency bound: one workgroup on the incremental path (4.5 us at 160k and 5.6 us at 4M particles, where
-// its launches took 46 us and 55 us); the full sort of 131k particles 69 us, the multi-block launches
-// 68 us without their gaps.
+// counter: per pass the items' digit counts, then their scatter, each tile put in order in LDS first (tile
+// order, and within a tile wavefront, row and lane order, as k_downsweep ranks them, so the permutation is the
+// same).  An item is a run of whole tiles, at most RS_ITEMS of them, so that a workgroup meets one or two a
+// phase.  Items of a phase wait for every item of the phase before, all of which were taken by workgroups
+// that are running: the queue needs no co-resident grid.
+// What other workgroups read is written through (st_agent) instead of by a fence that writes the whole L2 back
+// per item: with a tile an item, a third phase for the counts' scan and that fence the sort took 122, 274 and
+// 810 us at 270k, 1M and 4M particles (above the limit; the multi-block launches with their idle ones before
+// 86, 115 and 265), now 41, 107 and 230.
+// Latency bound: one workgroup on the incremental path (4.5 us at 160k and 5.6 us at 4M particles with 100 to
+// 400 changes, where its launches took 46 us and 55 us); per phase of the full sort some 8 us at 131k and 18 us
+// at 1M particles.
 constexpr int RESORT_BS = 1024;
 constexpr int RESORT_ITEMS = SORT_TILE / RESORT_BS;
 __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double *__restrict__ blanked,
@@ -405,15 +424,15 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
                                                       const int *__restrict__ old_keys, int *__restrict__ cell_start,
                                                       int N, int num_cell, int nb, int passes, int force, int cap,
                                                       int clear_old, int sort_here, int *k1, int *v1, int *k2, int *v2,
-                                                      int *__restrict__ hist, int *__restrict__ digit_tot, int *flags,
-                                                      int *sync, const int2 *__restrict__ clist, int2 *__restrict__ changed,
+                                                      int *__restrict__ hist, int *flags, int *sync, const int2 *__restrict__ clist, int2 *__restrict__ changed,
                                                       int *__restrict__ dests, int *__restrict__ removed) {
     __shared__ unsigned long long comp[SPHFEM_RESORT_CAP];
     __shared__ int gone[SPHFEM_RESORT_CAP];
-    // the sort's per-wavefront digit counts, in the bytes of the ranking's composites
-    static_assert(sizeof(int) * (RESORT_BS / WAVE) * RADIX <= sizeof(unsigned long long) * SPHFEM_RESORT_CAP, "LDS");
-    int (*wcount)[RADIX] = reinterpret_cast<int (*)[RADIX]>(comp);
-    __shared__ int off[RADIX], cnt[RADIX];
+    // the sort's per-wavefront digit counts and a tile in sorted order, in the bytes of the ranking's lists
+    static_assert(sizeof(int) * (RESORT_BS / WAVE) * RADIX <= sizeof(gone) && SORT_TILE <= SPHFEM_RESORT_CAP, "LDS");
+    int (*wcount)[RADIX] = reinterpret_cast<int (*)[RADIX]>(gone);
+    int (*sums)[RESORT_BS] = reinterpret_cast<int (*)[RESORT_BS]>(gone);
+    __shared__ int start[RADIX], cnt[RADIX], part[RADIX / WAVE];
     __shared__ int s_item, s_go;
     const int tid = threadIdx.x;
     const int m = sync[RS_COUNT];
@@ -473,9 +492,9 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
     if (!sort_here) return;
     const int w = tid / WAVE, lane = tid % WAVE;
     const uint64_t lt = lanemask_lt();
-    const bool scans = nb > RS_SCAN_TILES;
-    const int per_pass = scans ? 2 * nb + RADIX : 2 * nb;
-    const int items = passes * per_pass;
+    const int span = (nb + RS_ITEMS - 1) / RS_ITEMS * SORT_TILE;      // keys of an item
+    const int per_phase = (N + span - 1) / span;
+    const int items = passes * 2 * per_phase;
     // the item of a turn is taken and published between two barriers and read into a scalar, so that the
     // loop's control flow is uniform for the compiler too: a lane-dependent branch next to the back edge
     // lets it send the other lanes round the loop alone
@@ -483,31 +502,25 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
     __syncthreads();
     int item = __builtin_amdgcn_readfirstlane(s_item);
     while (item < items) {
-        // pass, step of the pass (0 counts, 1 scan, 2 scatter) and the item's number in it
-        const int ps = item / per_pass, at = item - ps * per_pass, shift = 8 * ps;
-        const int step = at < nb ? 0 : (scans && at < nb + RADIX ? 1 : 2);
-        const int tile = step == 0 ? at : (step == 1 ? at - nb : at - (per_pass - nb));
-        const int phase = 3 * ps + step;
+        // pass, step of the pass (0 counts, 1 scatter) and the item's number in it
+        const int phase = item / per_phase, at = item - phase * per_phase, ps = phase >> 1, shift = 8 * ps;
         if (phase > 0) {
-            const int before = step == 2 && !scans ? phase - 2 : phase - 1;
             if (tid == 0) {
-                s_go = wait_done(&sync[RS_DONE + before], step == 2 && scans ? RADIX : nb, flags) ? 1 : 0;
-                __threadfence();                      // the finished items' writes, from any XCD
+                s_go = wait_done(&sync[RS_DONE + phase - 1], per_phase, flags) ? 1 : 0;
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");   // the finished items' writes, from any XCD
             }
             __syncthreads();
             if (__builtin_amdgcn_readfirstlane(s_go) == 0) return;
         }
         // pass ps reads (ki, vi) and writes (ko, vo); the last pass ends in (k1, v1)
         const bool to1 = (passes - ps) % 2 != 0;
-        const int *ki = to1 ? k2 : k1, *vi = to1 ? v2 : v1;
-        int *ko = to1 ? k1 : k2, *vo = to1 ? v1 : v2;
-        const int base = tile * SORT_TILE;
-        if (step == 0) {                              // digit counts of the tile
+        int *ki = to1 ? k2 : k1, *ko = to1 ? k1 : k2, *vo = to1 ? v1 : v2;
+        const int *vi = to1 ? v2 : v1;
+        const int first = at * span, last = first + span < N ? first + span : N;
+        if ((phase & 1) == 0) {                       // digit counts of the item
             if (tid < RADIX) cnt[tid] = 0;
             __syncthreads();
-            for (int it = 0; it < RESORT_ITEMS; it++) {
-                const int i = base + it * RESORT_BS + tid;
-                if (i >= N) break;
+            for (int i = first + tid; i < last; i += RESORT_BS) {
                 int h;
                 if (ps == 0) {                        // the keys themselves, as k_hash_mark computed them
                     const int oh = old_keys[i];
@@ -515,110 +528,140 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
                     if (blanked[i] != 1.) h = hash_of(c, pos[i]);
                     h = h < 0 ? 0 : (h >= num_cell ? num_cell - 1 : h);
                     if (clear_old && h != oh && oh >= 0 && oh < num_cell) cell_start[oh] = -1;
-                    const_cast<int *>(ki)[i] = h;
+                    st_agent(&ki[i], h);
                 } else {
                     h = ki[i];
                 }
-                atomicAdd(&cnt[(h >> shift) & (RADIX - 1)], 1);
+                // nearly sorted keys: most wavefronts hold one value of the higher digits
+                const int d = (h >> shift) & (RADIX - 1), d0 = __builtin_amdgcn_readfirstlane(d);
+                const uint64_t same = __ballot(d == d0);
+                if (d != d0) atomicAdd(&cnt[d], 1);
+                else if (__popcll(same & lt) == 0) atomicAdd(&cnt[d0], __popcll(same));
             }
             __syncthreads();
-            if (tid < RADIX) hist[(long)tile * RADIX + tid] = cnt[tid];
-        } else if (step == 1) {                       // one digit's counts scanned over the tiles
-            int carry = 0;
-            for (int q0 = 0; q0 < nb; q0 += RESORT_BS) {
-                const int q = q0 + tid;
-                const int v = q < nb ? hist[(long)q * RADIX + tile] : 0;
-                int incl = v;
-                for (int o = 1; o < WAVE; o <<= 1) {
-                    const int u = __shfl_up(incl, o);
-                    if (lane >= o) incl += u;
-                }
-                if (lane == WAVE - 1) cnt[w] = incl;
-                __syncthreads();
-                int below = carry, all = carry;
-                for (int k = 0; k < RESORT_BS / WAVE; k++) {
-                    below += k < w ? cnt[k] : 0;
-                    all += cnt[k];
-                }
-                if (q < nb) hist[(long)q * RADIX + tile] = below + incl - v;
-                carry = all;
-                __syncthreads();
-            }
-            if (tid == 0) digit_tot[tile] = carry;
+            if (tid < RADIX) st_agent(&hist[(long)at * RADIX + tid], cnt[tid]);
         } else {
-            // offsets of the tile's digits: lower digits of all tiles, then lower tiles
-            if (tid < RADIX) {
+            // the item's digits in the output: lower digits of all items, then lower items; the items' counts
+            // are summed by a quarter of the lanes each
+            int key[RESORT_ITEMS], val[RESORT_ITEMS], next_key[RESORT_ITEMS], next_val[RESORT_ITEMS];
+            auto load = [&](int base) {               // of a tile, while the work before it runs
+#pragma unroll
+                for (int q = 0; q < RESORT_ITEMS; q++) {
+                    const int i = base + w * (RESORT_ITEMS * WAVE) + q * WAVE + lane;
+                    next_key[q] = i < last ? ki[i] : 0;
+                    next_val[q] = i < last ? (ps == 0 ? i : vi[i]) : 0;
+                }
+            };
+            load(first);
+            {
+                const int d = tid & (RADIX - 1);
                 int below = 0, all = 0;
-                if (scans) {
-                    below = hist[(long)tile * RADIX + tid];
-                    all = digit_tot[tid];
-                } else {
-                    for (int q = 0; q < nb; q++) {
-                        const int v = hist[(long)q * RADIX + tid];
-                        all += v;
-                        below += q < tile ? v : 0;
+                for (int q0 = tid / RADIX; q0 < per_phase; q0 += 16 * (RESORT_BS / RADIX)) {
+                    int v[16];                        // loaded together
+#pragma unroll
+                    for (int u = 0; u < 16; u++) {
+                        const int q = q0 + u * (RESORT_BS / RADIX);
+                        v[u] = q < per_phase ? hist[(long)q * RADIX + d] : 0;
+                    }
+#pragma unroll
+                    for (int u = 0; u < 16; u++) {
+                        all += v[u];
+                        below += q0 + u * (RESORT_BS / RADIX) < at ? v[u] : 0;
                     }
                 }
-                off[tid] = below;
-                cnt[tid] = all;
+                sums[0][tid] = below;
+                sums[1][tid] = all;
             }
-            for (int k = tid; k < (RESORT_BS / WAVE) * RADIX; k += RESORT_BS) (&wcount[0][0])[k] = 0;
             __syncthreads();
-            for (int o = 1; o < RADIX; o <<= 1) {
-                const int v = tid < RADIX && tid >= o ? cnt[tid - o] : 0;
+            int offset = 0;                           // of digit tid
+            if (tid < RADIX) {
+                int all = 0;
+                for (int q = 0; q < RESORT_BS / RADIX; q++) {
+                    offset += sums[0][q * RADIX + tid];
+                    all += sums[1][q * RADIX + tid];
+                }
+                const int incl = wave_inclusive(all);
+                if (lane == WAVE - 1) part[w] = incl;
+                offset += incl - all;
+            }
+            __syncthreads();
+            if (tid < RADIX)
+                for (int k = 0; k < w; k++) offset += part[k];
+            for (int base = first; base < last; base += SORT_TILE) {
+                int rank[RESORT_ITEMS];
+#pragma unroll
+                for (int q = 0; q < RESORT_ITEMS; q++) {
+                    key[q] = next_key[q];
+                    val[q] = next_val[q];
+                }
+                if (base + SORT_TILE < last) load(base + SORT_TILE);
+                for (int k = tid; k < (RESORT_BS / WAVE) * RADIX; k += RESORT_BS) (&wcount[0][0])[k] = 0;
                 __syncthreads();
-                if (tid < RADIX) cnt[tid] += v;
+#pragma unroll
+                for (int q = 0; q < RESORT_ITEMS; q++) {
+                    const bool valid = base + w * (RESORT_ITEMS * WAVE) + q * WAVE + lane < N;
+                    const int d = (key[q] >> shift) & (RADIX - 1);
+                    uint64_t peers = __ballot(valid);
+#pragma unroll
+                    for (int b = 0; b < 8; b++) {
+                        const uint64_t mm = __ballot((d >> b) & 1);
+                        peers &= ((d >> b) & 1) ? mm : ~mm;
+                    }
+                    const int before = __popcll(peers & lt);
+                    int old = 0;
+                    if (valid) old = wcount[w][d];
+                    __builtin_amdgcn_wave_barrier();
+                    if (valid && before == 0) wcount[w][d] = old + __popcll(peers);
+                    __builtin_amdgcn_wave_barrier();
+                    rank[q] = valid ? old + before : -1;
+                }
                 __syncthreads();
-            }
-            if (tid < RADIX && tid > 0) off[tid] += cnt[tid - 1];
-            int key[RESORT_ITEMS], val[RESORT_ITEMS], rank[RESORT_ITEMS];
-#pragma unroll
-            for (int q = 0; q < RESORT_ITEMS; q++) {
-                const int i = base + w * (RESORT_ITEMS * WAVE) + q * WAVE + lane;
-                const bool valid = i < N;
-                const int k = valid ? ki[i] : 0;
-                key[q] = k;
-                val[q] = valid ? (ps == 0 ? i : vi[i]) : 0;
-                const int d = (k >> shift) & (RADIX - 1);
-                uint64_t peers = __ballot(valid);
-#pragma unroll
-                for (int b = 0; b < 8; b++) {
-                    const uint64_t mm = __ballot((d >> b) & 1);
-                    peers &= ((d >> b) & 1) ? mm : ~mm;
+                // each digit's prefix over the tile's wavefronts, its start in the tile's sorted order, and
+                // (cnt) its place in the output less that
+                int mine = 0, incl = 0;
+                if (tid < RADIX) {
+                    for (int k = 0; k < RESORT_BS / WAVE; k++) {
+                        const int v = wcount[k][tid];
+                        wcount[k][tid] = mine;
+                        mine += v;
+                    }
+                    incl = wave_inclusive(mine);
+                    if (lane == WAVE - 1) part[w] = incl;
                 }
-                const int before = __popcll(peers & lt);
-                int old = 0;
-                if (valid) old = wcount[w][d];
-                __builtin_amdgcn_wave_barrier();
-                if (valid && before == 0) wcount[w][d] = old + __popcll(peers);
-                __builtin_amdgcn_wave_barrier();
-                rank[q] = valid ? old + before : -1;
-            }
-            __syncthreads();
-            if (tid < RADIX) {                        // prefix of each digit over the tile's wavefronts
-                int run = off[tid];
-                for (int k = 0; k < RESORT_BS / WAVE; k++) {
-                    const int v = wcount[k][tid];
-                    wcount[k][tid] = run;
-                    run += v;
+                __syncthreads();
+                if (tid < RADIX) {
+                    for (int k = 0; k < w; k++) incl += part[k];
+                    start[tid] = incl - mine;
+                    cnt[tid] = offset - (incl - mine);
+                    offset += mine;
                 }
-            }
-            __syncthreads();
+                __syncthreads();
+                // the tile in sorted order, so that the output is written in runs
 #pragma unroll
-            for (int q = 0; q < RESORT_ITEMS; q++) {
-                if (rank[q] < 0) continue;
-                const int dst = wcount[w][(key[q] >> shift) & (RADIX - 1)] + rank[q];
-                if ((unsigned)dst >= (unsigned)N) {   // cannot happen for consistent counts
-                    atomicOr(&flags[0], 2);
-                    continue;
+                for (int q = 0; q < RESORT_ITEMS; q++) {
+                    if (rank[q] < 0) continue;
+                    const int d = (key[q] >> shift) & (RADIX - 1);
+                    comp[start[d] + wcount[w][d] + rank[q]] =
+                        ((unsigned long long)(unsigned)key[q] << 32) | (unsigned)val[q];
                 }
-                ko[dst] = key[q];
-                vo[dst] = val[q];
+                __syncthreads();
+#pragma unroll
+                for (int q = 0; q < RESORT_ITEMS; q++) {
+                    const int l = q * RESORT_BS + tid;
+                    if (base + l >= N) break;
+                    const int k = (int)(comp[l] >> 32), v = (int)(unsigned)comp[l];
+                    const int dst = cnt[(k >> shift) & (RADIX - 1)] + l;
+                    if ((unsigned)dst >= (unsigned)N) {   // cannot happen for consistent counts
+                        atomicOr(&flags[0], 2);
+                        continue;
+                    }
+                    st_agent(&ko[dst], k);
+                    st_agent(&vo[dst], v);
+                }
             }
         }
         stores_done_barrier();                        // this item's writes before it counts as done
         if (tid == 0) {
-            __threadfence();
             atomicAdd(&sync[RS_DONE + phase], 1);
             s_item = atomicAdd(&sync[RS_TICKET], 1);
         }
@@ -665,7 +708,7 @@ void launch_resort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, sphfem_
         k_resort<<<blocks, RESORT_BS, 0, ctx->stream>>>(ctx->c, p.blanked, p.pos, p.hash, g->cell_start, N,
                                                         g->num_cell, nb, passes, force, cap, clear_old,
                                                         launches ? 0 : 1, g->keys_alt, p.idx, g->keys_tmp,
-                                                        g->vals_alt, g->hist, g->digit_tot, flags, g->sync, g->clist,
+                                                        g->vals_alt, g->hist, flags, g->sync, g->clist,
                                                         g->changed, g->dests, g->removed);
     }
     if (launches)

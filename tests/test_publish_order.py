@@ -31,19 +31,31 @@ def _body(asm, kernel):
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None and not os.path.exists("/opt/rocm/bin/hipcc"), reason="no hipcc")
-@pytest.mark.parametrize("source,kernel", [("sphfem_sort.hip", "k_resort"), ("sphfem_tool.hip", "k_near_contact")])
-def test_every_wavefront_waits_for_its_stores(source, kernel, tmp_path):
+@pytest.mark.parametrize("source,kernel,fenced", [("sphfem_sort.hip", "k_resort", False),
+                                                  ("sphfem_tool.hip", "k_near_contact", True)])
+def test_every_wavefront_waits_for_its_stores(source, kernel, fenced, tmp_path):
+    """fenced: plain stores, written back by the announcing lane's fence; else every store that other
+    workgroups read is written through (sc1) and the counter is bumped without a fence."""
     lines = _body(_assembly(source, tmp_path), kernel)
-    found = 0
-    for k, line in enumerate(lines):
-        if not line.startswith("buffer_wbl2"):
-            continue
-        after = next(l for l in lines[k + 1:] if l.startswith(("s_barrier", "buffer_wbl2", "global_atomic", "s_endpgm")))
-        if not after.startswith("global_atomic_add"):
-            continue                                    # the fence of a workgroup that reads others' results
-        found += 1
-        b = max(q for q in range(k) if lines[q] == "s_barrier")
-        before = next(l for l in reversed(lines[:b])
-                      if l.startswith(("global_", "flat_", "buffer_", "s_branch", "s_cbranch", ".LBB")) or "vmcnt(0)" in l)
-        assert "vmcnt(0)" in before, f"{kernel}: the barrier before the announcement follows `{before}`, not a wait"
-    assert found == 1
+
+    def announces(k):
+        if fenced:
+            if not lines[k].startswith("buffer_wbl2"):
+                return False
+            after = next(l for l in lines[k + 1:] if l.startswith(("s_barrier", "buffer_wbl2", "global_atomic", "s_endpgm")))
+            return after.startswith("global_atomic_add")   # else the fence of a workgroup that reads others' results
+        return lines[k].startswith("global_atomic_add") and "sc0" not in lines[k]       # returns nothing: the counter
+
+    found = [k for k in range(len(lines)) if announces(k)]
+    assert len(found) == 1
+    b = max(q for q in range(found[0]) if lines[q] == "s_barrier")
+    before = next(l for l in reversed(lines[:b])
+                  if l.startswith(("global_", "flat_", "buffer_", "s_branch", "s_cbranch", ".LBB")) or "vmcnt(0)" in l)
+    assert "vmcnt(0)" in before, f"{kernel}: the barrier before the announcement follows `{before}`, not a wait"
+    if not fenced:
+        queue = next(k for k, l in enumerate(lines) if l.startswith("global_atomic_add"))       # the first ticket
+        stores = [l for l in lines[queue:] if l.startswith("global_store")]
+        through = [l for l in stores if "sc1" in l]
+        # the keys of pass 0, the counts, and keys and sources of the scatter; the only other store clears cells
+        assert len(through) >= 4 and len(stores) - len(through) <= 1, stores
+        assert not any(l.startswith("buffer_wbl2") for l in lines)
