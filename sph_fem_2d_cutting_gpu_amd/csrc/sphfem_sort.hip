@@ -270,6 +270,10 @@ enum { RS_COUNT = 0, RS_TICKET = 1, RS_DONE = 2 };   // RS_DONE + phase: finishe
 constexpr int RS_USED = RS_DONE + 2 * 4;             // at most four passes of two phases
 static_assert(RS_USED <= SPHFEM_RESORT_SYNC, "counters");
 constexpr int RS_ITEMS = 256;                        // work items of a phase at most, of whole tiles
+// changes up to which their ranks are counted (one change a lane, m comparisons), above by a bitonic sort: steps of
+// 65k particles with 90, 820, 1890 and 3140 changes 134, 142, 230 and 281 us by counting, 140, 146, 167 and 179
+// by the sort
+constexpr int RS_COUNTED = 768;
 
 struct StepStart {            // what else begins with the step (see k_hash_mark)
     sphfem_tool tool;
@@ -443,45 +447,73 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
     }
     if (!full) {
         if (blockIdx.x != 0) return;
-        for (int k = tid; k < m; k += RESORT_BS) {
-            const int2 e = clist[k];
+        // the changed particles by (new key, position) and their positions alone, by counting or a bitonic sort
+        int np = 64;
+        while (np < m) np <<= 1;
+        for (int k = tid; k < np; k += RESORT_BS) {
+            const int2 e = k < m ? clist[k] : make_int2(-1, INT_MAX);
             comp[k] = ((unsigned long long)(unsigned)e.x << 32) | (unsigned)e.y;
+            gone[k] = e.y;
         }
         __syncthreads();
-        // ranks by counting: r by (new key, position), rp by position
-        int r[SPHFEM_RESORT_CAP / RESORT_BS], P[SPHFEM_RESORT_CAP / RESORT_BS];
-#pragma unroll
-        for (int u = 0; u < SPHFEM_RESORT_CAP / RESORT_BS; u++) {
-            const int k = tid + u * RESORT_BS;
-            if (k >= m) continue;
-            const unsigned long long ck = comp[k];
-            const int at = (int)(unsigned)ck;
-            P[u] = insert_position(old_keys, cell_start, N, (int)(ck >> 32), at);
+        if (m <= RS_COUNTED) {
+            const unsigned long long mine = tid < m ? comp[tid] : 0ull;
+            const int at = (int)(unsigned)mine;
             int rank = 0, rp = 0;
-            for (int q = 0; q < m; q++) {
-                const unsigned long long cq = comp[q];
-                rank += cq < ck;
-                rp += (int)(unsigned)cq < at;
+            if (tid < m)
+                for (int q = 0; q < m; q++) {
+                    const unsigned long long other = comp[q];
+                    rank += other < mine;
+                    rp += (int)(unsigned)other < at;
+                }
+            __syncthreads();
+            if (tid < m) {
+                comp[rank] = mine;
+                gone[rp] = at;
             }
-            r[u] = rank;
-            gone[rp] = at;
-            removed[rp] = at;
+            __syncthreads();
+        } else {
+            for (int size = 2; size <= np; size <<= 1) {
+                for (int stride = size >> 1; stride > 0; stride >>= 1) {
+                    for (int q = tid; q < np >> 1; q += RESORT_BS) {
+                        const int a = 2 * q - (q & (stride - 1)), b = a + stride;
+                        const bool up = (a & size) == 0;
+                        const unsigned long long ca = comp[a], cb = comp[b];
+                        if ((ca > cb) == up) {
+                            comp[a] = cb;
+                            comp[b] = ca;
+                        }
+                        const int ga = gone[a], gb = gone[b];
+                        if ((ga > gb) == up) {
+                            gone[a] = gb;
+                            gone[b] = ga;
+                        }
+                    }
+                    __syncthreads();
+                }
+            }
         }
-        __syncthreads();
+        int P[SPHFEM_RESORT_CAP / RESORT_BS];
 #pragma unroll
         for (int u = 0; u < SPHFEM_RESORT_CAP / RESORT_BS; u++) {
-            const int k = tid + u * RESORT_BS;
-            if (k >= m) continue;
-            const unsigned long long ck = comp[k];
-            const int at = (int)(unsigned)ck;
+            const int r = tid + u * RESORT_BS;
+            if (r < m) P[u] = insert_position(old_keys, cell_start, N, (int)(comp[r] >> 32), (int)(unsigned)comp[r]);
+        }
+        __syncthreads();                              // before any cell is cleared
+#pragma unroll
+        for (int u = 0; u < SPHFEM_RESORT_CAP / RESORT_BS; u++) {
+            const int r = tid + u * RESORT_BS;
+            if (r >= m) continue;
+            const int at = (int)(unsigned)comp[r];
             int lo = 0, hi = m;                       // removed positions below P
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
                 if (gone[mid] < P[u]) lo = mid + 1;
                 else hi = mid;
             }
-            dests[r[u]] = r[u] + P[u] - lo;
-            changed[r[u]] = make_int2((int)(ck >> 32), at);
+            dests[r] = r + P[u] - lo;
+            changed[r] = make_int2((int)(comp[r] >> 32), at);
+            removed[r] = gone[r];
             // a cell that keeps one of its particles gets its start again from the reorder; one that all
             // of them left is cleared by each of them
             const int oh = old_keys[at];
