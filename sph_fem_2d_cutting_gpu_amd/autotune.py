@@ -10,9 +10,8 @@ Tunables (all result-neutral except the FP32 summation blocks of the FP32C form)
                     one wavefront per workgroup, so pair_block does not apply); same sums.  Each
                     also fused with the update (the particle's update right after its sums: no
                     pair-sum round trip, update_block does not apply); same step result
-  * resort_one_block -- 0 or 1 (N <= 2^19); both run the same kernels (the step's full-sort fallback
-                    is one launch), tried with the best of the others
   * graph_steps  -- steps per captured graph in a batch (2 ... 32): fewer graph launches per step
+(resort_one_block of the tuning selects nothing and stays 0.)
 The tuner times each candidate on the live workload (it advances the simulation: run it in the
 warm-up), keeps the fastest and can store the choice in a JSON cache keyed by workload size,
 precision and device.
@@ -68,14 +67,6 @@ def tune_simulation(sim, precision, steps=6, repeats=2, pair_kernel=None) -> dic
         rows.append((t, cand))
     sim.ctx.check_error()
     t_best, best = min(rows, key=lambda r: r[0])
-    if sim.case.N <= _lib.SORT_ONE_BLOCK_MAX:
-        cand = dict(best, resort_one_block=1)
-        sim.set_tuning(**cand)
-        t = min(_time_steps(sim, steps) for _ in range(repeats))
-        rows.append((t, cand))
-        sim.ctx.check_error()
-        if t < t_best:
-            t_best, best = t, cand
     sim.set_tuning(**best)
     return {"best": best, "ms_per_step": t_best * 1e3,
             "timings": [{**c, "ms_per_step": t * 1e3} for t, c in rows]}

@@ -28,3 +28,27 @@ def test_cache_roundtrip(tmp_path):
     autotune.save_cache(path, {key: {"pair_block": 128, "pair_chunk": 48, "update_block": 256}})
     assert autotune.load_cache(path)[key]["pair_chunk"] == 48
     assert autotune.load_cache(str(tmp_path / "absent.json")) == {}
+
+
+def test_tuner_times_each_candidate_and_no_other():
+    """resort_one_block selects nothing, so no candidate differs in it alone."""
+    class Sim:
+        class ctx:
+            check_error = synchronize = staticmethod(lambda: None)
+
+        class case:
+            N = 6400
+
+        def __init__(self):
+            self.tried = []
+
+        def set_tuning(self, **kw):
+            self.tried.append(kw)
+
+        def step(self, n):
+            pass
+
+    sim = Sim()
+    res = autotune.tune_simulation(sim, _lib.FP32C, steps=1, repeats=1)
+    assert sim.tried[:-1] == autotune.candidates(_lib.FP32C) and sim.tried[-1] == res["best"]
+    assert res["best"]["resort_one_block"] == 0

@@ -79,9 +79,9 @@ def test_tune_simulation_applies_a_candidate():
     sim = S.Simulation(cases.small_cutting_case(nx=32, ny=12), precision=_lib.FP32C)
     sim.step(1)
     res = autotune.tune_simulation(sim, _lib.FP32C, steps=2, repeats=1)
-    assert dict(res["best"], resort_one_block=0) in autotune.candidates(_lib.FP32C)
+    assert res["best"] in autotune.candidates(_lib.FP32C)
     assert sim.get_tuning() == res["best"]
-    assert len(res["timings"]) == len(autotune.candidates(_lib.FP32C)) + 1     # + the one-block fallback
+    assert len(res["timings"]) == len(autotune.candidates(_lib.FP32C))
     sim.close()
 
 
