@@ -38,8 +38,8 @@ __device__ __forceinline__ void column_range(const int *__restrict__ cs, const i
 // particle step's kernel while a pair's fields took 13 loads of 8 to 32 byte records, and a candidate's
 // position and blanked flag two (503 us).  Eight loads of 16-byte records, and four candidates at a time:
 // 417 us; all eight issued before the first is used: 358 us.  Loading the next pair's fields ahead costs
-// a third of the wavefronts (188 registers): 392 us.  The in-support neighbours go through a per-lane list of CHUNK entries in
-// LDS (list = this lane's first entry, stride LIST_BS) before their terms are evaluated.
+// a third of the wavefronts (188 registers): 392 us.  The in-support neighbours go through a per-lane list
+// of CHUNK entries in LDS (list = this lane's first entry, stride LIST_BS) before their terms are evaluated.
 // WIN: every non-blanked particle of the 5x5 cells is evaluated, as the reference does, instead of
 // the in-support ones only.  The kernel's zeros outside the support make the two the same sums for
 // finite inputs; a neighbour with a non-finite input turns the sums NaN (0 * NaN) in the reference
@@ -88,8 +88,9 @@ __device__ __forceinline__ PairSums pair_sums_fp64(const DevConsts &c, const sph
         const double xij = pi.x - pj.x, yij = pi.y - pj.y;
         const bool heat = thermal_alpha != 0.;
         const double r2 = xij * xij + yij * yij;
-        // the shared-reciprocal form (the 1M-particle step's k_pairs_fp64 529 -> 497 us) while the single-precision radius and the quotients by it are normal
-        // numbers (in any length unit a case is set up in), else, and in the window form, the plain one
+        // the shared-reciprocal form (the 1M-particle step's k_pairs_fp64 529 -> 497 us) while the
+        // single-precision radius and the quotients by it are normal numbers (in any length unit a case is
+        // set up in), else, and in the window form, the plain one
         RadialTerms t;
         if (!WIN && r2 > 1e-36 && r2 < 1e36) t = radial_terms(xij, yij, r2, hi, h1, heat);
         else t = radial_terms_plain(pi.x, pi.y, pj.x, pj.y, xij, yij, r2, hi, rr2_min, heat);
@@ -358,10 +359,10 @@ __device__ __forceinline__ double2 wide_pos(const RecView &rv, int ny, int j, in
 // ROLL: the columns in a loop, which leaves the kernel with 128 registers and four wavefronts per SIMD
 // where no update follows the sums (16 M particles: 3000 -> 2827 us); with the update's 166 registers there
 // are three either way, and the unrolled columns are the faster (4 M: 779 us against 796).  Copying all
-// records of 256-particle tiles to LDS cut the L1's accesses by five and cost as much in other issue.  Positions of 16 bytes
-// (cell-relative FP32 and the cell row, with the column in the list entry) and kernel factors applied
-// per pair took 868 us (with the update) on 4 M particles and 3337 us (sums alone) on 16 M, against 779
-// and 2827 us.
+// records of 256-particle tiles to LDS cut the L1's accesses by five and cost as much in other issue.
+// Positions of 16 bytes (cell-relative FP32 and the cell row, with the column in the list entry) and kernel
+// factors applied per pair took 868 us (with the update) on 4 M particles and 3337 us (sums alone) on 16 M,
+// against 779 and 2827 us.
 // General form (GEN; the SPHFEM_FORM_ bits): kernel widths other than the cell size, at a fifth load per pair and
 // the factors of h_i; and (SPECIAL), with a test of every candidate's record, widths that reach the place of
 // blanked records, positions that the wrapped ones cannot tell apart, taken in FP64, and the window form, where
@@ -795,7 +796,7 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
         };
 
         int end = 0;               // BS times the number of entries
-#pragma unroll (ROLL ? 1 : 5)
+#pragma unroll ROLL ? 1 : 5
         for (int d = 0; d < 5; d++) {
             const int col = gi - 2 + d;
             int first = lo_s, last = hi_s != -1 ? hi_e : -1;
@@ -894,7 +895,8 @@ __device__ __forceinline__ PairOut pairs_fp32c_list(const DevConsts &c, const in
                                                     int form) {
     const GlobalPos pos{rv.pos};
     if (form == 0)
-        return pairs_fp32c_one<BS, CHUNK, false, false, TO != TO_UPDATE>(c, hash, N, rv, cs, ce, i, list, pos, nullptr, 0);
+        return pairs_fp32c_one<BS, CHUNK, false, false, TO != TO_UPDATE>(c, hash, N, rv, cs, ce, i, list, pos, nullptr,
+                                                                         0);
     if (TO != TO_UPDATE && form == SPHFEM_FORM_WIDTH)
         return pairs_fp32c_one<BS, CHUNK, true, false, true>(c, hash, N, rv, cs, ce, i, list, pos, nullptr, form);
     return pairs_fp32c_one<BS, CHUNK, true, true, true>(c, hash, N, rv, cs, ce, i, list, pos, nullptr, form);
@@ -1009,8 +1011,8 @@ __global__ void __launch_bounds__(64) k_pairs_fp32c_staged(DevConsts c, const in
     if (i >= N) return;
     PairOut o;
     if (staged)
-        o = pairs_fp32c_one<64, CHUNK, false, false, false, StagedPos>(c, hash, N, rv, cs, ce, i, list16 + lane, sp, flags,
-                                                                       0);
+        o = pairs_fp32c_one<64, CHUNK, false, false, false, StagedPos>(c, hash, N, rv, cs, ce, i, list16 + lane, sp,
+                                                                       flags, 0);
     else
         o = pairs_fp32c_list<64, CHUNK, TO>(c, hash, N, rv, cs, ce, i, list32 + lane, form);
     emit_pairs<TO, RIGID>(c, u, psum, psum_T, N, i, o);

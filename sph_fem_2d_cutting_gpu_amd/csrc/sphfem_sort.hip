@@ -250,10 +250,10 @@ void launch_radix_sort(sphfem_ctx *ctx, sphfem_grid *g, sphfem_particles &p, int
 // key or index array is written and read back in between.  The full sort runs on the first step and
 // whenever more than `cap` particles changed cells: k_resort's workgroups run it in that one launch.
 // Where the host knows of it before (force) and N is above SPHFEM_SORT_ONE_LAUNCH_MAX it is the
-// multi-block radix sort, whose launches beat the queue's waits there (steps of 131k, 400k, 550k, 750k and 1M
-// particles 199, 303, 366, 443 and 549 us by the queue; 314, 362, 428 and 511 us by launches from 400k on).  (Per step with the incremental
-// path before: the hash pass, scan, three idle launches per radix pass, compaction, ranking and
-// scatter, each a dependent launch of about 4.5 us.)
+// multi-block radix sort, whose launches beat the queue's waits there (steps of 400k, 550k, 750k and 1M
+// particles 303, 366, 443 and 549 us by the queue, 314, 362, 428 and 511 us by launches).  (Per step with
+// the incremental path before: the hash pass, scan, three idle launches per radix pass, compaction, ranking
+// and scatter, each a dependent launch of about 4.5 us.)
 // Sorted keys and permutation end in (g->keys_alt, p.idx); the caller swaps keys_alt and p.hash.
 // ---------------------------------------------------------------------------------------------
 
@@ -428,7 +428,8 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
                                                       const int *__restrict__ old_keys, int *__restrict__ cell_start,
                                                       int N, int num_cell, int nb, int passes, int force, int cap,
                                                       int clear_old, int sort_here, int *k1, int *v1, int *k2, int *v2,
-                                                      int *__restrict__ hist, int *flags, int *sync, const int2 *__restrict__ clist, int2 *__restrict__ changed,
+                                                      int *__restrict__ hist, int *flags, int *sync,
+                                                      const int2 *__restrict__ clist, int2 *__restrict__ changed,
                                                       int *__restrict__ dests, int *__restrict__ removed) {
     __shared__ unsigned long long comp[SPHFEM_RESORT_CAP];
     __shared__ int gone[SPHFEM_RESORT_CAP];
@@ -1103,9 +1104,10 @@ __device__ __forceinline__ void flag_nonfinite(int *__restrict__ form, double bl
 // factors of the pair sum, (S - p)/rho^2 and S_xy/rho^2; the temperature is stored as T - T_init, so
 // that the FP32 differences T_i - T_j of a nearly uniform field keep ~1e-7 of the deviation instead of
 // ~1e-7 of T.
-__device__ __forceinline__ void write_records(const DevConsts &c, const RecView &rec, double inv_dx, int *__restrict__ form, int i, int h,
-                                             sphfem_double2 pos, sphfem_double2 vel, sphfem_double4 S, double rho, double T, double blanked,
-                                             double tool, double hh, double pr, sphfem_double4 R) {
+__device__ __forceinline__ void write_records(const DevConsts &c, const RecView &rec, double inv_dx,
+                                              int *__restrict__ form, int i, int h, sphfem_double2 pos,
+                                              sphfem_double2 vel, sphfem_double4 S, double rho, double T,
+                                              double blanked, double tool, double hh, double pr, sphfem_double4 R) {
     const int ny = c.geom.ny;
     const int ix = h / ny, iy = h - ix * ny;
     // cell units from the centre of the particle's cell.  Blanked particles are put 8 cells from it along
@@ -1136,7 +1138,7 @@ __device__ __forceinline__ void write_records(const DevConsts &c, const RecView 
         uy += (unsigned)(int)rint(cy * unit);
     }
     const int2 r0 = make_int2((int)ux, (int)uy);
-    // the form of the pair sums: one store per wavefront and bit
+    // the form of the pair sums: one store per wavefront and word
     const int bits = (__any(live && hh != c.geom.dx) ? SPHFEM_FORM_WIDTH : 0) |
                      (__any(live && !near) ? SPHFEM_FORM_AWAY : 0) |
                      (__any(live && hh > 2. * c.geom.dx) ? SPHFEM_FORM_REACH : 0);

@@ -777,7 +777,8 @@ __device__ __forceinline__ void seg_add(const SegSink &s, int n, SegLds &l, cons
     }
 }
 
-template <int Q0, int NV, int BS> __device__ __forceinline__ void seg_sums(const SegSink &s, int n, SegLds &l, const SegDst &d) {
+template <int Q0, int NV, int BS>
+__device__ __forceinline__ void seg_sums(const SegSink &s, int n, SegLds &l, const SegDst &d) {
     static_assert(SPHFEM_SEG_SINK_CAP % BS == 0, "sink capacity: whole records per lane");
     seg_order<BS>(s, n, l);
     if (n <= BS) seg_add<Q0, NV, BS, 1>(s, n, l, d);

@@ -62,15 +62,22 @@ def test_stage_calls_skip_blanked_particles_anywhere():
     sim.close()
 
 
+@pytest.mark.parametrize("which", ["chip", "cutting"])
 @pytest.mark.parametrize("prec", [_lib.FP64, _lib.FP32C])
-def test_one_nan_velocity_stays_in_its_window(prec):
-    case = cases.chip_case(n_target=800)
+def test_one_nan_velocity_stays_in_its_window(prec, which):
+    """Without a tool, and with one (the near-tool pass and the tool's end of the step)."""
+    if which == "chip":
+        case = cases.chip_case(n_target=800)
+        at = np.median(case.pos, axis=0)
+    else:
+        case = cases.perturbed(cases.small_cutting_case(nx=48, ny=16, wear=True))
+        at = np.array([0.0140, 0.0590])
     vel = case.vel.copy()
-    vel[int(np.argmin(np.hypot(*(case.pos - np.median(case.pos, axis=0)).T)))] = [0.0, np.nan]
+    vel[int(np.argmin(np.hypot(*(case.pos - at).T)))] = [0.0, np.nan]
     case = dataclasses.replace(case, vel=vel)
     o, sim = Oracle(case), S.Simulation(case, precision=prec)
     for step in range(1, 4):
-        print(prec, "step", step, flush=True)
+        print(which, prec, "step", step, flush=True)
         o.step(1)
         sim.step(1)
         sim.ctx.check_error()
