@@ -418,12 +418,14 @@ __device__ __forceinline__ bool wait_done(int *counter, int want, int *flags) {
 // per item: with a tile an item, a third phase for the counts' scan and that fence the sort took 122, 274 and
 // 810 us at 270k, 1M and 4M particles (above the limit; the multi-block launches with their idle ones before
 // 86, 115 and 265), now 41, 107 and 230.
+// 72 registers at most: the workgroups that find nothing to do wait for room beside other streams' kernels (84
+// registers: a sweep of 16 cases 1297 us against 1283).
 // Latency bound: one workgroup on the incremental path (4.5 us at 160k and 5.6 us at 4M particles with 100 to
 // 400 changes, where its launches took 46 us and 55 us); per phase of the full sort some 8 us at 131k and 18 us
 // at 1M particles.
 constexpr int RESORT_BS = 1024;
 constexpr int RESORT_ITEMS = SORT_TILE / RESORT_BS;
-__global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double *__restrict__ blanked,
+__global__ void __launch_bounds__(RESORT_BS, 7) k_resort(DevConsts c, const double *__restrict__ blanked,
                                                       const sphfem_double2 *__restrict__ pos,
                                                       const int *__restrict__ old_keys, int *__restrict__ cell_start,
                                                       int N, int num_cell, int nb, int passes, int force, int cap,
@@ -589,15 +591,15 @@ __global__ void __launch_bounds__(RESORT_BS) k_resort(DevConsts c, const double 
             {
                 const int d = tid & (RADIX - 1);
                 int below = 0, all = 0;
-                for (int q0 = tid / RADIX; q0 < per_phase; q0 += 16 * (RESORT_BS / RADIX)) {
-                    int v[16];                        // loaded together
+                for (int q0 = tid / RADIX; q0 < per_phase; q0 += 8 * (RESORT_BS / RADIX)) {
+                    int v[8];                         // loaded together
 #pragma unroll
-                    for (int u = 0; u < 16; u++) {
+                    for (int u = 0; u < 8; u++) {
                         const int q = q0 + u * (RESORT_BS / RADIX);
                         v[u] = q < per_phase ? hist[(long)q * RADIX + d] : 0;
                     }
 #pragma unroll
-                    for (int u = 0; u < 16; u++) {
+                    for (int u = 0; u < 8; u++) {
                         all += v[u];
                         below += q0 + u * (RESORT_BS / RADIX) < at ? v[u] : 0;
                     }
