@@ -37,8 +37,9 @@ __device__ __forceinline__ void column_range(const int *__restrict__ cs, const i
 // drift apart, each load touches some 30 lines, and 2.3e8 of them filled 82 % of the cycles of the 1 M
 // particle step's kernel while a pair's fields took 13 loads of 8 to 32 byte records, and a candidate's
 // position and blanked flag two (503 us).  Eight loads of 16-byte records, and four candidates at a time:
-// 417 us; all eight issued before the first is used: 358 us.  Loading the next pair's fields ahead costs
-// a third of the wavefronts (188 registers): 392 us.  The in-support neighbours go through a per-lane list
+// 417 us; all eight issued before the first is used: 358 us (371 with dividends outside 2^+-600 divided plainly;
+// 145 M accesses, 69 % of the cycles, and 59 % of the VALU's).  Loading the next pair's fields ahead costs a
+// third of the wavefronts (188 registers): 392 us.  The in-support neighbours go through a per-lane list
 // of CHUNK entries in LDS (list = this lane's first entry, stride LIST_BS) before their terms are evaluated.
 // WIN: every non-blanked particle of the 5x5 cells is evaluated, as the reference does, instead of
 // the in-support ones only.  The kernel's zeros outside the support make the two the same sums for
@@ -1052,7 +1053,7 @@ __global__ void __launch_bounds__(256) k_pre_state(DevConsts c, const sphfem_par
 // and the FP64 arithmetic of the in-support pairs: evaluating the whole window instead (about twice
 // the pairs, with each neighbour's factors divided out again per pair) took 3106 us per launch at
 // 2.07M particles of the chip domain, this and k_pre_state 2140 us, 2010 us with the shared reciprocals,
-// 1320 us with the fields in 16-byte records (pair_sums_fp64).
+// 1320 us with the fields in 16-byte records, 1360 us with extreme dividends divided plainly (pair_sums_fp64).
 __global__ void __launch_bounds__(256) k_interactions_ref(DevConsts c, sphfem_particles P, const int *__restrict__ cs,
                                                           const int *__restrict__ ce,
                                                           const PreView pre,
