@@ -279,7 +279,7 @@ __device__ __forceinline__ void pair_term(const PairI &I, float dx, float dy, co
     float w = outer ? s * s * s : 0.0625f - (0.09375f * ku * ku) * D2 * u;
     float g = outer ? s * rinv : ku - (0.75f * ku * ku) * r;
     if constexpr (GEN) {
-        if (win && !(D2 < I.D2max && D2 >= I.D2min)) {
+        if (win && (D2 >= I.D2max || D2 < I.D2min)) {        // a NaN distance keeps its NaN kernel
             w = 0.f;
             g = 0.f;
         }
@@ -371,6 +371,9 @@ __device__ __forceinline__ double2 wide_pos(const RecView &rv, int ny, int j, in
 // reference does (see pair_sums_fp64).  With a third of the widths at 0.9 of the cell size the stage call takes
 // 165 us at 204k and 580 us at 2M particles, a 1M-particle step 296 us; 178, 663 and 322 us with the 16-byte
 // records, 302, 897 and 390 us while every state other than the first form's took the whole of the tests.
+// The window form, met in the step after a value turns non-finite, takes 296 us at 204k and 980 us at 2M particles;
+// 480 and 1627 us with every candidate's position taken in FP64, 239 and 883 us with the 16-byte records.
+// Telling blanked records by their position instead of their sound speed: 284 and 900 us, but 168 registers.
 __device__ __forceinline__ double interaction_alpha(const DevConsts &c, double is_tool) {
     // interactions_gpu.cu:164: the tool block (interactions_gpu.cu:19) is zero unless
     // interactions_setup_thermal_constants_tool set it (the rigid-tool setup does, benchmarks.cpp:518;
@@ -673,7 +676,10 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
                                                    typename Pos::Entry *__restrict__ list, const Pos &pos,
                                                    int *__restrict__ flags, int form) {
 #pragma clang fp contract(fast)
-    const bool win = SPECIAL && (form & SPHFEM_FORM_WINDOW), wide = SPECIAL && (form & ~SPHFEM_FORM_WIDTH);
+    // of a window's candidates the blanked ones are left out by their records; a finite position near its cell
+    // (one that is not sets AWAY) lies where the wrapped one says
+    const bool win = SPECIAL && (form & SPHFEM_FORM_WINDOW), tests = SPECIAL && (form & ~SPHFEM_FORM_WIDTH);
+    const bool wide = SPECIAL && (form & (SPHFEM_FORM_AWAY | SPHFEM_FORM_REACH));
     double d_v0 = 0., d_v1 = 0., d_v2 = 0., d_v3 = 0.;
     double d_ax = 0., d_ay = 0., d_p0 = 0., d_p1 = 0., d_T = 0.;
     const float4 a3 = rv.r3[i];
@@ -816,7 +822,7 @@ __device__ __forceinline__ PairOut pairs_fp32c_one(const DevConsts &c, const int
                 pos.scan4(d, j, b);
 #pragma unroll
                 for (int u = 0; u < 4; u++) {
-                    if (SPECIAL && wide && (j + u >= last || rv.r3[j + u].z == -INFINITY)) continue;
+                    if (SPECIAL && tests && (j + u >= last || rv.r3[j + u].z == -INFINITY)) continue;
                     float dx, dy;
                     distance((unsigned)(j + u), b[u], dx, dy);
                     const float D2 = dx * dx + dy * dy;

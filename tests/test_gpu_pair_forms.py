@@ -99,7 +99,7 @@ def test_fp32c_stage_call_form_switch():
     S.interactions_setup_geometry_constants(sim.grid)
     clean = {f: o.P[f].copy() for f in STATE}
     clean["blanked"][5::11] = 1.0
-    for fault in (None, ("S", np.nan), None, ("vel", np.nan), ("h", 0.8), None):
+    for fault in (None, ("S", np.nan), None, ("vel", np.nan), ("h", 0.8), ("pos", np.nan), None):
         got = {}
         for which in ("fp32c", "fp64"):
             for f in STATE:
